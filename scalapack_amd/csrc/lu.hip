@@ -111,6 +111,7 @@ PanelWork<T> Handle::panel_work()
     pw.zero_col = zero_col;
     pw.spin_limit = spin_limit;
     pw.target_wgs = panel_wgs;
+    pw.num_cus = num_cus;
     return pw;
 }
 

@@ -3,26 +3,49 @@
 // workgroups that hold the leaf in registers.
 //
 // Per column j the reference does PDAMAX (pivot search) -> PDSWAP (row
-// interchange) -> PDSCAL(1/GMAX) -> PDGER(-1) (rank-1 update).  Here:
-//   1. every thread scans its rows >= j; a wave64 shuffle reduction and a
-//      4-wave LDS step give the workgroup's candidate (|v|, row), ties to
-//      the lower row as IDAMAX does;
-//   2. each workgroup publishes its candidate row (index and W values) and
-//      workgroup 0 publishes row j, into mailbox words of column j;
-//   3. every workgroup gathers the G candidates and row j; each word is
-//      written once per launch and starts out empty, so a word that is no
-//      longer empty holds this column's value: one round trip, no counter;
-//   4. every workgroup reduces the G candidates in the same total order, so
-//      all agree on the pivot row p;
-//   5. the owners of rows j and p exchange them in registers;
-//   6. rows below j are scaled by the reciprocal 1/pivot (the reference's
+// interchange) -> PDSCAL(1/GMAX) -> PDGER(-1) (rank-1 update).  Here no row
+// changes place while the leaf is factored: every row carries the position
+// the interchanges have brought it to, a row whose position is below j is
+// done, and the interchange of j and p is an exchange of two positions.
+//   1. every wave finds the largest |v| among its rows of position >= j (ties
+//      to the lowest position, as IDAMAX) and posts that row to LDS together
+//      with 1 / v; one workgroup barrier; every wave folds the posts itself;
+//   2. with more than one workgroup, each publishes its candidate row (the
+//      columns from j on, the reciprocal, the position) in mailbox words of
+//      column j and gathers the other G - 1; each word is written once per
+//      launch and starts out empty, so a word that is no longer empty holds
+//      this column's value: one round trip, no counter; every wave reduces
+//      the G candidates in the same total order, so all agree on p;
+//   3. rows of position > j are scaled by the reciprocal (the reference's
 //      ONE / GMAX multiply, pdgetf2.f:224) and updated a -= l * u with one fma.
-// PDGETF2 swaps the full JB-wide panel rows (pdgetf2.f:219-220): the leaf's
-// interchanges, composed into one row permutation, are applied to the rest
-// of the block column after the last column (no other access touches those
+// The rows are written to their final positions at the end, and PDGETF2's
+// interchanges of the other columns of the block column (pdgetf2.f:219-220)
+// follow as the leaf's net row permutation (no other access touches those
 // columns meanwhile, so the result is the same as swapping per column).
 // A zero pivot skips the interchange and the scaling and records the first
 // such column (pdgetf2.f:226-228); the update still runs, as PDGER does.
+//
+// What bounds it is the latency of that chain, W times per leaf.  Two choices
+// shorten it.  A row lies in the four lanes of a quad, column c in lane c % 4
+// (register c / 4): the pivot row costs a lane NC LDS reads instead of W, the
+// posting quad writes it with NC / 2 16-byte stores, and the multiplier reaches
+// the quad by one DPP move.  And the column loop is a run-time loop whose body
+// handles one column and rotates the registers by one after every fourth, so
+// that every register index is a constant in a body of a few KB: unrolled over
+// all columns, as before, the leaf was 340 KB of code that every launch fetched
+// anew.
+//
+// The exchange is as fast as the path between the workgroups: a word written
+// and read through the L2 of one XCD takes 230 ns, through the device-coherent
+// path 440 ns within an XCD and 500 - 620 ns between two (ping-pong of two
+// workgroups).  So a leaf of at most 32 workgroups puts them all on one XCD, a
+// different one from leaf to leaf, because the trailing update beside it is
+// dealt evenly over all of them.
+//
+// Measured on 32 FP64 columns, alone on the GPU, us per leaf, before (all
+// columns unrolled, rows interchanged in registers, the workgroups spread over
+// the XCDs) and now: m = 100: 125, 37; 1000: 136, 78; 4000: 149, 90; 16384:
+// 165, 95; 32768: 183, 121.
 //
 // Mailbox: two regions of 32 column blocks; launch L uses region L & 1 and
 // refills the words launch L - 1 wrote in region (L + 1) & 1 -- that launch
@@ -32,24 +55,19 @@
 #include "sla_kernels.h"
 
 #include <algorithm>
-#include <type_traits>
-
 #include <climits>
-
-// wavefront-wide maximum of the ROCm device library
-extern "C" __device__ __attribute__((const)) unsigned long long __ockl_wfred_max_u64(
-    unsigned long long);
 
 namespace sla {
 
 namespace {
 
-constexpr int PT = 512;          // threads per workgroup (8 waves)
+constexpr int PT = 512;          // threads per workgroup at most (8 waves)
 constexpr int NWV = PT / 64;
 constexpr int LEAF_GMAX = 128;   // workgroups per leaf launch at most
+constexpr int XCDS = 8, XCD_CUS = 32;  // the dies of the GPU and the CUs of one
 static_assert(LEAF_GMAX <= PANEL_MAIL_GMAX, "mailbox too small for the leaf's grid");
 
-constexpr uint64_t MAIL_EMPTY = ~0ull;  // no row index or value word has this pattern
+constexpr uint64_t MAIL_EMPTY = ~0ull;  // no position or value word has this pattern
 
 // Storage of one value in a mailbox word.  A double whose bits equal the
 // empty pattern (a NaN) is stored as the neighbouring NaN pattern.
@@ -69,295 +87,500 @@ __device__ __forceinline__ T mail_value(uint64_t w)
     else return __builtin_bit_cast(T, (uint32_t)w);
 }
 
-template <int I, int N, typename F>
-__device__ __forceinline__ void static_for(F &&f)
-{
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
-
-typedef unsigned long long u64x2_t __attribute__((ext_vector_type(2)));
-typedef int i32x4_t __attribute__((ext_vector_type(4)));
-
-// Pivot key of a candidate: the bits of |v| plus one, monotone in |v|; 0 for
-// no candidate and for a NaN, which IDAMAX's comparisons never select.
-__device__ __forceinline__ uint64_t mag_key(double v, bool valid)
+// Pivot key of a candidate: monotone in |v|, more than 1 for a nonzero v; 0
+// for no candidate and for a NaN, which IDAMAX's comparisons never select.  A
+// NaN in row j itself (top) counts as a zero: a column without anything larger
+// keeps row j.
+__device__ __forceinline__ uint64_t mag_key(double v, bool valid, bool top)
 {
     const double a = fabs(v);
-    return (valid && a == a) ? __builtin_bit_cast(uint64_t, a) + 1ull : 0ull;
+    return !valid ? 0ull : a == a ? __builtin_bit_cast(uint64_t, a) + 1ull : (top ? 1ull : 0ull);
+}
+__device__ __forceinline__ uint64_t mag_key(float v, bool valid, bool top)
+{
+    return mag_key((double)v, valid, top);
 }
 
-// Wave-wide first maximum: the largest key and, among the lanes holding it,
-// the lowest row (INT_MAX when no lane holds a key), in every lane.
-__device__ __forceinline__ void wave_argmax(uint64_t &key, int &row)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_max(uint32_t x)
 {
-    const uint64_t km = __ockl_wfred_max_u64(key);
-    uint64_t tied = __ballot(km != 0 && key == km);
-    int best = INT_MAX;
-    while (tied) {  // uniform; one lane unless magnitudes tie
-        const int l = __ffsll((unsigned long long)tied) - 1;
-        best = min(best, __builtin_amdgcn_readlane(row, l));
-        tied &= tied - 1;
+    // lanes the move does not reach combine with 0
+    const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
+    return x > y ? x : y;
+}
+
+// Wave-wide maximum, uniform: within rows of 16 lanes by rotation, then the
+// row maxima broadcast upwards (row_bcast:15 and :31), the result in lane 63.
+__device__ __forceinline__ uint32_t wave_max(uint32_t x)
+{
+    x = dpp_max<0x121, 0xf>(x);
+    x = dpp_max<0x122, 0xf>(x);
+    x = dpp_max<0x124, 0xf>(x);
+    x = dpp_max<0x128, 0xf>(x);
+    x = dpp_max<0x142, 0xa>(x);
+    x = dpp_max<0x143, 0xc>(x);
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+
+// The wave's first maximum by full keys: the lane holding the largest key and,
+// among equal keys, the lowest position; its key and position in every lane.
+__device__ __forceinline__ int wave_pick(uint64_t &key, int &pos)
+{
+    const uint32_t hi = (uint32_t)(key >> 32), lo = (uint32_t)key;
+    const uint32_t hm = wave_max(hi);
+    const uint32_t lm = wave_max(hi == hm ? lo : 0u);
+    const bool in = hi == hm && lo == lm;
+    const uint32_t np = in ? ~(uint32_t)pos : 0u;  // positions are >= 0
+    const uint32_t nm = wave_max(np);
+    const int l = __builtin_ctzll(__ballot(in && np == nm));
+    const uint32_t kl = __builtin_amdgcn_readlane(lo, l), kh = __builtin_amdgcn_readlane(hi, l);
+    key = ((uint64_t)kh << 32) | kl;
+    pos = __builtin_amdgcn_readlane(pos, l);
+    return l;
+}
+
+// The leading 32 bits of |v|, monotone in |v|.  One maximum of them decides a
+// pivot search unless it is shared (the rest of the bits, then the position
+// decide), is zero (zeros, denormals, no row) or is not finite; those searches
+// use the full keys.
+__device__ __forceinline__ uint32_t mag_hi(double v)
+{
+    return (uint32_t)(__builtin_bit_cast(uint64_t, v) >> 32) & 0x7fffffffu;
+}
+__device__ __forceinline__ uint32_t mag_hi(float v)
+{
+    return __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
+}
+template <typename T>
+__device__ __forceinline__ bool decides(uint32_t hm)
+{
+    return hm - 1u < (sizeof(T) == 8 ? 0x7ff00000u : 0x7f800000u) - 1u;
+}
+
+// v[q] <- the value of lane S of the quad, in all four lanes.
+template <int S, int NQ>
+__device__ __forceinline__ void quad_bcast(double (&v)[NQ])
+{
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v[q]);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, S * 0x55, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), S * 0x55, 0xf, 0xf, false);
+        v[q] = __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
     }
-    key = km;
-    row = best;
+}
+template <int S, int NQ>
+__device__ __forceinline__ void quad_bcast(float (&v)[NQ])
+{
+#pragma unroll
+    for (int q = 0; q < NQ; q++)
+        v[q] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                                             0, __builtin_bit_cast(int, v[q]), S * 0x55, 0xf, 0xf, false));
 }
 
-// Gathered word idx of a column into LDS: candidate idx / (W + 1) (row
-// index, then W values) for idx < ncand, else row j.
-template <typename T, int W>
-__device__ __forceinline__ void mail_put(int idx, int ncand, uint64_t v, int *s_cr,
-                                         T (*s_rows)[W + 1], T *s_rowj)
+// Words of one candidate: the row, 4 NC values in register order, lane by lane.
+// In LDS a row takes 34 words: that spreads column j of all candidates over the
+// banks and keeps the rows 16-byte aligned.
+constexpr int CW = PANEL_MAIL_CW, CWL = 34;
+
+template <typename T>
+struct alignas(16) LeafLds {
+    T wrow[2][NWV][CWL];          // each wave's candidate, by column parity
+    int wpos[2][NWV];             // its position; INT_MAX: no candidate
+    T u[32][CWL];                 // the pivot rows of the leaf
+    int s_pv[32];                 // interchange of each column; -1: a zero pivot, none
+    int s_dst[64], s_src[64], s_npair;
+    int s_abort;
+};
+template <typename T, bool SOLO>
+struct alignas(16) LeafCands {
+    T rows[SOLO ? 1 : LEAF_GMAX][CWL];
+    uint64_t pos[SOLO ? 1 : LEAF_GMAX];  // position, XCD in the upper half
+};
+
+struct LeafArgs {
+    uint64_t *box;  // this launch's mailbox region
+    int *abort_flag;
+    uint64_t spin_limit, t0;
+    int G, g;       // workgroups of the leaf, this one
+    uint32_t xcd;   // the die it runs on
+};
+
+// A word for the other workgroups: through the L2 of the XCD (local: every
+// workgroup of the leaf runs on this one, and a load that bypasses the L1 finds
+// it there) or to where every XCD sees it.
+__device__ __forceinline__ void post_word(uint64_t *p, uint64_t v, bool local)
 {
-    if (idx < ncand) {
-        const int gg = idx / (W + 1), e = idx - gg * (W + 1);
-        if (e == 0) s_cr[gg] = (int)v;
-        else s_rows[gg][e - 1] = mail_value<T>(v);
-    } else {
-        s_rowj[idx - ncand] = mail_value<T>(v);
+    if (local) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else coherent_store(p, v);
+}
+
+// Publishes the workgroup's candidate of column j (row src, position cpos;
+// INT_MAX: none) and gathers everyone's into LDS.  Only the registers below
+// `live` hold columns right of j.  The position word's upper half carries the
+// XCD.  An abort (sl.s_abort) leaves what was gathered so far.
+template <typename T, int NC>
+__device__ __forceinline__ void exchange(const LeafArgs &ar, int j, int live, bool local,
+                                         const T *src, int cpos, LeafLds<T> &sl,
+                                         LeafCands<T, false> &sc)
+{
+    const int G = ar.G, tid = threadIdx.x, lane = tid & 63;
+    uint64_t *cb = ar.box + (size_t)j * PANEL_MAIL_COL;
+    constexpr int NV = 4 * NC;  // value words of a candidate
+    if (tid < NV + 1) {
+        uint64_t *mine = cb + (size_t)ar.g * CW;
+        if (lane < NV) {
+            if (lane % NC < live) post_word(&mine[lane], mail_word(src[lane]), local);
+        } else {
+            post_word(&cb[PANEL_MAIL_POS + ar.g], ((uint64_t)ar.xcd << 32) | (uint32_t)cpos, local);
+        }
     }
-}
-
-// Waits until the mailbox word *p is written; false once the launch has
-// been aborted (by this wait after spin_limit ticks since t0, or elsewhere).
-__device__ __forceinline__ bool mail_wait(const uint64_t *p, uint64_t &v, int *abort_flag,
-                                          uint64_t t0, uint64_t spin_limit)
-{
+    // gather: NV threads per candidate for the values, one for its position,
+    // GL candidates a pass.  All loads of a pass are in flight before the first
+    // is looked at; a word still empty is loaded again.
+    constexpr int per = PT / NV, GL = 2;  // an exchanging launch has PT threads
+    const int e = tid % NV, g0 = tid / NV;
+    const bool want = e % NC < live;
+    const unsigned wp = PANEL_MAIL_POS + min(tid, G - 1);
+    bool nopos = tid < G;
     unsigned it = 0;
-    while ((v = coherent_load(p)) == MAIL_EMPTY) {
-        if ((++it & 15u) == 0) {
-            if (coherent_load(abort_flag)) return false;
-            if (wall_clock64() - t0 > spin_limit) {
-                coherent_store(abort_flag, 1);
-                return false;
+    for (int gb = 0; gb < G; gb += per * GL) {
+        unsigned w[GL];
+        bool miss[GL];
+#pragma unroll
+        for (int k = 0; k < GL; k++) {
+            const int g = gb + g0 + k * per;
+            miss[k] = want && g < G;
+            w[k] = min(g, G - 1) * CW + e;
+        }
+        for (;;) {
+            uint64_t v[GL];
+#pragma unroll
+            for (int k = 0; k < GL; k++) v[k] = coherent_load(&cb[w[k]]);
+            const uint64_t vp = coherent_load(&cb[wp]);
+            bool again = false;
+#pragma unroll
+            for (int k = 0; k < GL; k++) {
+                if (miss[k] && v[k] != MAIL_EMPTY) {
+                    sc.rows[gb + g0 + k * per][e] = mail_value<T>(v[k]);
+                    miss[k] = false;
+                }
+                again = again || miss[k];
+            }
+            if (nopos && vp != MAIL_EMPTY) {
+                sc.pos[tid] = vp;
+                nopos = false;
+            }
+            if (!again && !nopos) break;
+            if ((++it & 15u) == 0) {
+                if (coherent_load(ar.abort_flag)) sl.s_abort = 1;
+                else if (wall_clock64() - ar.t0 > ar.spin_limit) {
+                    coherent_store(ar.abort_flag, 1);
+                    sl.s_abort = 1;
+                }
+                if (sl.s_abort) break;
             }
         }
-        __builtin_amdgcn_s_sleep(1);
     }
-    return true;
+    __syncthreads();
 }
 
-template <typename T, int W, int RPT>
+// x[0] .. x[NC-1] rotated down by one.  Written out by recursion: as a loop it
+// may become a memmove, which keeps the array in scratch memory.
+template <int NC, int I = 0, typename T>
+__device__ __forceinline__ void rotate_row(T (&x)[NC], T first)
+{
+    if constexpr (I + 1 < NC) {
+        x[I] = x[I + 1];
+        rotate_row<NC, I + 1>(x, first);
+    } else {
+        x[I] = first;
+    }
+}
+
+// x[q][i] -= l[q] u[i] for 1 <= i < live (uniform).
+template <int I = 1, int NQ, int NC, typename T>
+__device__ __forceinline__ void update_rows(T (&x)[NQ][NC], const T (&l)[NQ], const T (&u)[NC],
+                                            int live)
+{
+    if constexpr (I < NC) {
+        if (I < live) {
+#pragma unroll
+            for (int q = 0; q < NQ; q++) x[q][I] = fma(-l[q], u[I], x[q][I]);
+            update_rows<I + 1>(x, l, u, live);
+        }
+    }
+}
+
+// Column j, in register 0 of the lanes with cg = j % 4 = S; the registers
+// 1 .. live-1 hold the columns further right.  A row that is done (or beyond
+// the leaf) holds zeros there, so it neither wins a search nor is changed by an
+// update; its multipliers stay.
+template <typename T, int NC, int NQ, bool SOLO>
+__device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][NC],
+                                          int (&pos)[NQ], bool &local, LeafLds<T> &sl,
+                                          LeafCands<T, SOLO> &sc)
+{
+    typedef T v2_t __attribute__((ext_vector_type(2)));
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, cg = lane & 3;
+    const int nw = (int)blockDim.x >> 6, pb = j & 1, S = j & 3, live = NC - (j >> 2);
+
+    // 1. candidate of the wave: row q of lane wl
+    int wl = 0, uq = 0;
+    bool found;
+    {
+        const uint64_t cols = 0x1111111111111111ull << S;  // the lanes holding column j
+        uint32_t h[NQ], hx = 0;
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            h[q] = mag_hi(a[q][0]);
+            hx = h[q] > hx ? h[q] : hx;
+        }
+        const uint32_t hm = wave_max(cg == S ? hx : 0u);
+        int cnt = 0;
+        uint64_t t = 0;
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            const uint64_t tq = __ballot(h[q] == hm) & cols;
+            cnt += __builtin_popcountll(tq);
+            uq = tq ? q : uq;
+            t |= tq;
+        }
+        found = true;
+        if (cnt == 1 && decides<T>(hm)) {
+            wl = __builtin_ctzll(t);
+        } else {
+            uint64_t bk = 0;
+            int bp = INT_MAX, bq = 0;
+#pragma unroll
+            for (int q = 0; q < NQ; q++) {
+                const uint64_t k = mag_key(a[q][0], cg == S && pos[q] >= j, pos[q] == j);
+                const bool take = k > bk || (k != 0 && k == bk && pos[q] < bp);
+                bk = take ? k : bk;
+                bp = take ? pos[q] : bp;
+                bq = take ? q : bq;
+            }
+            wl = wave_pick(bk, bp);
+            uq = __builtin_amdgcn_readlane(bq, wl);
+            found = bk != 0;
+        }
+    }
+    if (found && (lane >> 2) == (wl >> 2)) {
+        T *dst = &sl.wrow[pb][wave][cg * NC];
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            if (uq == q) {
+#pragma unroll
+                for (int i = 0; i < NC; i += 2) {
+                    const v2_t x = {a[q][i], a[q][i + 1]};
+                    *reinterpret_cast<v2_t *>(&dst[i]) = x;
+                }
+                sl.wpos[pb][wave] = pos[q];
+                // keeps the branches apart: merged, they select a row by
+                // address, and the array goes to scratch memory
+                asm volatile("; row %0" ::"i"(q));
+            }
+        }
+    }
+    if (!found && lane == 0) sl.wpos[pb][wave] = INT_MAX;
+    __syncthreads();
+    // the workgroup's: lane x looks at the candidate of wave x % 8
+    int p, fw;
+    bool nonzero = true;
+    T pv;
+    {
+        const int x = lane & (NWV - 1);
+        const int xp = x < nw ? sl.wpos[pb][x] : INT_MAX;
+        const T xv = sl.wrow[pb][x][S * NC];
+        const uint32_t h = xp != INT_MAX ? mag_hi(xv) : 0u;
+        uint32_t hm = dpp_max<0x121, 0xf>(h);
+        hm = dpp_max<0x122, 0xf>(hm);
+        hm = dpp_max<0x124, 0xf>(hm);
+        hm = (uint32_t)__builtin_amdgcn_readfirstlane((int)hm);
+        const unsigned t = (unsigned)__ballot(h == hm) & 0xffu;
+        if (decides<T>(hm) && (t & (t - 1)) == 0) {
+            fw = __builtin_ctz(t);
+            p = __builtin_amdgcn_readlane(xp, fw);
+        } else {
+            uint64_t ck = mag_key(xv, xp != INT_MAX, xp == j);
+            p = ck != 0 ? xp : INT_MAX;
+            fw = wave_pick(ck, p) & (NWV - 1);
+            nonzero = ck > 1;
+        }
+        pv = lane_read(xv, fw);
+    }
+    const T *prow = sl.wrow[pb][fw];
+
+    // 2. the other workgroups
+    if constexpr (!SOLO) {
+        exchange<T, NC>(ar, j, live, local, prow, p, sl, sc);
+        const int G = ar.G, x = lane < G ? lane : 0;
+        const int xp = lane < G ? (int)sc.pos[x] : INT_MAX;
+        const T xv = sc.rows[x][S * NC];
+        const uint32_t h = xp != INT_MAX ? mag_hi(xv) : 0u;
+        const uint32_t hm = wave_max(h);
+        const uint64_t t = __ballot(h == hm);
+        nonzero = true;
+        int gw;
+        if (G <= 64 && decides<T>(hm) && (t & (t - 1)) == 0) {
+            gw = __builtin_ctzll(t);
+            p = __builtin_amdgcn_readlane(xp, gw);
+            pv = lane_read(xv, gw);
+        } else {
+            uint64_t ck = 0;
+            int bg = 0;
+            p = INT_MAX;
+            for (int y = lane; y < G; y += 64) {
+                const int yp = (int)sc.pos[y];
+                const uint64_t yk = mag_key(sc.rows[y][S * NC], yp != INT_MAX, yp == j);
+                const bool take = yk > ck || (yk != 0 && yk == ck && yp < p);
+                ck = take ? yk : ck;
+                p = take ? yp : p;
+                bg = take ? y : bg;
+            }
+            const int l = wave_pick(ck, p);
+            gw = __builtin_amdgcn_readlane(bg, l);
+            nonzero = ck > 1;
+            pv = sc.rows[gw][S * NC];
+        }
+        prow = sc.rows[gw];
+        if (j == 0) {
+            // from here on through the L2, if every workgroup is on this XCD
+            bool same = true;
+            for (int y = lane; y < G; y += 64)
+                same = same && (sc.pos[y] >> 32) == (sc.pos[0] >> 32);
+            local = __all(same);
+        }
+    }
+
+    // 3. interchange, scaling, rank-1 update
+    T u[NC];
+#pragma unroll
+    for (int i = 0; i < NC; i += 2) {
+        const v2_t x = *reinterpret_cast<const v2_t *>(&prow[cg * NC + i]);
+        u[i] = x[0];
+        u[i + 1] = x[1];
+    }
+    T l[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) l[q] = a[q][0];
+    if (S == 0) quad_bcast<0>(l);
+    else if (S == 1) quad_bcast<1>(l);
+    else if (S == 2) quad_bcast<2>(l);
+    else quad_bcast<3>(l);
+    // a zero pivot keeps row j (p = j) and leaves the column unscaled
+    const T rcp = nonzero ? T(1) / pv : T(1);
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+        const int x = pos[q];
+        const bool own = x == p;
+        pos[q] = own ? j : (x == j ? p : x);
+        // the pivot row with l = 1 becomes zero right of the diagonal
+        l[q] = own ? T(1) : l[q] * rcp;
+    }
+    if (wave == (j & (nw - 1)) && lane < 4 * NC) sl.u[j][lane] = prow[lane];
+    if (tid == 0) sl.s_pv[j] = nonzero ? p : -1;
+    if (cg >= S) {
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            const T x0 = fma(-l[q], u[0], a[q][0]);
+            a[q][0] = cg == S ? l[q] : x0;
+        }
+    }
+    update_rows(a, l, u, live);
+}
+
+// NC: registers per row and lane (leaf width 4 NC), NQ: rows per quad; a wave
+// holds 16 NQ rows.  SOLO: a single workgroup, no exchange.
+// stride: the leaf's workgroups are every stride-th of the launch (the others
+// leave at once): with 8, the number of XCDs over which consecutive workgroups
+// are dealt, they share one XCD and its L2 (checked in column 0).
+template <typename T, int NC, int NQ, bool SOLO>
 __global__ __launch_bounds__(PT) void panel_leaf_kernel(
     T *__restrict__ A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0,
     int *__restrict__ ipiv, uint64_t *__restrict__ mail, int region, int prev_wa, int prev_g,
-    int prev_cs, int *abort_flag, int *zero_col, uint64_t spin_limit)
+    int *abort_flag, int *zero_col, uint64_t spin_limit, int stride, int first)
 {
-    const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    constexpr int R = RPT * PT;  // rows per workgroup
-    constexpr int CS = W + 1;    // words per candidate: row index, W values
-    // gathered words per thread: G * CS candidate words + W words of row j
-    constexpr int KW = (LEAF_GMAX * CS + W + PT - 1) / PT;
+    if (!SOLO && (int)blockIdx.x % stride != first) return;
+    const int G = SOLO ? 1 : gridDim.x / stride, g = SOLO ? 0 : blockIdx.x / stride;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = tid >> 6, nw = (int)blockDim.x >> 6;
+    const int cg = lane & 3, rg = lane >> 2;
+    const int base = (g * nw + wave) * (16 * NQ) + rg;  // row q of this quad: base + 16 q
 
-    __shared__ __align__(16) uint64_t s_wk[NWV];
-    __shared__ __align__(16) int s_wr[NWV];
-    __shared__ int s_cr[LEAF_GMAX];
-    __shared__ T s_rows[LEAF_GMAX][W + 1];  // odd stride: column j of all rows without bank conflicts
-    __shared__ T s_rowj[W];
-    __shared__ int s_abort;
-    __shared__ int s_pv[W];              // interchange of each column (p; j when none)
-    __shared__ int s_dst[2 * W], s_src[2 * W], s_npair;
+    __shared__ LeafLds<T> sl;
+    __shared__ LeafCands<T, SOLO> sc;
+    if (tid == 0) sl.s_abort = 0;
 
-    if (tid == 0) s_abort = 0;
-
-    // empty the words the previous launch wrote (the other region):
-    // columns < prev_wa, its prev_g candidates of prev_cs words, row j
-    {
+    if constexpr (!SOLO) {
+        // empty the words the previous launch that used the mailbox wrote (the
+        // other region): columns < prev_wa, its prev_g candidates
         uint64_t *o = mail + (size_t)(region ^ 1) * PANEL_MAIL_REGION;
-        const int per = prev_g * prev_cs + 32;
-        for (int i = g * PT + tid; i < prev_wa * per; i += G * PT) {
-            const int jj = i / per, e = i - jj * per;
-            const int off = e < prev_g * prev_cs ? e : PANEL_MAIL_ROWJ + (e - prev_g * prev_cs);
-            coherent_store(&o[(size_t)jj * PANEL_MAIL_COL + off], MAIL_EMPTY);
+        const int per = prev_g * (CW + 1);
+        for (int jj = 0; jj < prev_wa; jj++)
+            for (int e = g * (int)blockDim.x + tid; e < per; e += G * (int)blockDim.x)
+                coherent_store(&o[(size_t)jj * PANEL_MAIL_COL +
+                                  (e < prev_g * CW ? e : PANEL_MAIL_POS + e - prev_g * CW)],
+                               MAIL_EMPTY);
+    }
+
+    // column 4 i + cg of the leaf in register i; columns right of a narrow
+    // leaf are zeros that no step pivots on
+    T a[NQ][NC];
+    int pos[NQ];  // current position of the row; -1: no row
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+        const int r = base + 16 * q;
+        pos[q] = r < m ? r : -1;
+#pragma unroll
+        for (int i = 0; i < NC; i++) {
+            const int c = 4 * i + cg;
+            a[q][i] = (r < m && c < wa) ? A[r + (size_t)c * lda] : T(0);
         }
     }
-    uint64_t *box = mail + (size_t)region * PANEL_MAIL_REGION;
-
-    T a[RPT][W];
+    const LeafArgs ar{mail + (size_t)region * PANEL_MAIL_REGION, abort_flag, spin_limit, (uint64_t)wall_clock64(), G, g,
+                      SOLO ? 0u : (uint32_t)__builtin_amdgcn_s_getreg(63508) & 0xffffu};  // XCC_ID
+    bool local = false;
+    __syncthreads();
+    // After the last column of a group of four the registers rotate by one.
+    // Nothing in the loop writes to global memory but the exchange: the waits
+    // for a store's completion would join the chain.  After an abort the
+    // workgroup leaves at the end of the group.
+#pragma unroll 1
+    for (int t = 0; t < NC; t++) {
+        const int je = (!SOLO && sl.s_abort) ? 0 : min(4 * t + 4, wa);
+#pragma unroll 1
+        for (int j = 4 * t; j < je; j++) leaf_step<T, NC, NQ, SOLO>(ar, j, a, pos, local, sl, sc);
 #pragma unroll
-    for (int q = 0; q < RPT; q++) {
-        const int r = g * R + q * PT + tid;
-#pragma unroll
-        for (int c = 0; c < W; c++)
-            a[q][c] = (r < m && c < wa) ? A[r + (size_t)c * lda] : T(0);
+        for (int q = 0; q < NQ; q++) rotate_row<NC>(a[q], a[q][0]);
     }
-    const uint64_t t0 = wall_clock64();
 
-    // The columns as a compile-time loop: every index into a[][] is a
-    // constant, so the leaf stays in registers.  (A run-time column loop
-    // with selects instead of constant indices measured slower.)
-    bool alive = true;
-    static_for<0, W>([&](auto jc) {
-        constexpr int j = decltype(jc)::value;
-        if (!alive || j >= wa) return;  // wa and the abort flag are uniform across the grid
-        uint64_t *cb = box + (size_t)j * PANEL_MAIL_COL;  // this column's words
-
-        // 1. candidate of this workgroup: per thread, per wave (packed
-        //    magnitude keys, one wave reduction), then every thread folds
-        //    the NWV wave results itself
-        uint64_t bk = 0;
-        int br = INT_MAX;
+    // Every row to its final position (every workgroup has loaded its rows:
+    // it took part in the last column's exchange).  NC rotations have brought
+    // every column back to its register.  Of a pivot row the multipliers are
+    // here; its part of U is in sl.u, in the register order of its column.
+    __syncthreads();
+    if (!SOLO && sl.s_abort) return;
 #pragma unroll
-        for (int q = 0; q < RPT; q++) {
-            const int r = g * R + q * PT + tid;
-            const uint64_t k = mag_key((double)a[q][j], r < m && r >= j);
-            if (k > bk) { bk = k; br = r; }
-        }
-        wave_argmax(bk, br);
-        if (lane == 0) { s_wk[wave] = bk; s_wr[wave] = br; }
-        __syncthreads();
-        // all NWV posts in one round of 16-byte LDS reads, then a
-        // branch-free fold in registers
-        uint64_t wk[NWV];
-        int wr[NWV];
+    for (int q = 0; q < NQ; q++) {
+        if (pos[q] >= 0) {
 #pragma unroll
-        for (int w = 0; w < NWV; w += 2) {
-            const u64x2_t k2 = *reinterpret_cast<const u64x2_t *>(&s_wk[w]);
-            wk[w] = k2[0];
-            wk[w + 1] = k2[1];
-        }
-#pragma unroll
-        for (int w = 0; w < NWV; w += 4) {
-            const i32x4_t r4 = *reinterpret_cast<const i32x4_t *>(&s_wr[w]);
-#pragma unroll
-            for (int e = 0; e < 4; e++) wr[w + e] = r4[e];
-        }
-        uint64_t ck = wk[0];
-        int cr = wr[0];
-#pragma unroll
-        for (int w = 1; w < NWV; w++) {
-            const bool take = wk[w] > ck || (wk[w] == ck && wr[w] < cr);
-            ck = take ? wk[w] : ck;
-            cr = take ? wr[w] : cr;
-        }
-
-        // 2. publish the candidate (row index and the row's W values; a
-        //    workgroup without rows >= j publishes INT_MAX and zeros) and,
-        //    from the owner of row j, row j
-        uint64_t *mine = cb + (size_t)g * CS;
-        if (cr == INT_MAX && tid == 0) {
-#pragma unroll
-            for (int c = 0; c < W; c++) coherent_store(&mine[1 + c], mail_word(T(0)));
-            coherent_store(&mine[0], (uint64_t)INT_MAX);
-        }
-#pragma unroll
-        for (int q = 0; q < RPT; q++) {
-            const int r = g * R + q * PT + tid;
-            if (r == cr) {
-#pragma unroll
-                for (int c = 0; c < W; c++) coherent_store(&mine[1 + c], mail_word(a[q][c]));
-                coherent_store(&mine[0], (uint64_t)cr);
-            }
-            if (r == j) {
-                uint64_t *dst = cb + PANEL_MAIL_ROWJ;
-#pragma unroll
-                for (int c = 0; c < W; c++) coherent_store(&dst[c], mail_word(a[q][c]));
+            for (int i = 0; i < NC; i++) {
+                const int c = 4 * i + cg;
+                if (c < wa && (pos[q] >= wa || c < pos[q])) A[pos[q] + (size_t)c * lda] = a[q][i];
             }
         }
-
-        // 3. gather: all loads in flight at once; a word still empty is
-        //    then awaited on its own (bounded wait)
-        {
-            const int nword = G * CS + W;
-            unsigned miss = 0;  // bit k: word tid + k PT not written yet
-#pragma unroll
-            for (int k = 0; k < KW; k++) {
-                const int idx = tid + k * PT;
-                if (idx < nword) {
-                    const int off = idx < G * CS ? idx : PANEL_MAIL_ROWJ + (idx - G * CS);
-                    const uint64_t v = coherent_load(&cb[off]);
-                    if (v == MAIL_EMPTY) miss |= 1u << k;
-                    else mail_put<T, W>(idx, G * CS, v, s_cr, s_rows, s_rowj);
-                }
-            }
-            while (miss) {
-                const int idx = tid + (__ffs(miss) - 1) * PT;
-                const int off = idx < G * CS ? idx : PANEL_MAIL_ROWJ + (idx - G * CS);
-                uint64_t v;
-                if (!mail_wait(&cb[off], v, abort_flag, t0, spin_limit)) {
-                    s_abort = 1;
-                    break;
-                }
-                mail_put<T, W>(idx, G * CS, v, s_cr, s_rows, s_rowj);
-                miss &= miss - 1;
-            }
-        }
-        __syncthreads();
-        if (s_abort) {
-            alive = false;
-            return;
-        }
-
-        // 4. global pivot: every wave reduces the G candidates itself (the
-        //    same result everywhere, no further barrier); a candidate's value
-        //    is |its row's entry in column j|
-        int p;
-        {
-            uint64_t k = 0;
-            int r = INT_MAX;
-            for (int x = lane; x < G; x += 64) {
-                const int xr = s_cr[x];
-                const uint64_t xk = mag_key((double)s_rows[x][j], xr != INT_MAX);
-                if (xk > k || (xk == k && xr < r)) { k = xk; r = xr; }
-            }
-            wave_argmax(k, r);
-            p = (r == INT_MAX) ? j : r;  // an all-NaN column keeps row j
-        }
-        const int gw = p / R;
-        const T piv = s_rows[gw][j];
-        const bool nonzero = (piv != T(0));
-
-        // 5. interchange rows j and p in registers (only if the pivot is
-        //    nonzero); the rest of the block column follows after the leaf
-        if (nonzero && p != j) {
-#pragma unroll
-            for (int q = 0; q < RPT; q++) {
-                const int r = g * R + q * PT + tid;
-                if (r == p) {
-#pragma unroll
-                    for (int c = 0; c < W; c++) a[q][c] = s_rowj[c];
-                }
-                if (r == j) {
-#pragma unroll
-                    for (int c = 0; c < W; c++) a[q][c] = s_rows[gw][c];
-                }
-            }
-        }
-        if (tid == 0) s_pv[j] = nonzero ? p : j;
-        if (g == 0 && tid == 0) {
+    }
+    if (g == 0) {
+        if (tid < wa) {
             // PDAMAX returns INDX = IX for a zero maximum (pdamax_.c:486).
-            ipiv[row0 + j] = row0 + (nonzero ? p : j) + 1;
-            if (!nonzero) atomicMin(zero_col, col0 + j + 1);
+            const int p = sl.s_pv[tid];
+            ipiv[row0 + tid] = row0 + (p >= 0 ? p : tid) + 1;
+            if (p < 0) atomicMin(zero_col, col0 + tid + 1);
         }
-
-        // 6. scale by the reciprocal and rank-1 update of the rows below j
-        const T rcp = nonzero ? T(1) / piv : T(0);
-#pragma unroll
-        for (int q = 0; q < RPT; q++) {
-            const int r = g * R + q * PT + tid;
-            if (r < m && r > j) {
-                T l = a[q][j];
-                if (nonzero) {
-                    l = l * rcp;
-                    a[q][j] = l;
-                }
-#pragma unroll
-                for (int c = j + 1; c < W; c++) a[q][c] = fma(-l, s_rows[gw][c], a[q][c]);
-            }
-        }
-    });
-    if (!alive) return;
-
-#pragma unroll
-    for (int q = 0; q < RPT; q++) {
-        const int r = g * R + q * PT + tid;
-        if (r < m) {
-#pragma unroll
-            for (int c = 0; c < W; c++)
-                if (c < wa) A[r + (size_t)c * lda] = a[q][c];
+        for (int idx = tid; idx < wa * wa; idx += (int)blockDim.x) {
+            const int j = idx % wa, c = idx / wa;
+            if (c >= j) A[j + (size_t)c * lda] = sl.u[j][(c & 3) * NC + (c >> 2) - (j >> 2)];
         }
     }
 
@@ -369,12 +592,11 @@ __global__ __launch_bounds__(PT) void panel_leaf_kernel(
     // of a column all complete before its stores to that column.
     const int ne = lcols + rcols;
     if (ne <= 0) return;
-    __syncthreads();  // s_pv complete
     if (wave == 0) {
         int dst = -1, src = -1, cnt = 0;
         for (int j = 0; j < wa; j++) {
-            const int p = s_pv[j];
-            if (p == j) continue;
+            const int p = sl.s_pv[j];
+            if (p == j || p < 0) continue;
             const uint64_t mj = __ballot(dst == j), mp = __ballot(dst == p);
             const int lj = mj ? __ffsll((unsigned long long)mj) - 1 : -1;
             const int lp = mp ? __ffsll((unsigned long long)mp) - 1 : -1;
@@ -385,14 +607,14 @@ __global__ __launch_bounds__(PT) void panel_leaf_kernel(
             if (lp >= 0) { if (lane == lp) src = sj; }
             else { if (lane == cnt) { dst = p; src = sj; } cnt++; }
         }
-        if (lane < cnt) { s_dst[lane] = dst; s_src[lane] = src; }
-        if (lane == 0) s_npair = cnt;
+        if (lane < cnt) { sl.s_dst[lane] = dst; sl.s_src[lane] = src; }
+        if (lane == 0) sl.s_npair = cnt;
     }
     __syncthreads();
-    if (lane >= s_npair) return;
+    if (lane >= sl.s_npair) return;
     constexpr int CR = 8;
-    const int rd = s_dst[lane], rs = s_src[lane];
-    for (int e0 = (g * NWV + wave) * CR; e0 < ne; e0 += G * NWV * CR) {
+    const int rd = sl.s_dst[lane], rs = sl.s_src[lane];
+    for (int e0 = (g * nw + wave) * CR; e0 < ne; e0 += G * nw * CR) {
         T v[CR];
 #pragma unroll
         for (int c = 0; c < CR; c++) {
@@ -409,42 +631,31 @@ __global__ __launch_bounds__(PT) void panel_leaf_kernel(
     }
 }
 
-template <typename T, int W, int RPT>
-void launch_leaf_rpt(T *A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0,
-                     int *ipiv, const PanelWork<T> &pw, int G, hipStream_t s)
+template <typename T, int NC, int NQ>
+void launch_leaf(T *A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0, int *ipiv,
+                 const PanelWork<T> &pw, int threads, int G, hipStream_t s)
 {
-    // Only register-resident shapes are instantiated: at most 64 values of
-    // T per thread (128 VGPRs for doubles; floats get the same cap, beyond
-    // which the leaf's other registers no longer fit without scratch).
-    if constexpr (RPT * W <= 64) {
-        PanelMailState &ms = *pw.mail_state;
-        hipLaunchKernelGGL((panel_leaf_kernel<T, W, RPT>), dim3(G), dim3(PT), 0, s, A, lda, m,
-                           wa, lcols, rcols, row0, col0, ipiv, pw.mail, (int)(ms.launches & 1u),
-                           ms.prev_wa, ms.prev_g, ms.prev_cs, pw.abort_flag, pw.zero_col,
-                           pw.spin_limit);
+    PanelMailState &ms = *pw.mail_state;
+    if (G == 1) {
+        // the mailbox and its record stay as the last exchanging launch left them
+        hipLaunchKernelGGL((panel_leaf_kernel<T, NC, NQ, true>), dim3(1), dim3(threads), 0, s, A,
+                           lda, m, wa, lcols, rcols, row0, col0, ipiv, pw.mail, 0, 0, 0,
+                           pw.abort_flag, pw.zero_col, pw.spin_limit, 1, 0);
         SLA_LAUNCH_CHECK();
-        ms.launches++;
-        ms.prev_wa = wa;
-        ms.prev_g = G;
-        ms.prev_cs = W + 1;
-    } else {
-        throw std::logic_error("panel leaf: rows per thread exceed the register budget");
+        return;
     }
-}
-
-template <typename T, int W>
-void launch_leaf_w(T *A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0,
-                   int *ipiv, const PanelWork<T> &pw, int G, int rpt,
-                   hipStream_t s)
-{
-#define SLA_RPT(R) launch_leaf_rpt<T, W, R>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, G, s)
-    switch (rpt) {
-    case 1: SLA_RPT(1); break;
-    case 2: SLA_RPT(2); break;
-    case 4: SLA_RPT(4); break;
-    default: SLA_RPT(8); break;
-    }
-#undef SLA_RPT
+    // One XCD holds at most a workgroup per CU, so only on the whole GPU and
+    // for at most as many workgroups as an XCD has CUs.
+    const int stride = G <= XCD_CUS && pw.num_cus == XCDS * XCD_CUS ? XCDS : 1;
+    const int first = stride > 1 ? (int)(ms.launches % XCDS) : 0;
+    hipLaunchKernelGGL((panel_leaf_kernel<T, NC, NQ, false>), dim3(G * stride), dim3(threads), 0, s,
+                       A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw.mail,
+                       (int)(ms.launches & 1u), ms.prev_wa, ms.prev_g, pw.abort_flag, pw.zero_col,
+                       pw.spin_limit, stride, first);
+    SLA_LAUNCH_CHECK();
+    ms.launches++;
+    ms.prev_wa = wa;
+    ms.prev_g = G;
 }
 
 }  // namespace
@@ -453,30 +664,33 @@ template <typename T>
 unsigned panel_leaf(T *A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0,
                     int *ipiv, const PanelWork<T> &pw, hipStream_t s)
 {
-    // Rows per thread grows (1, 2, 4, 8) until the grid is within the target
-    // workgroup count; the register budget caps rows/thread * W at 64.
-    const int max_rpt_w = 64;
-    const int wcap = wa <= 8 ? 8 : (wa <= 16 ? 16 : 32);
-    int rpt_cap = max_rpt_w / wcap;
-    if (rpt_cap > 8) rpt_cap = 8;
+    if (wa > 32) throw std::runtime_error("panel leaf: width above 32");
+    // Registers per row and lane, by the leaf's width, and rows per quad: 32
+    // values a thread, 64 (the most its registers hold) where that brings the
+    // grid within the target workgroup count or the leaf into one workgroup.
+    const int nc = wa <= 8 ? 2 : (wa <= 16 ? 4 : 8);
+    int nq = 32 / nc;
     // the caller's preferred grid, capped by what the leaf's exchange holds
     const int target = std::min(pw.target_wgs, LEAF_GMAX);
-    int rpt = 1;
-    int G = ceil_div(m, PT * rpt);
-    while (G > target && rpt < rpt_cap) {
-        rpt *= 2;
-        G = ceil_div(m, PT * rpt);
-    }
+    auto grid = [&](int q) { return ceil_div(m, 16 * q * NWV); };
+    if (grid(nq) > target || (grid(nq) > 1 && grid(2 * nq) == 1)) nq *= 2;
+    const int G = grid(nq);
     if (G > LEAF_GMAX)
         throw std::runtime_error("panel leaf: panel too tall for the leaf's workgroup limit");
-    if (wa <= 8)
-        launch_leaf_w<T, 8>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, G, rpt, s);
-    else if (wa <= 16)
-        launch_leaf_w<T, 16>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, G, rpt, s);
-    else if (wa <= 32)
-        launch_leaf_w<T, 32>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, G, rpt, s);
-    else
-        throw std::runtime_error("panel leaf: width above 32");
+    const int threads = G > 1 ? PT : 64 * ceil_div(m, 16 * nq);
+#define SLA_LEAF(NCV, NQV) \
+    launch_leaf<T, NCV, NQV>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, threads, G, s)
+    if (nc == 2) {
+        if (nq == 16) SLA_LEAF(2, 16);
+        else SLA_LEAF(2, 32);
+    } else if (nc == 4) {
+        if (nq == 8) SLA_LEAF(4, 8);
+        else SLA_LEAF(4, 16);
+    } else {
+        if (nq == 4) SLA_LEAF(8, 4);
+        else SLA_LEAF(8, 8);
+    }
+#undef SLA_LEAF
     return 0;  // the mailbox exchange adds no barrier arrivals
 }
 

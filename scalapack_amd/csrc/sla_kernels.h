@@ -78,20 +78,22 @@ void convert_f64_f32(int m, int n, const double *A, int lda, float *B, int ldb, 
 
 // ---- panel leaf (PDGETF2 on <= 32 columns) --------------------------------
 // Mailbox of the leaf's per-column exchange: 2 regions x 32 column blocks of
-// PANEL_MAIL_COL 64-bit words -- PANEL_MAIL_GMAX candidates of up to 33 words
-// (row index, 32 values), then the 32 words of row j at PANEL_MAIL_ROWJ.
+// PANEL_MAIL_COL 64-bit words -- PANEL_MAIL_GMAX candidate rows of up to
+// PANEL_MAIL_CW values, then (at PANEL_MAIL_POS) their positions.
 // Every word holds the empty pattern (all ones) until a launch writes it.
 constexpr int PANEL_MAIL_GMAX = 128;
-constexpr int PANEL_MAIL_ROWJ = PANEL_MAIL_GMAX * 33;
-constexpr int PANEL_MAIL_COL = PANEL_MAIL_ROWJ + 32;
+constexpr int PANEL_MAIL_CW = 32;
+constexpr int PANEL_MAIL_POS = PANEL_MAIL_GMAX * PANEL_MAIL_CW;
+constexpr int PANEL_MAIL_COL = PANEL_MAIL_POS + PANEL_MAIL_GMAX;
 constexpr size_t PANEL_MAIL_REGION = 32 * (size_t)PANEL_MAIL_COL;
 constexpr size_t PANEL_MAIL_WORDS = 2 * PANEL_MAIL_REGION;
 
-// Host-side record of the mailbox's last launch (whose words the next
-// launch empties) and the launch count (whose parity picks the region).
+// Host-side record of the last launch that used the mailbox (whose words the
+// next one empties) and the count of such launches (whose parity picks the
+// region); a leaf of one workgroup does not use it.
 struct PanelMailState {
     unsigned launches = 0;
-    int prev_wa = 0, prev_g = 0, prev_cs = 0;
+    int prev_wa = 0, prev_g = 0;
 };
 
 template <typename T>
@@ -103,6 +105,7 @@ struct PanelWork {
     int *zero_col;       // min over zero pivots of the 1-based column (INT_MAX: none)
     uint64_t spin_limit; // wall-clock ticks a barrier may wait
     int target_wgs;      // preferred number of workgroups per leaf launch
+    int num_cus;         // CUs of the device
 };
 
 // Factors the m x wa leaf at A (global rows row0.., columns col0.. relative to
