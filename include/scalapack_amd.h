@@ -178,7 +178,8 @@ int sla_get_stats(sla_handle_t h, int cls, double *ms, double *work, long long *
  * aid): ms = summed execution intervals from the first workgroup's start to
  * the last workgroup's end on the device wall clock (the stream's event pair
  * also counts the wait for CUs held by the look-ahead panel stream),
- * work = summed 2 m n k flops of the 128 x 128-tiled interiors. */
+ * work = summed 2 m n k flops of those launches (low-precision updates: of
+ * their 128 x 128-tiled interiors). */
 int sla_get_update_exec(sla_handle_t h, double *ms, double *work, long long *launches);
 int sla_reset_stats(sla_handle_t h);
 

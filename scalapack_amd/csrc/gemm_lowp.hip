@@ -752,45 +752,35 @@ void sgemm_nn_sub(int m, int n, int k, const float *A, int lda, const float *B, 
                   unsigned long long *stamp)
 {
     if (m <= 0 || n <= 0 || k <= 0) return;
-    if (!trailing && gemm_small<float>(m, n, k, A, lda, B, ldb, C, ldc, s)) return;
     const int mf = (m / 128) * 128, nf = (n / 128) * 128;
-    if (mf > 0 && nf > 0 && k % 16 == 0 && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 &&
-        aligned16(A) && aligned16(B) && aligned16(C)) {
+    if (trailing && mf > 0 && nf > 0 && k % 16 == 0 && lda % 4 == 0 && ldb % 4 == 0 &&
+        ldc % 4 == 0 && aligned16(A) && aligned16(B) && aligned16(C)) {
         const int tiles = (mf / 128) * (nf / 128);
         const int grid = (max_wgs >= 8 && tiles > max_wgs) ? (max_wgs / 8) * 8 : tiles;
-        if (trailing) {
-            // reserve_lds: LDS the kernel does not use, reserved so that at
-            // most floor(LDS per CU / reserve_lds) workgroups share a CU and
-            // registers stay free for the panel running beside the update
-            if (reserve_lds > 0) {
-                static int attr_set = 0;
-                if (reserve_lds > attr_set) {
-                    SLA_HIP(hipFuncSetAttribute(
-                        reinterpret_cast<const void *>(&sgemm_nn_sub_direct_kernel<1>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, reserve_lds));
-                    attr_set = reserve_lds;
-                }
+        // reserve_lds: LDS the kernel does not use, reserved so that at most
+        // floor(LDS per CU / reserve_lds) workgroups share a CU and registers
+        // stay free for the panel running beside the update
+        if (reserve_lds > 0) {
+            static int attr_set = 0;
+            if (reserve_lds > attr_set) {
+                SLA_HIP(hipFuncSetAttribute(
+                    reinterpret_cast<const void *>(&sgemm_nn_sub_direct_kernel<1>),
+                    hipFuncAttributeMaxDynamicSharedMemorySize, reserve_lds));
+                attr_set = reserve_lds;
             }
-            hipLaunchKernelGGL(sgemm_nn_sub_direct_kernel<1>, dim3(grid), dim3(256),
-                               (unsigned)std::max(0, reserve_lds), s, mf, nf, k, A, lda, B, ldb, C,
-                               ldc, stamp);
         }
-        else
-            hipLaunchKernelGGL(sgemm_nn_sub_direct_kernel<0>, dim3((mf / 128) * (nf / 128)),
-                               dim3(256), 0, s, mf, nf, k, A, lda, B, ldb, C, ldc,
-                               (unsigned long long *)nullptr);
+        hipLaunchKernelGGL(sgemm_nn_sub_direct_kernel<1>, dim3(grid), dim3(256),
+                           (unsigned)std::max(0, reserve_lds), s, mf, nf, k, A, lda, B, ldb, C, ldc,
+                           stamp);
         SLA_LAUNCH_CHECK();
         if (m > mf)
-            sgemm_nn_sub(m - mf, n, k, A + mf, lda, B, ldb, C + mf, ldc, s, trailing, max_wgs,
-                         reserve_lds);
+            gemm_tile_sub<float>(false, m - mf, n, k, A + mf, lda, B, ldb, C + mf, ldc, s, true);
         if (n > nf)
-            sgemm_nn_sub(mf, n - nf, k, A, lda, B + (size_t)nf * ldb, ldb, C + (size_t)nf * ldc,
-                         ldc, s, trailing, max_wgs, reserve_lds);
+            gemm_tile_sub<float>(false, mf, n - nf, k, A, lda, B + (size_t)nf * ldb, ldb,
+                                 C + (size_t)nf * ldc, ldc, s, true);
         return;
     }
-    hipLaunchKernelGGL((gemm_lp_edge_kernel<float, false>), dim3(ceil_div(m, 16), ceil_div(n, 16)),
-                       dim3(256), 0, s, m, n, k, A, lda, B, ldb, C, ldc);
-    SLA_LAUNCH_CHECK();
+    gemm_tile_sub<float>(false, m, n, k, A, lda, B, ldb, C, ldc, s, trailing, max_wgs, false, stamp);
 }
 
 void gemm_bf16_nn_sub(int m, int n, int k, const __bf16 *Ap, int ldak, const __bf16 *Bp, int ldbk,

@@ -5,7 +5,7 @@
 //   PDGETF2 on A(J:M, J:J+JB)                  -> panel()  (recursive, below)
 //   PDLASWP on the columns left and right of it -> laswp_pairs + laswp_apply
 //   PDTRSM  U12 <- L11^{-1} A12                  -> trsm_llnu
-//   PDGEMM  A22 <- A22 - L21 U12                 -> dgemm_nn_sub (MFMA)
+//   PDGEMM  A22 <- A22 - L21 U12                 -> gemm_tile_sub (MFMA)
 // The panel is factored recursively: halves of the column block are split
 // until leaves of <= 32 columns, which one device-wide-barrier kernel
 // factors; between halves the same swap / trsm / gemm steps update the right
@@ -258,6 +258,7 @@ struct Lu {
     int *ipiv;  // device, indexed by global row (0-based), 1-based values
     PanelWork<T> pw;
     int schur = SCHUR_NATIVE;  // precision of the outer trailing update
+    bool beside = false;       // the next trailing update runs beside a panel
     bool l_packed = false;     // L21 of the current block column is packed
     hipStream_t s_main = nullptr, s_panel = nullptr;  // update stream, panel stream
     const T *inv_of[2] = {nullptr, nullptr};  // L11 whose inverses each stream's area holds
@@ -400,6 +401,11 @@ struct Lu {
                 update(M - jn, jb2, jb, at(jn, j), at(j, jn), at(jn, jn), s0);
                 SLA_HIP(hipEventRecord(h.ev_next, s0));
                 SLA_HIP(hipStreamWaitEvent(s1, h.ev_next, 0));
+                // a trailing update that outlasts a leaf: the leaf has to start
+                // beside it, not after it
+                const double update_us = 2.0 * (M - jn) * (N - jn - jb2) * jb / 50e6;
+                beside = s0 != s1;
+                pw.beside = beside && update_us > 100.0;
                 panel(jn, jn, jb2, jn, jn + jb2, s1);
                 make_pairs(jn, jn + jb2, q ^ 1, s1);
                 SLA_HIP(hipEventRecord(h.ev_panel, s1));
@@ -410,6 +416,7 @@ struct Lu {
             if (rest > 0) {
                 trsm(jb, rest, at(j, j), at(j, c), s0);
                 if (jn < M) update(M - jn, rest, jb, at(jn, j), at(j, c), at(jn, c), s0);
+                beside = false;
             }
             if (has_next) SLA_HIP(hipStreamWaitEvent(s0, h.ev_panel, 0));
         }
@@ -423,7 +430,7 @@ void Lu<double>::gemm(int m, int n, int k, const double *a, const double *b, dou
 {
     if (m <= 0 || n <= 0 || k <= 0) return;
     h.timing_begin(CAT_GEMM_PANEL, s);
-    dgemm_nn_sub(m, n, k, a, lda, b, lda, c, lda, s);
+    gemm_tile_sub<double>(false, m, n, k, a, lda, b, lda, c, lda, s);
     h.timing_end(2.0 * m * n * k, s);
 }
 
@@ -433,8 +440,9 @@ void Lu<double>::update(int m, int n, int k, const double *l21, const double *u1
 {
     if (m <= 0 || n <= 0 || k <= 0) return;
     h.timing_begin(CAT_GEMM, s);
-    unsigned long long *st = h.next_kstamp(2.0 * (m / 128 * 128) * (n / 128 * 128) * k);
-    dgemm_nn_sub(m, n, k, l21, lda, u12, lda, c, lda, s, true, h.update_cus, st);
+    unsigned long long *st = h.next_kstamp(2.0 * m * n * k);
+    gemm_tile_sub<double>(false, m, n, k, l21, lda, u12, lda, c, lda, s, true,
+                          GEMM_TILE_WGS_PER_CU * h.update_cus, beside, st);
     h.timing_end(2.0 * m * n * k, s);
 }
 
@@ -466,7 +474,7 @@ void Lu<float>::gemm(int m, int n, int k, const float *a, const float *b, float 
 {
     if (m <= 0 || n <= 0 || k <= 0) return;
     h.timing_begin(CAT_GEMM_PANEL, s);
-    sgemm_nn_sub(m, n, k, a, lda, b, lda, c, lda, s);
+    gemm_tile_sub<float>(false, m, n, k, a, lda, b, lda, c, lda, s);
     h.timing_end(2.0 * m * n * k, s);
 }
 

@@ -10,12 +10,12 @@
 //   1. every wave finds the largest |v| among its rows of position >= j (ties
 //      to the lowest position, as IDAMAX) and posts that row to LDS together
 //      with 1 / v; one workgroup barrier; every wave folds the posts itself;
-//   2. with more than one workgroup, each publishes its candidate row (the
-//      columns from j on, the reciprocal, the position) in mailbox words of
-//      column j and gathers the other G - 1; each word is written once per
-//      launch and starts out empty, so a word that is no longer empty holds
-//      this column's value: one round trip, no counter; every wave reduces
-//      the G candidates in the same total order, so all agree on p;
+//   2. with more than one workgroup, each publishes its candidate (value,
+//      position and row) in mailbox words of column j; each word is written
+//      once per launch and starts out empty, so a word that is no longer empty
+//      holds this column's value: no counter, no barrier.  Every wave gathers
+//      the G values and positions, reduces them in the same total order, so
+//      all agree on p, and fetches that row;
 //   3. rows of position > j are scaled by the reciprocal (the reference's
 //      ONE / GMAX multiply, pdgetf2.f:224) and updated a -= l * u with one fma.
 // The rows are written to their final positions at the end, and PDGETF2's
@@ -40,12 +40,19 @@
 // path 440 ns within an XCD and 500 - 620 ns between two (ping-pong of two
 // workgroups).  So a leaf of at most 32 workgroups puts them all on one XCD, a
 // different one from leaf to leaf, because the trailing update beside it is
-// dealt evenly over all of them.
+// dealt evenly over all of them.  The pivot row is fetched once the pivot is
+// known: gathering all G candidate rows in one trip, to LDS, took 85 us at m =
+// 2000 where this takes 77, and 57 KB of LDS where this takes 13.
+//
+// A workgroup of four waves with at most 128 registers starts beside the
+// trailing update (which leaves that much of every CU free, gemm_tile.hip).
+// There it takes 180 - 220 us instead of 80: every instruction of its chain
+// waits for the update's.
 //
 // Measured on 32 FP64 columns, alone on the GPU, us per leaf, before (all
 // columns unrolled, rows interchanged in registers, the workgroups spread over
-// the XCDs) and now: m = 100: 125, 37; 1000: 136, 78; 4000: 149, 90; 16384:
-// 165, 95; 32768: 183, 121.
+// the XCDs) and now: m = 100: 125, 36; 1000: 136, 79; 4000: 149, 80; 8192: 158,
+// 81; 16384: 165, 101; 32768: 183, 126.
 //
 // Mailbox: two regions of 32 column blocks; launch L uses region L & 1 and
 // refills the words launch L - 1 wrote in region (L + 1) & 1 -- that launch
@@ -61,8 +68,7 @@ namespace sla {
 
 namespace {
 
-constexpr int PT = 512;          // threads per workgroup at most (8 waves)
-constexpr int NWV = PT / 64;
+constexpr int NWV = 8;           // waves per workgroup at most
 constexpr int LEAF_GMAX = 128;   // workgroups per leaf launch at most
 constexpr int XCDS = 8, XCD_CUS = 32;  // the dies of the GPU and the CUs of one
 static_assert(LEAF_GMAX <= PANEL_MAIL_GMAX, "mailbox too small for the leaf's grid");
@@ -178,24 +184,19 @@ __device__ __forceinline__ void quad_bcast(float (&v)[NQ])
                                              0, __builtin_bit_cast(int, v[q]), S * 0x55, 0xf, 0xf, false));
 }
 
-// Words of one candidate: the row, 4 NC values in register order, lane by lane.
-// In LDS a row takes 34 words: that spreads column j of all candidates over the
-// banks and keeps the rows 16-byte aligned.
-constexpr int CW = PANEL_MAIL_CW, CWL = 34;
+// A row in LDS: 4 NC values in register order, lane by lane; 34 words apart, which
+// spreads one column of all rows over the banks and keeps them 16-byte aligned.
+constexpr int CWL = 34;
 
 template <typename T>
 struct alignas(16) LeafLds {
     T wrow[2][NWV][CWL];          // each wave's candidate, by column parity
     int wpos[2][NWV];             // its position; INT_MAX: no candidate
+    T prow[NWV][CWL];             // the pivot row, a copy for each wave that fetched it
     T u[32][CWL];                 // the pivot rows of the leaf
     int s_pv[32];                 // interchange of each column; -1: a zero pivot, none
     int s_dst[64], s_src[64], s_npair;
-    int s_abort;
-};
-template <typename T, bool SOLO>
-struct alignas(16) LeafCands {
-    T rows[SOLO ? 1 : LEAF_GMAX][CWL];
-    uint64_t pos[SOLO ? 1 : LEAF_GMAX];  // position, XCD in the upper half
+    int s_abort[2];               // a wait gave up, by column parity
 };
 
 struct LeafArgs {
@@ -215,74 +216,35 @@ __device__ __forceinline__ void post_word(uint64_t *p, uint64_t v, bool local)
     else coherent_store(p, v);
 }
 
-// Publishes the workgroup's candidate of column j (row src, position cpos;
-// INT_MAX: none) and gathers everyone's into LDS.  Only the registers below
-// `live` hold columns right of j.  The position word's upper half carries the
-// XCD.  An abort (sl.s_abort) leaves what was gathered so far.
+// Publishes the workgroup's candidate of column j: its row, its value and its
+// position (INT_MAX: none), whose word's upper half carries the XCD.  One wave.
 template <typename T, int NC>
-__device__ __forceinline__ void exchange(const LeafArgs &ar, int j, int live, bool local,
-                                         const T *src, int cpos, LeafLds<T> &sl,
-                                         LeafCands<T, false> &sc)
+__device__ __forceinline__ void publish(const LeafArgs &ar, uint64_t *cb, bool local, const T *src,
+                                        T val, int cpos, int lane)
 {
-    const int G = ar.G, tid = threadIdx.x, lane = tid & 63;
-    uint64_t *cb = ar.box + (size_t)j * PANEL_MAIL_COL;
-    constexpr int NV = 4 * NC;  // value words of a candidate
-    if (tid < NV + 1) {
-        uint64_t *mine = cb + (size_t)ar.g * CW;
-        if (lane < NV) {
-            if (lane % NC < live) post_word(&mine[lane], mail_word(src[lane]), local);
-        } else {
-            post_word(&cb[PANEL_MAIL_POS + ar.g], ((uint64_t)ar.xcd << 32) | (uint32_t)cpos, local);
-        }
+    constexpr int NV = 4 * NC;  // values of a row
+    if (lane < NV + 2) {
+        const int at = lane < NV ? ar.g * PANEL_MAIL_CW + lane
+                                 : (lane == NV ? PANEL_MAIL_VAL : PANEL_MAIL_POS) + ar.g;
+        const uint64_t w = lane < NV   ? mail_word(src[lane])
+                         : lane == NV ? mail_word(val)
+                                      : ((uint64_t)ar.xcd << 32) | (uint32_t)cpos;
+        post_word(&cb[at], w, local);
     }
-    // gather: NV threads per candidate for the values, one for its position,
-    // GL candidates a pass.  All loads of a pass are in flight before the first
-    // is looked at; a word still empty is loaded again.
-    constexpr int per = PT / NV, GL = 2;  // an exchanging launch has PT threads
-    const int e = tid % NV, g0 = tid / NV;
-    const bool want = e % NC < live;
-    const unsigned wp = PANEL_MAIL_POS + min(tid, G - 1);
-    bool nopos = tid < G;
-    unsigned it = 0;
-    for (int gb = 0; gb < G; gb += per * GL) {
-        unsigned w[GL];
-        bool miss[GL];
-#pragma unroll
-        for (int k = 0; k < GL; k++) {
-            const int g = gb + g0 + k * per;
-            miss[k] = want && g < G;
-            w[k] = min(g, G - 1) * CW + e;
-        }
-        for (;;) {
-            uint64_t v[GL];
-#pragma unroll
-            for (int k = 0; k < GL; k++) v[k] = coherent_load(&cb[w[k]]);
-            const uint64_t vp = coherent_load(&cb[wp]);
-            bool again = false;
-#pragma unroll
-            for (int k = 0; k < GL; k++) {
-                if (miss[k] && v[k] != MAIL_EMPTY) {
-                    sc.rows[gb + g0 + k * per][e] = mail_value<T>(v[k]);
-                    miss[k] = false;
-                }
-                again = again || miss[k];
-            }
-            if (nopos && vp != MAIL_EMPTY) {
-                sc.pos[tid] = vp;
-                nopos = false;
-            }
-            if (!again && !nopos) break;
-            if ((++it & 15u) == 0) {
-                if (coherent_load(ar.abort_flag)) sl.s_abort = 1;
-                else if (wall_clock64() - ar.t0 > ar.spin_limit) {
-                    coherent_store(ar.abort_flag, 1);
-                    sl.s_abort = 1;
-                }
-                if (sl.s_abort) break;
-            }
-        }
+}
+
+// Whether a wait goes on: false after spin_limit or when another wait gave up.
+__device__ __forceinline__ bool keep_waiting(const LeafArgs &ar, unsigned &it, int *s_abort)
+{
+    if ((++it & 15u) != 0) return true;
+    bool on = true;
+    if (coherent_load(ar.abort_flag)) on = false;
+    else if (wall_clock64() - ar.t0 > ar.spin_limit) {
+        coherent_store(ar.abort_flag, 1);
+        on = false;
     }
-    __syncthreads();
+    if (!on) *s_abort = 1;
+    return on;
 }
 
 // x[0] .. x[NC-1] rotated down by one.  Written out by recursion: as a loop it
@@ -318,8 +280,7 @@ __device__ __forceinline__ void update_rows(T (&x)[NQ][NC], const T (&l)[NQ], co
 // update; its multipliers stay.
 template <typename T, int NC, int NQ, bool SOLO>
 __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][NC],
-                                          int (&pos)[NQ], bool &local, LeafLds<T> &sl,
-                                          LeafCands<T, SOLO> &sc)
+                                          int (&pos)[NQ], bool &local, bool &dead, LeafLds<T> &sl)
 {
     typedef T v2_t __attribute__((ext_vector_type(2)));
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, cg = lane & 3;
@@ -384,6 +345,8 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
     }
     if (!found && lane == 0) sl.wpos[pb][wave] = INT_MAX;
     __syncthreads();
+    // a wait of the column before that gave up: all waves see it here
+    if (!SOLO) dead = sl.s_abort[pb ^ 1] != 0;
     // the workgroup's: lane x looks at the candidate of wave x % 8
     int p, fw;
     bool nonzero = true;
@@ -397,7 +360,7 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
         hm = dpp_max<0x122, 0xf>(hm);
         hm = dpp_max<0x124, 0xf>(hm);
         hm = (uint32_t)__builtin_amdgcn_readfirstlane((int)hm);
-        const unsigned t = (unsigned)__ballot(h == hm) & 0xffu;
+        const unsigned t = (unsigned)__ballot(h == hm) & ((1u << NWV) - 1u);
         if (decides<T>(hm) && (t & (t - 1)) == 0) {
             fw = __builtin_ctz(t);
             p = __builtin_amdgcn_readlane(xp, fw);
@@ -410,13 +373,31 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
         pv = lane_read(xv, fw);
     }
     const T *prow = sl.wrow[pb][fw];
+    T u[NC];
 
     // 2. the other workgroups
     if constexpr (!SOLO) {
-        exchange<T, NC>(ar, j, live, local, prow, p, sl, sc);
-        const int G = ar.G, x = lane < G ? lane : 0;
-        const int xp = lane < G ? (int)sc.pos[x] : INT_MAX;
-        const T xv = sc.rows[x][S * NC];
+        uint64_t *cb = ar.box + (size_t)j * PANEL_MAIL_COL;
+        if (wave == nw - 1) publish<T, NC>(ar, cb, local, prow, pv, p, lane);
+        const int G = ar.G;
+        // values and positions of candidates lane and lane + 64
+        uint64_t kv[2], kp[2];
+        unsigned it = 0;
+        const int x0 = min(lane, G - 1), x1 = min(lane + 64, G - 1);
+        do {
+            kv[0] = coherent_load(&cb[PANEL_MAIL_VAL + x0]);
+            kp[0] = coherent_load(&cb[PANEL_MAIL_POS + x0]);
+            kv[1] = kv[0];
+            kp[1] = kp[0];
+            if (G > 64) {
+                kv[1] = coherent_load(&cb[PANEL_MAIL_VAL + x1]);
+                kp[1] = coherent_load(&cb[PANEL_MAIL_POS + x1]);
+            }
+        } while ((kv[0] == MAIL_EMPTY || kp[0] == MAIL_EMPTY || kv[1] == MAIL_EMPTY ||
+                  kp[1] == MAIL_EMPTY) &&
+                 keep_waiting(ar, it, &sl.s_abort[pb]));
+        int xp = lane < G ? (int)kp[0] : INT_MAX;
+        T xv = mail_value<T>(kv[0]);
         const uint32_t h = xp != INT_MAX ? mag_hi(xv) : 0u;
         const uint32_t hm = wave_max(h);
         const uint64_t t = __ballot(h == hm);
@@ -427,40 +408,47 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
             p = __builtin_amdgcn_readlane(xp, gw);
             pv = lane_read(xv, gw);
         } else {
-            uint64_t ck = 0;
-            int bg = 0;
-            p = INT_MAX;
-            for (int y = lane; y < G; y += 64) {
-                const int yp = (int)sc.pos[y];
-                const uint64_t yk = mag_key(sc.rows[y][S * NC], yp != INT_MAX, yp == j);
-                const bool take = yk > ck || (yk != 0 && yk == ck && yp < p);
-                ck = take ? yk : ck;
-                p = take ? yp : p;
-                bg = take ? y : bg;
+            uint64_t ck = mag_key(xv, xp != INT_MAX, xp == j);
+            int bg = lane;
+            if (G > 64) {
+                const int yp = lane + 64 < G ? (int)kp[1] : INT_MAX;
+                const T yv = mail_value<T>(kv[1]);
+                const uint64_t yk = mag_key(yv, yp != INT_MAX, yp == j);
+                if (yk > ck || (yk == ck && yp < xp)) {
+                    ck = yk;
+                    xp = yp;
+                    xv = yv;
+                    bg = lane + 64;
+                }
             }
+            p = ck != 0 ? xp : INT_MAX;
             const int l = wave_pick(ck, p);
             gw = __builtin_amdgcn_readlane(bg, l);
             nonzero = ck > 1;
-            pv = sc.rows[gw][S * NC];
+            pv = lane_read(xv, l);
         }
-        prow = sc.rows[gw];
         if (j == 0) {
             // from here on through the L2, if every workgroup is on this XCD
-            bool same = true;
-            for (int y = lane; y < G; y += 64)
-                same = same && (sc.pos[y] >> 32) == (sc.pos[0] >> 32);
-            local = __all(same);
+            local = __all((kp[0] >> 32) == ar.xcd && (kp[1] >> 32) == ar.xcd);
         }
+        // the pivot row: a word a lane (one request for the 256 bytes), then
+        // through the wave's own slot in LDS
+        const uint64_t *rw = cb + (size_t)gw * PANEL_MAIL_CW + lane % (4 * NC);
+        uint64_t w;
+        while ((w = coherent_load(rw)) == MAIL_EMPTY && keep_waiting(ar, it, &sl.s_abort[pb])) {
+        }
+        if (lane < 4 * NC) sl.prow[wave][lane] = mail_value<T>(w);
+        prow = sl.prow[wave];
     }
-
-    // 3. interchange, scaling, rank-1 update
-    T u[NC];
 #pragma unroll
     for (int i = 0; i < NC; i += 2) {
         const v2_t x = *reinterpret_cast<const v2_t *>(&prow[cg * NC + i]);
         u[i] = x[0];
         u[i + 1] = x[1];
     }
+    if (wave == (j & (nw - 1)) && lane < 4 * NC) sl.u[j][lane] = prow[lane];
+
+    // 3. interchange, scaling, rank-1 update
     T l[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; q++) l[q] = a[q][0];
@@ -478,7 +466,6 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
         // the pivot row with l = 1 becomes zero right of the diagonal
         l[q] = own ? T(1) : l[q] * rcp;
     }
-    if (wave == (j & (nw - 1)) && lane < 4 * NC) sl.u[j][lane] = prow[lane];
     if (tid == 0) sl.s_pv[j] = nonzero ? p : -1;
     if (cg >= S) {
 #pragma unroll
@@ -495,8 +482,8 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
 // stride: the leaf's workgroups are every stride-th of the launch (the others
 // leave at once): with 8, the number of XCDs over which consecutive workgroups
 // are dealt, they share one XCD and its L2 (checked in column 0).
-template <typename T, int NC, int NQ, bool SOLO>
-__global__ __launch_bounds__(PT) void panel_leaf_kernel(
+template <typename T, int NC, int NQ, bool SOLO, int PT, int WPE>
+__global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(WPE))) void panel_leaf_kernel(
     T *__restrict__ A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0,
     int *__restrict__ ipiv, uint64_t *__restrict__ mail, int region, int prev_wa, int prev_g,
     int *abort_flag, int *zero_col, uint64_t spin_limit, int stride, int first)
@@ -509,18 +496,20 @@ __global__ __launch_bounds__(PT) void panel_leaf_kernel(
     const int base = (g * nw + wave) * (16 * NQ) + rg;  // row q of this quad: base + 16 q
 
     __shared__ LeafLds<T> sl;
-    __shared__ LeafCands<T, SOLO> sc;
-    if (tid == 0) sl.s_abort = 0;
+    if (tid < 2) sl.s_abort[tid] = 0;
 
     if constexpr (!SOLO) {
         // empty the words the previous launch that used the mailbox wrote (the
         // other region): columns < prev_wa, its prev_g candidates
         uint64_t *o = mail + (size_t)(region ^ 1) * PANEL_MAIL_REGION;
-        const int per = prev_g * (CW + 1);
+        const int per = prev_g * (PANEL_MAIL_CW + 2);
         for (int jj = 0; jj < prev_wa; jj++)
             for (int e = g * (int)blockDim.x + tid; e < per; e += G * (int)blockDim.x)
                 coherent_store(&o[(size_t)jj * PANEL_MAIL_COL +
-                                  (e < prev_g * CW ? e : PANEL_MAIL_POS + e - prev_g * CW)],
+                                  (e < prev_g * PANEL_MAIL_CW ? e
+                                   : e < prev_g * (PANEL_MAIL_CW + 1)
+                                       ? PANEL_MAIL_VAL + e - prev_g * PANEL_MAIL_CW
+                                       : PANEL_MAIL_POS + e - prev_g * (PANEL_MAIL_CW + 1))],
                                MAIL_EMPTY);
     }
 
@@ -544,13 +533,13 @@ __global__ __launch_bounds__(PT) void panel_leaf_kernel(
     __syncthreads();
     // After the last column of a group of four the registers rotate by one.
     // Nothing in the loop writes to global memory but the exchange: the waits
-    // for a store's completion would join the chain.  After an abort the
-    // workgroup leaves at the end of the group.
+    // for a store's completion would join the chain.
+    bool dead = false;  // uniform
 #pragma unroll 1
-    for (int t = 0; t < NC; t++) {
-        const int je = (!SOLO && sl.s_abort) ? 0 : min(4 * t + 4, wa);
+    for (int t = 0; t < NC && !dead; t++) {
 #pragma unroll 1
-        for (int j = 4 * t; j < je; j++) leaf_step<T, NC, NQ, SOLO>(ar, j, a, pos, local, sl, sc);
+        for (int j = 4 * t; j < min(4 * t + 4, wa) && !dead; j++)
+            leaf_step<T, NC, NQ, SOLO>(ar, j, a, pos, local, dead, sl);
 #pragma unroll
         for (int q = 0; q < NQ; q++) rotate_row<NC>(a[q], a[q][0]);
     }
@@ -560,7 +549,7 @@ __global__ __launch_bounds__(PT) void panel_leaf_kernel(
     // every column back to its register.  Of a pivot row the multipliers are
     // here; its part of U is in sl.u, in the register order of its column.
     __syncthreads();
-    if (!SOLO && sl.s_abort) return;
+    if (!SOLO && (sl.s_abort[0] | sl.s_abort[1])) return;
 #pragma unroll
     for (int q = 0; q < NQ; q++) {
         if (pos[q] >= 0) {
@@ -631,31 +620,63 @@ __global__ __launch_bounds__(PT) void panel_leaf_kernel(
     }
 }
 
-template <typename T, int NC, int NQ>
+template <typename T, int NC, int NQ, bool SOLO, int PT, int WPE>
 void launch_leaf(T *A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0, int *ipiv,
                  const PanelWork<T> &pw, int threads, int G, hipStream_t s)
 {
     PanelMailState &ms = *pw.mail_state;
-    if (G == 1) {
+    if (threads > PT) throw std::logic_error("panel leaf: workgroup larger than its kernel's");
+    if constexpr (SOLO) {
         // the mailbox and its record stay as the last exchanging launch left them
-        hipLaunchKernelGGL((panel_leaf_kernel<T, NC, NQ, true>), dim3(1), dim3(threads), 0, s, A,
-                           lda, m, wa, lcols, rcols, row0, col0, ipiv, pw.mail, 0, 0, 0,
+        hipLaunchKernelGGL((panel_leaf_kernel<T, NC, NQ, true, PT, WPE>), dim3(1), dim3(threads), 0,
+                           s, A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw.mail, 0, 0, 0,
                            pw.abort_flag, pw.zero_col, pw.spin_limit, 1, 0);
         SLA_LAUNCH_CHECK();
-        return;
+    } else {
+        // One XCD for all only on the whole GPU, and if each of its CUs takes one at
+        // most: beside a trailing update a CU has room for one.
+        const int stride = G <= XCD_CUS && pw.num_cus == XCDS * XCD_CUS ? XCDS : 1;
+        const int first = stride == 1 ? 0 : (int)(ms.launches % XCDS);
+        hipLaunchKernelGGL((panel_leaf_kernel<T, NC, NQ, false, PT, WPE>), dim3(G * stride),
+                           dim3(threads), 0, s, A, lda, m, wa, lcols, rcols, row0, col0, ipiv,
+                           pw.mail, (int)(ms.launches & 1u), ms.prev_wa, ms.prev_g, pw.abort_flag,
+                           pw.zero_col, pw.spin_limit, stride, first);
+        SLA_LAUNCH_CHECK();
+        ms.launches++;
+        ms.prev_wa = wa;
+        ms.prev_g = G;
     }
-    // One XCD holds at most a workgroup per CU, so only on the whole GPU and
-    // for at most as many workgroups as an XCD has CUs.
-    const int stride = G <= XCD_CUS && pw.num_cus == XCDS * XCD_CUS ? XCDS : 1;
-    const int first = stride > 1 ? (int)(ms.launches % XCDS) : 0;
-    hipLaunchKernelGGL((panel_leaf_kernel<T, NC, NQ, false>), dim3(G * stride), dim3(threads), 0, s,
-                       A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw.mail,
-                       (int)(ms.launches & 1u), ms.prev_wa, ms.prev_g, pw.abort_flag, pw.zero_col,
-                       pw.spin_limit, stride, first);
-    SLA_LAUNCH_CHECK();
-    ms.launches++;
-    ms.prev_wa = wa;
-    ms.prev_g = G;
+}
+
+// Rows per quad (V / NC) for V values a thread.
+template <typename T, int NC>
+void leaf_of_width(T *A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0,
+                   int *ipiv, const PanelWork<T> &pw, hipStream_t s)
+{
+    // V values a thread: 32 take at most 128 registers, 64 up to 256.
+    constexpr int V = NC == 2 ? 16 : 32;
+    auto grid = [&](int v, int waves) { return ceil_div(m, 16 * (v / NC) * waves); };
+#define SLA_LEAF(V, SOLO, PTV, WPE, threads, G)                                                     \
+    launch_leaf<T, NC, (V) / NC, SOLO, PTV, WPE>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, \
+                                                 threads, G, s)
+    // One workgroup while it holds the leaf: 78 us at m = 1000 and without the
+    // other streams' kernels in the way of an exchange.  (16 waves of 32 values
+    // instead of 8 of 64: 80 us; a SIMD's four waves wait for each other.)
+    if (grid(V, 8) == 1) return SLA_LEAF(V, true, 512, 4, 64 * grid(V, 1), 1);
+    if (grid(64, 8) == 1) return SLA_LEAF(64, true, 512, 2, 64 * grid(64, 1), 1);
+    // Then as many as one XCD runs, of the smallest kind: 82 us at m = 8192 with
+    // four waves.  Beside a long trailing update only those find room, so there
+    // they go on, across the XCDs: m = 16384 alone 139 us, with eight waves 95 us,
+    // but these wait for the end of the update.  The caller's preferred grid
+    // counts the largest kind.
+    const int target = std::min(pw.target_wgs, XCD_CUS);
+    if (grid(V, 4) <= (pw.beside ? std::min(4 * pw.target_wgs, LEAF_GMAX) : target))
+        return SLA_LEAF(V, false, 256, 4, 256, grid(V, 4));
+    if (grid(V, 8) <= target) return SLA_LEAF(V, false, 512, 4, 512, grid(V, 8));
+    if (grid(64, 8) > LEAF_GMAX)
+        throw std::runtime_error("panel leaf: panel too tall for the leaf's workgroup limit");
+    SLA_LEAF(64, false, 512, 2, 512, grid(64, 8));
+#undef SLA_LEAF
 }
 
 }  // namespace
@@ -664,33 +685,15 @@ template <typename T>
 unsigned panel_leaf(T *A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0,
                     int *ipiv, const PanelWork<T> &pw, hipStream_t s)
 {
-    if (wa > 32) throw std::runtime_error("panel leaf: width above 32");
-    // Registers per row and lane, by the leaf's width, and rows per quad: 32
-    // values a thread, 64 (the most its registers hold) where that brings the
-    // grid within the target workgroup count or the leaf into one workgroup.
-    const int nc = wa <= 8 ? 2 : (wa <= 16 ? 4 : 8);
-    int nq = 32 / nc;
-    // the caller's preferred grid, capped by what the leaf's exchange holds
-    const int target = std::min(pw.target_wgs, LEAF_GMAX);
-    auto grid = [&](int q) { return ceil_div(m, 16 * q * NWV); };
-    if (grid(nq) > target || (grid(nq) > 1 && grid(2 * nq) == 1)) nq *= 2;
-    const int G = grid(nq);
-    if (G > LEAF_GMAX)
-        throw std::runtime_error("panel leaf: panel too tall for the leaf's workgroup limit");
-    const int threads = G > 1 ? PT : 64 * ceil_div(m, 16 * nq);
-#define SLA_LEAF(NCV, NQV) \
-    launch_leaf<T, NCV, NQV>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, threads, G, s)
-    if (nc == 2) {
-        if (nq == 16) SLA_LEAF(2, 16);
-        else SLA_LEAF(2, 32);
-    } else if (nc == 4) {
-        if (nq == 8) SLA_LEAF(4, 8);
-        else SLA_LEAF(4, 16);
-    } else {
-        if (nq == 4) SLA_LEAF(8, 4);
-        else SLA_LEAF(8, 8);
-    }
-#undef SLA_LEAF
+    // registers per row and lane by the leaf's width
+    if (wa <= 8)
+        leaf_of_width<T, 2>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, s);
+    else if (wa <= 16)
+        leaf_of_width<T, 4>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, s);
+    else if (wa <= 32)
+        leaf_of_width<T, 8>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, s);
+    else
+        throw std::runtime_error("panel leaf: width above 32");
     return 0;  // the mailbox exchange adds no barrier arrivals
 }
 

@@ -5,23 +5,17 @@
 
 namespace sla {
 
-// ---- Schur-complement update: C[m x n] -= A[m x k] * B[k x n] (FP64) -----
-// trailing: the launch is PDGETRF's outer trailing update (a kernel symbol of
-// its own in traces); max_wgs > 0 caps its workgroups (a persistent grid that
-// leaves CUs to the panel running beside it).
-// stamp: launch_stamp pair of the interior (128 x 128-tiled) launch of a
-// trailing update, or null.
-void dgemm_nn_sub(int m, int n, int k, const double *A, int lda, const double *B, int ldb,
-                  double *C, int ldc, hipStream_t s, bool trailing = false, int max_wgs = 0,
-                  unsigned long long *stamp = nullptr);
-
-// ---- thin GEMMs of the recursive panel and TRSM (gemm_small.hip) -----------
-// C -= A * B when n, k <= 64 with m >= 4n (tall-narrow) or m, k <= 64
-// (short-wide); returns false (nothing launched) for other shapes.
-constexpr int SMALL_NMAX = 64, SMALL_KMAX = 64;
+// ---- C[m x n] -= op(A) * B (gemm_tile.hip), any shape and alignment --------
+// ta: op(A) = A^T (A k x m), else A (m x k).  trailing: the launch is PDGETRF's
+// outer trailing update (a kernel symbol of its own in traces); max_wgs > 0 caps
+// its workgroups (a persistent grid that leaves CUs to the panel running beside
+// it); beside: a panel runs on another stream meanwhile, so three workgroups a CU
+// instead of four; stamp: launch_stamp pair of a trailing update, or null.
 template <typename T>
-bool gemm_small(int m, int n, int k, const T *A, int lda, const T *B, int ldb, T *C, int ldc,
-                hipStream_t s);
+void gemm_tile_sub(bool ta, int m, int n, int k, const T *A, int lda, const T *B, int ldb, T *C,
+                   int ldc, hipStream_t s, bool trailing = false, int max_wgs = 0, bool beside = false,
+                   unsigned long long *stamp = nullptr);
+constexpr int GEMM_TILE_WGS_PER_CU = 4;  // workgroups that share a CU
 
 // ---- low-precision Schur-complement updates (FP32 storage) -----------------
 // C[m x n] -= A[m x k] * B[k x n], FP32 operands on FP32 MFMA.
@@ -79,11 +73,13 @@ void convert_f64_f32(int m, int n, const double *A, int lda, float *B, int ldb, 
 // ---- panel leaf (PDGETF2 on <= 32 columns) --------------------------------
 // Mailbox of the leaf's per-column exchange: 2 regions x 32 column blocks of
 // PANEL_MAIL_COL 64-bit words -- PANEL_MAIL_GMAX candidate rows of up to
-// PANEL_MAIL_CW values, then (at PANEL_MAIL_POS) their positions.
+// PANEL_MAIL_CW values, then their values in the column itself (PANEL_MAIL_VAL)
+// and their positions (PANEL_MAIL_POS).
 // Every word holds the empty pattern (all ones) until a launch writes it.
 constexpr int PANEL_MAIL_GMAX = 128;
 constexpr int PANEL_MAIL_CW = 32;
-constexpr int PANEL_MAIL_POS = PANEL_MAIL_GMAX * PANEL_MAIL_CW;
+constexpr int PANEL_MAIL_VAL = PANEL_MAIL_GMAX * PANEL_MAIL_CW;
+constexpr int PANEL_MAIL_POS = PANEL_MAIL_VAL + PANEL_MAIL_GMAX;
 constexpr int PANEL_MAIL_COL = PANEL_MAIL_POS + PANEL_MAIL_GMAX;
 constexpr size_t PANEL_MAIL_REGION = 32 * (size_t)PANEL_MAIL_COL;
 constexpr size_t PANEL_MAIL_WORDS = 2 * PANEL_MAIL_REGION;
@@ -106,6 +102,7 @@ struct PanelWork {
     uint64_t spin_limit; // wall-clock ticks a barrier may wait
     int target_wgs;      // preferred number of workgroups per leaf launch
     int num_cus;         // CUs of the device
+    bool beside = false; // a long trailing update runs on another stream meanwhile
 };
 
 // Factors the m x wa leaf at A (global rows row0.., columns col0.. relative to

@@ -69,6 +69,73 @@ __global__ __launch_bounds__(256) void trsm_llnu_strip_kernel(int m, int n, cons
     }
 }
 
+// m <= 32 rows: the solves between two leaves of a panel.  One wave takes 16
+// columns, the four lanes of a quad one of them, lane q rows q, q + 4, ..: a
+// step is one DPP move of the solved value and at most eight products a lane
+// with L's column from LDS.  The same products in the same order as above, in
+// 13 KB of LDS and one wave instead of 102 KB and four.
+constexpr int T32_NC = 16;
+
+template <int S, typename T>
+__device__ __forceinline__ T quad_lane(T v)
+{
+    if constexpr (sizeof(T) == 8) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, S * 0x55, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), S * 0x55, 0xf, 0xf, false);
+        return __builtin_bit_cast(T, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+    } else {
+        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                                                 S * 0x55, 0xf, 0xf, false));
+    }
+}
+
+template <int K, typename T>
+__device__ __forceinline__ void t32_steps(T (&b)[8], const T (*Ls)[33], int q)
+{
+    if constexpr (K < 31) {
+        const T x = quad_lane<K % 4>(b[K / 4]);
+        const T own = fma(-Ls[K][K / 4 * 4 + q], x, b[K / 4]);
+        b[K / 4] = q > K % 4 ? own : b[K / 4];
+#pragma unroll
+        for (int i = K / 4 + 1; i < 8; i++) b[i] = fma(-Ls[K][4 * i + q], x, b[i]);
+        t32_steps<K + 1>(b, Ls, q);
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(64) void trsm_llnu32_kernel(int m, int n, const T *__restrict__ L,
+                                                         int ldl, T *__restrict__ B, int ldb)
+{
+    __shared__ T Ls[32][33];  // column k of L in row k, zeros outside the triangle
+    __shared__ T Bs[T32_NC][33];
+    const int c0 = blockIdx.x * T32_NC, lane = threadIdx.x, r = lane & 31, h = lane >> 5;
+    const int c = lane >> 2, q = lane & 3;
+#pragma unroll
+    for (int k = 0; k < 32; k += 2) {
+        const int kk = k + h;
+        Ls[kk][r] = (r < m && kk < r) ? L[(size_t)r + (size_t)kk * ldl] : T(0);
+    }
+#pragma unroll
+    for (int k = 0; k < T32_NC; k += 2) {
+        const int cc = k + h;
+        Bs[cc][r] = (r < m && c0 + cc < n) ? B[(size_t)r + (size_t)(c0 + cc) * ldb] : T(0);
+    }
+    __syncthreads();
+    T b[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) b[i] = Bs[c][4 * i + q];
+    t32_steps<0>(b, Ls, q);
+#pragma unroll
+    for (int i = 0; i < 8; i++) Bs[c][4 * i + q] = b[i];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < T32_NC; k += 2) {
+        const int cc = k + h;
+        if (r < m && c0 + cc < n) B[(size_t)r + (size_t)(c0 + cc) * ldb] = Bs[cc][r];
+    }
+}
+
 // ---------------------------------------------------------------------------
 constexpr int TV_BS = 64, TV_NR = 16, TV_PART = TV_BS / 4;
 
@@ -532,6 +599,12 @@ void trsm_llnu(int m, int n, const T *L, int ldl, T *B, int ldb, hipStream_t s)
 {
     if (m <= 0 || n <= 0) return;
     if (m > TS_MAXM) throw std::logic_error("trsm_llnu: at most 256 rows per call");
+    if (m <= 32) {
+        hipLaunchKernelGGL(trsm_llnu32_kernel<T>, dim3(ceil_div(n, T32_NC)), dim3(64), 0, s, m, n, L,
+                           ldl, B, ldb);
+        SLA_LAUNCH_CHECK();
+        return;
+    }
     hipLaunchKernelGGL(trsm_llnu_strip_kernel<T>, dim3(ceil_div(n, TS_CW)), dim3(256), 0, s, m, n,
                        L, ldl, B, ldb);
     SLA_LAUNCH_CHECK();
@@ -555,7 +628,7 @@ template void trsm_llnu<float>(int, int, const float *, int, float *, int, hipSt
 // block's inverse operands are loaded during the current block's update.
 namespace {
 
-constexpr int TB_M = 512, TB_NC = 16, TB_LD = TB_NC + 1, TB_T = 512;
+constexpr int TB_M = 512, TB_NC = 16, TB_LD = TB_NC + 1;
 typedef double bd4_t __attribute__((ext_vector_type(4)));
 typedef float bf4_t __attribute__((ext_vector_type(4)));
 
@@ -596,15 +669,19 @@ __device__ __forceinline__ int mfma_row(int lk, int r)
     return sizeof(T) == 8 ? lk + 4 * r : 4 * lk + r;
 }
 
-template <typename T>
-__global__ __launch_bounds__(TB_T) void trsm_llnu_blocked_kernel(int m, int n,
-                                                                 const T *__restrict__ L, int ldl,
-                                                                 const T *__restrict__ inv,
-                                                                 T *__restrict__ B, int ldb)
+// MM: rows at most.  The panel's solves (MM <= 256) run beside the trailing
+// update, whose workgroups fill every CU four at a time: 256 threads and a strip
+// of MM rows fit where one of them has left, 512 threads with 70 KB of LDS wait
+// until a CU is nearly empty (22 us a solve alone, 155 us beside the update).
+template <typename T, int MM>
+__global__ __launch_bounds__(MM > 256 ? 512 : 256)
+__attribute__((amdgpu_waves_per_eu(4))) void trsm_llnu_blocked_kernel(
+    int m, int n, const T *__restrict__ L, int ldl, const T *__restrict__ inv, T *__restrict__ B,
+    int ldb)
 {
     using acc_t = typename std::conditional<sizeof(T) == 8, bd4_t, bf4_t>::type;
-    constexpr int NW = TB_T / 64;
-    __shared__ T Xs[TB_M][TB_LD];
+    constexpr int TB_T = MM > 256 ? 512 : 256, NW = TB_T / 64;
+    __shared__ T Xs[MM][TB_LD];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 15, lk = lane >> 4;
     const int c0 = blockIdx.x * TB_NC;
@@ -694,8 +771,14 @@ void trsm_llnu_blocked(int m, int n, const T *L, int ldl, T *B, int ldb, T *inv,
         hipLaunchKernelGGL(trsm_diag_inv_kernel<T>, dim3(nblk), dim3(1024), 0, s, m, L, ldl, inv);
         SLA_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(trsm_llnu_blocked_kernel<T>, dim3(ceil_div(n, TB_NC)), dim3(TB_T), 0, s, m,
-                       n, L, ldl, (const T *)inv, B, ldb);
+#define SLA_TB(MV, TV)                                                                            \
+    hipLaunchKernelGGL((trsm_llnu_blocked_kernel<T, MV>), dim3(ceil_div(n, TB_NC)), dim3(TV), 0, s, \
+                       m, n, L, ldl, (const T *)inv, B, ldb)
+    if (m <= 64) SLA_TB(64, 256);
+    else if (m <= 128) SLA_TB(128, 256);
+    else if (m <= 256) SLA_TB(256, 256);
+    else SLA_TB(512, 512);
+#undef SLA_TB
     SLA_LAUNCH_CHECK();
 }
 template void trsm_llnu_blocked<double>(int, int, const double *, int, double *, int, double *,
