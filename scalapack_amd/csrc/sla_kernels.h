@@ -176,6 +176,9 @@ struct TrsvWork {
     int *abort_flag;
     uint64_t spin_limit;
 };
+// The same for any number of right-hand sides in blocks of 256 rows (trsm.hip).
+void trsm_solve(TrsvOp op, int n, int nrhs, const double *A, int lda, double *X, int ldx,
+                hipStream_t s);
 // TA: storage type of the triangle, T: type of X and of the arithmetic
 // (<double, double>, <float, float>, <float, double>).
 template <typename TA, typename T>

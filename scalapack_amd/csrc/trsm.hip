@@ -23,6 +23,8 @@
 #include "sla_common.h"
 #include "sla_kernels.h"
 
+#include <algorithm>
+#include <cstddef>
 #include <type_traits>
 
 namespace sla {
@@ -758,7 +760,143 @@ __attribute__((amdgpu_waves_per_eu(4))) void trsm_llnu_blocked_kernel(
     }
 }
 
+// ---------------------------------------------------------------------------
+// trsm_tri: one diagonal block (at most 256 rows) of PDGETRS's solves for many
+// right-hand sides; the products with the rest of the triangle are GEMMs between
+// these launches (trsm_solve).  All four triangles are forward substitutions
+// with a lower triangle E of signed strides: E(i, j) = E[i rs + j cs], row i of X
+// at X[i xs]; U and L^T run from their last row up, U^T and L^T are read along
+// their columns.
+//
+// A workgroup of four waves keeps 16 columns of X in LDS and walks E in 32-row
+// blocks: one wave solves the diagonal block by substitution (a quad of lanes a
+// column, as trsm_llnu32_kernel; a non-unit diagonal as products with its
+// reciprocals), then all waves subtract E_ik X_k from the rows below on MFMA, 16
+// rows a tile, the first tile's E loaded before the solve it waits for.  Bound
+// by that chain, about 3 us per 32 rows, and not by the work: with the GEMMs
+// n = 5000 and 400 right-hand sides take 2.9 ms where sixteen at a time through
+// trsv_persistent took 96 ms.
+constexpr int TT_M = 256, TT_T = 256;
+
+template <int K, bool UNIT, typename T>
+__device__ __forceinline__ void tri_steps(T (&b)[8], const T (*Es)[33], const T *rd, int q)
+{
+    if constexpr (K < 32) {
+        if (!UNIT) {
+            const T x = b[K / 4] * rd[K];
+            b[K / 4] = q == K % 4 ? x : b[K / 4];
+        }
+        const T x = quad_lane<K % 4>(b[K / 4]);
+        const T own = fma(-Es[K][K / 4 * 4 + q], x, b[K / 4]);
+        b[K / 4] = q > K % 4 ? own : b[K / 4];
+#pragma unroll
+        for (int i = K / 4 + 1; i < 8; i++) b[i] = fma(-Es[K][4 * i + q], x, b[i]);
+        tri_steps<K + 1, UNIT>(b, Es, rd, q);
+    }
+}
+
+template <typename T, bool UNIT>
+__global__ __launch_bounds__(TT_T) void trsm_tri_kernel(int m, int n, const T *__restrict__ E,
+                                                        ptrdiff_t rs, ptrdiff_t cs,
+                                                        T *__restrict__ X, ptrdiff_t xs, size_t ldx)
+{
+    using acc_t = typename std::conditional<sizeof(T) == 8, bd4_t, bf4_t>::type;
+    constexpr int NW = TT_T / 64;
+    __shared__ T Xs[TT_M][TB_LD];
+    __shared__ T Es[32][33];  // the diagonal block, column k in row k
+    __shared__ T rd[32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lr = lane & 15, lk = lane >> 4, c0 = blockIdx.x * TB_NC;
+    const int nblk = (m + 31) / 32, m32 = 32 * nblk;
+    for (int idx = tid; idx < m32 * TB_NC; idx += TT_T) {
+        const int r = idx % m32, c = idx / m32;
+        Xs[r][c] = (r < m && c0 + c < n) ? X[r * xs + (size_t)(c0 + c) * ldx] : T(0);
+    }
+    // the 16 rows of tile t below block k, columns kr .. kr + 31 of E
+    auto load_tile = [&](T (&a)[8], int kr, int t, int ntile) {
+        const int row = kr + 32 + 16 * t + lr;
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            const int col = kr + 4 * s + lk;
+            a[s] = (t < ntile && row < m) ? E[row * rs + col * cs] : T(0);  // col < m: rows follow
+        }
+    };
+    for (int k = 0; k < nblk; k++) {
+        const int kr = 32 * k, ntile = (m32 - kr - 32) / 16;
+        // (the barrier at the end of the last block's update frees Es)
+        for (int idx = tid; idx < 1024; idx += TT_T) {
+            const int r = idx & 31, c = idx >> 5;
+            Es[c][r] = (c < r && kr + r < m) ? E[(kr + r) * rs + (kr + c) * cs] : T(0);
+        }
+        if (!UNIT && tid < 32) rd[tid] = kr + tid < m ? T(1) / E[(kr + tid) * (rs + cs)] : T(1);
+        T a[8];
+        load_tile(a, kr, wave, ntile);
+        __syncthreads();  // Es, and X_k's last update
+        if (wave == 0) {
+            const int c = lane >> 2, q = lane & 3;
+            T b[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) b[i] = Xs[kr + 4 * i + q][c];
+            tri_steps<0, UNIT>(b, Es, rd, q);
+#pragma unroll
+            for (int i = 0; i < 8; i++) Xs[kr + 4 * i + q][c] = b[i];
+        }
+        __syncthreads();  // X_k is final
+        if (ntile <= 0) break;
+        T xb[8];
+#pragma unroll
+        for (int s = 0; s < 8; s++) xb[s] = -Xs[kr + 4 * s + lk][lr];
+        for (int t = wave; t < ntile; t += NW) {
+            T an[8];
+            load_tile(an, kr, t + NW, ntile);
+            const int r0 = kr + 32 + 16 * t;
+            acc_t c;
+#pragma unroll
+            for (int r = 0; r < 4; r++) c[r] = Xs[r0 + mfma_row<T>(lk, r)][lr];
+#pragma unroll
+            for (int s = 0; s < 8; s++) c = mfma16x4<T>(a[s], xb[s], c);
+#pragma unroll
+            for (int r = 0; r < 4; r++) Xs[r0 + mfma_row<T>(lk, r)][lr] = c[r];
+#pragma unroll
+            for (int s = 0; s < 8; s++) a[s] = an[s];
+        }
+    }
+    for (int idx = tid; idx < m * TB_NC; idx += TT_T) {
+        const int r = idx % m, c = idx / m;
+        if (c0 + c < n) X[r * xs + (size_t)(c0 + c) * ldx] = Xs[r][c];
+    }
+}
+
 }  // namespace
+
+// X <- op(T)^{-1} X, n x nrhs: the diagonal blocks in order, each followed by the
+// product of its solution with the rest of its block column (row).
+void trsm_solve(TrsvOp op, int n, int nrhs, const double *A, int lda, double *X, int ldx,
+                hipStream_t s)
+{
+    if (n <= 0 || nrhs <= 0) return;
+    const bool fwd = op == TrsvOp::L || op == TrsvOp::UT;
+    const bool trans = op == TrsvOp::UT || op == TrsvOp::LT;
+    const ptrdiff_t rs = (fwd ? 1 : -1) * (trans ? (ptrdiff_t)lda : 1);
+    const ptrdiff_t cs = (fwd ? 1 : -1) * (trans ? 1 : (ptrdiff_t)lda);
+    const int nblk = ceil_div(n, TT_M);
+    for (int i = 0; i < nblk; i++) {
+        const int k0 = (fwd ? i : nblk - 1 - i) * TT_M, kb = std::min(TT_M, n - k0), k1 = k0 + kb;
+        const int first = fwd ? k0 : k1 - 1;  // the block's row 0 as the kernel counts
+        const double *E = A + (size_t)first + (size_t)first * lda;
+        const dim3 grid(ceil_div(nrhs, TB_NC));
+        if (op == TrsvOp::L || op == TrsvOp::LT)
+            hipLaunchKernelGGL((trsm_tri_kernel<double, true>), grid, dim3(TT_T), 0, s, kb, nrhs, E,
+                               rs, cs, X + first, (ptrdiff_t)(fwd ? 1 : -1), (size_t)ldx);
+        else
+            hipLaunchKernelGGL((trsm_tri_kernel<double, false>), grid, dim3(TT_T), 0, s, kb, nrhs, E,
+                               rs, cs, X + first, (ptrdiff_t)(fwd ? 1 : -1), (size_t)ldx);
+        SLA_LAUNCH_CHECK();
+        const int r0 = fwd ? k1 : 0, r1 = fwd ? n : k0;  // rows still to be solved
+        const double *off = trans ? A + (size_t)k0 + (size_t)r0 * lda : A + (size_t)r0 + (size_t)k0 * lda;
+        gemm_tile_sub<double>(trans, r1 - r0, nrhs, kb, off, lda, X + k0, ldx, X + r0, ldx, s);
+    }
+}
 
 template <typename T>
 void trsm_llnu_blocked(int m, int n, const T *L, int ldl, T *B, int ldb, T *inv, bool inv_ready,
