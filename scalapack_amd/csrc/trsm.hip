@@ -31,6 +31,24 @@ namespace sla {
 
 namespace {
 
+typedef double bd4_t __attribute__((ext_vector_type(4)));
+typedef float bf4_t __attribute__((ext_vector_type(4)));
+
+template <typename T>
+__device__ __forceinline__ auto mfma16x4(T a, T b, typename std::conditional<sizeof(T) == 8, bd4_t,
+                                                                            bf4_t>::type c)
+{
+    if constexpr (sizeof(T) == 8) return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// row of accumulator element r of lane (lr, lk) within a 16 x 16 tile
+template <typename T>
+__device__ __forceinline__ int mfma_row(int lk, int r)
+{
+    return sizeof(T) == 8 ? lk + 4 * r : 4 * lk + r;
+}
+
 constexpr int TS_CW = 16, TS_KB = 32, TS_MAXM = 256;
 
 template <typename T>
@@ -153,12 +171,26 @@ constexpr int TV_BS = 64, TV_NR = 16, TV_PART = TV_BS / 4;
 // Hand-off between blocks: a solved block publishes its values in a mailbox
 // of 64-bit words, each holding 32 bits of a value and the launch's epoch in
 // the upper half (a double takes two words), written with agent-coherent
-// stores.  A waiting workgroup polls the words themselves (wave 0, lane = row)
-// until every one carries the epoch -- one memory round trip from producer to
-// consumer, no separate flag and no store drain.  Stale words of earlier
-// launches hold older epochs; the mailbox is zeroed when allocated.  The next
-// off-diagonal block of the triangle is loaded into registers before the
-// wait, so the matrix read stays off the chain.
+// stores.  A waiting workgroup polls the words themselves until every one
+// carries the epoch -- one memory round trip from producer to consumer, no
+// separate flag and no store drain.  Stale words of earlier launches hold older
+// epochs; the mailbox is zeroed when allocated.  The next off-diagonal block of
+// the triangle is loaded into registers before the wait, so the matrix read
+// stays off the chain.
+//
+// Bound: the chain of n / 64 blocks, each a mailbox round trip (about 1.3 us),
+// a 64 x 64 product and the 64 steps of the diagonal block.  So all four waves
+// poll (a wave has at most four columns, not sixteen), and look at the abort
+// flag and the clock every 16th time only: the answer costs a trip of its own.
+// Two to sixteen right-hand sides go through the matrix cores, which takes the
+// product's reads of X from LDS down to one per 16 rows.  The diagonal block is
+// solved as four 16 x 16 triangles with one column in each row of 16 lanes, the
+// solved value passed on by a DPP move (4 cycles; a lane read through a scalar
+// register, with its hazards, took about twice as long) and every column of a
+// group of 16 at once, where one wave used to step through them in turn.
+// L and U solve together, n = 16384, us, before -> this: one right-hand side
+// 2027 -> 1863, four 3827 -> 2134, sixteen 12379 -> 2618; n = 1024: 148 -> 139,
+// 263 -> 153, 810 -> 182; n = 100: 33 -> 32, -, 93 -> 37.
 template <typename T>
 __device__ __forceinline__ uint32_t tv_half(T v, int w)
 {
@@ -181,23 +213,63 @@ __device__ __forceinline__ T tv_join(uint32_t lo, uint32_t hi)
     }
 }
 
+// The value of lane K of every row of 16 lanes, in all of them.
+template <int K, typename T>
+__device__ __forceinline__ T row_lane(T v)
+{
+    if constexpr (sizeof(T) == 8) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, 0x150 + K, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), 0x150 + K, 0xf, 0xf, false);
+        return __builtin_bit_cast(T, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+    } else {
+        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                                                 0x150 + K, 0xf, 0xf, false));
+    }
+}
+
+// Steps of a 16 x 16 triangle: lane l holds row l of b[0] and a row each of what
+// the solved values are to be subtracted from, b[1] .. b[3]; e[q][k (TV_BS + 1)]
+// is column k of the triangle and of those rows, rd the reciprocals of a non-unit
+// diagonal.  Lane l's solved value goes to x.  (Lanes already solved go on
+// subtracting; only x counts.)  The chain of a step is a product, a DPP move and
+// an fma; the other rows' are off it.
+template <int S, bool FORWARD, bool UNIT, typename T>
+__device__ __forceinline__ void tv_steps(T (&b)[4], T &x, const T *const (&e)[4], const T *rd, int l)
+{
+    if constexpr (S < 16) {
+        constexpr int K = FORWARD ? S : 15 - S;
+        const T v = row_lane<K>(UNIT ? b[0] : b[0] * rd[K]);
+        x = l == K ? v : x;
+#pragma unroll
+        for (int q = 0; q < 4; q++) b[q] = fma(-e[q][K * (TV_BS + 1)], v, b[q]);
+        tv_steps<S + 1, FORWARD, UNIT>(b, x, e, rd, l);
+    }
+}
+
 template <typename TA, typename T, bool FORWARD, bool TRANS, int NR>
 __global__ __launch_bounds__(256) void trsv_persistent_kernel(
     int n, int nrhs, const TA *__restrict__ A, int lda, T *X, int ldx, int *ticket,
     uint64_t *mail, unsigned epoch, int *abort_flag, uint64_t spin_limit)
 {
+    using acc_t = typename std::conditional<sizeof(T) == 8, bd4_t, bf4_t>::type;
     constexpr int WPV = sizeof(T) / 4;  // mailbox words per value
-    __shared__ int s_b, s_abort;
-    __shared__ T Xs[TV_BS][NR];
-    __shared__ T Part[4][TV_BS][NR + 1];
-    __shared__ T Ds[TV_BS][TV_BS + 1];  // diagonal block, row-major
+    constexpr bool MF = NR > 1;         // products on MFMA: wave w has rows 16 w ..
+    constexpr bool UNIT = (FORWARD != TRANS);  // L and L^T have a unit diagonal
+    constexpr int NC = MF ? 16 : 1;     // columns of the LDS arrays
+    __shared__ int s_b, s_abort[2];
+    __shared__ T Xs[2][TV_BS][NC];
+    __shared__ T Ys[NC][TV_BS + 1];
+    __shared__ T Part[MF ? 1 : 4][TV_BS];
+    __shared__ T Es[TV_BS][TV_BS + 1];  // diagonal block, column k of op(T) in row k
+    __shared__ T rd[TV_BS];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lr = lane & 15, lk = lane >> 4;
     const int nblk = ceil_div(n, TV_BS);
 
-    if (tid == 0) {
-        s_b = atomicAdd(ticket, 1);
-        s_abort = 0;
-    }
+    if (tid == 0) s_b = atomicAdd(ticket, 1);
+    if (tid < 2) s_abort[tid] = 0;
+    for (int i = tid; i < 2 * TV_BS * NC; i += 256) (&Xs[0][0][0])[i] = T(0);
     __syncthreads();
     const int t = s_b;
     if (t >= nblk) return;
@@ -208,150 +280,150 @@ __global__ __launch_bounds__(256) void trsv_persistent_kernel(
         return mail + ((((size_t)c * NR + j) * WPV + w) * TV_BS + r);
     };
 
-    // Diagonal block staged in LDS before any wait (it does not depend on
-    // other blocks); wave 0 lane r keeps 1 / U(r, r) and its right-hand side.
+    // The diagonal block, its reciprocals and the right-hand sides before any
+    // wait: they do not depend on other blocks.
     for (int idx = tid; idx < TV_BS * TV_BS; idx += 256) {
-        const int r = idx % TV_BS, k = idx / TV_BS;
-        Ds[r][k] = (r < rows && k < rows) ? (T)A[(size_t)(rb + r) + (size_t)(rb + k) * lda] : T(0);
+        const int r = idx % TV_BS, k = idx / TV_BS;  // stored element (r, k)
+        const T x = (r < rows && k < rows) ? (T)A[(size_t)(rb + r) + (size_t)(rb + k) * lda] : T(0);
+        if (TRANS) Es[r][k] = x;
+        else Es[k][r] = x;
     }
-    constexpr bool UNIT = (FORWARD != TRANS);  // L and L^T have a unit diagonal
-    T rdiag = T(1);
-    T rhs[NR];
+    if (!UNIT && tid < TV_BS) rd[tid] = tid < rows ? T(1) / (T)A[(size_t)(rb + tid) * (lda + 1)] : T(1);
+    // MF: element r of the lane is row 16 wave + mfma_row(lk, r), column lr;
+    // else thread (wave 0, lane) has row lane
+    T rhs[MF ? 4 : 1];
 #pragma unroll
-    for (int j = 0; j < NR; j++) rhs[j] = T(0);
-    if (wave == 0 && lane < rows) {
-        if (!UNIT) rdiag = T(1) / (T)A[(size_t)(rb + lane) * (lda + 1)];
-#pragma unroll
-        for (int j = 0; j < NR; j++)
-            if (j < nrhs) rhs[j] = X[(size_t)(rb + lane) + (size_t)j * ldx];
+    for (int r = 0; r < (MF ? 4 : 1); r++) {
+        const int row = MF ? 16 * wave + mfma_row<T>(lk, r) : lane, col = MF ? lr : 0;
+        rhs[r] = (row < rows && col < nrhs) ? X[(size_t)(rb + row) + (size_t)col * ldx] : T(0);
     }
 
-    T part[NR];
-#pragma unroll
-    for (int j = 0; j < NR; j++) part[j] = T(0);
-
-    // wave w covers k in [16w, 16w+16) of the 64 x 64 block A[rb.., cb..]
-    // (TRANS: of the block A[cb.., rb..], read down its columns); zero
-    // outside the block
+    // A 64 x 64 block of op(T) right of (left of) the diagonal block, 16 elements
+    // a thread.  MF: row 16 wave + lr, k = 16 lk ..; else row lane, k = 16 wave ..
+    const int prow = MF ? 16 * wave + lr : lane, pk = 16 * (MF ? lk : wave);
     TA a[TV_PART];
     auto load_block = [&](int s) {
         const int c = FORWARD ? s : nblk - 1 - s;
         const int cb = c * TV_BS, crows = min(TV_BS, n - cb);
-        const TA *Ar = TRANS ? A + (size_t)cb + (size_t)(rb + lane) * lda
-                             : A + (size_t)(rb + lane) + (size_t)cb * lda;
+        const TA *Ar = TRANS ? A + (size_t)cb + (size_t)(rb + prow) * lda
+                             : A + (size_t)(rb + prow) + (size_t)cb * lda;
         const size_t kstride = TRANS ? 1 : (size_t)lda;
 #pragma unroll
-        for (int kk = 0; kk < TV_PART; kk++) {
-            const int k = wave * TV_PART + kk;
-            a[kk] = (lane < rows && k < crows) ? Ar[(size_t)k * kstride] : TA(0);
-        }
+        for (int kk = 0; kk < TV_PART; kk++)
+            a[kk] = (prow < rows && pk + kk < crows) ? Ar[(size_t)(pk + kk) * kstride] : TA(0);
     };
     if (t > 0) load_block(0);
 
-    // Off-diagonal contributions, in dependency order.
+    // four sums of a quarter of the terms each: their rounding errors are half
+    // those of one long sum
+    acc_t acc[4] = {};
+    T part = T(0);
+    // Contributions of the solved blocks, in dependency order.  All threads poll:
+    // row lane of columns wave, wave + 4, ..; Xs and s_abort alternate, so one
+    // barrier a block is enough.
     for (int s = 0; s < t; s++) {
-        const int c = FORWARD ? s : nblk - 1 - s;
+        const int c = FORWARD ? s : nblk - 1 - s, sb = s & 1;
         const int crows = min(TV_BS, n - c * TV_BS);
-        if (wave == 0) {
-            uint32_t got[NR][WPV];
-            int ab = 0;
+        constexpr int JP = (NR + 3) / 4;  // columns a thread polls
+        if (lane < crows && wave < nrhs) {
             const uint64_t t0 = wall_clock64();
+            unsigned it = 0;
             for (;;) {
+                uint64_t got[JP][WPV];
                 bool ok = true;
-                if (lane < crows) {
 #pragma unroll
-                    for (int j = 0; j < NR; j++) {
-                        if (j < nrhs) {
+                for (int i = 0; i < JP; i++)
 #pragma unroll
-                            for (int w = 0; w < WPV; w++) {
-                                const uint64_t u = __hip_atomic_load(
-                                    mbox(c, j, w, lane), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                                got[j][w] = (uint32_t)u;
-                                ok = ok && (uint32_t)(u >> 32) == epoch;
-                            }
-                        }
+                    for (int w = 0; w < WPV; w++)
+                        got[i][w] = __hip_atomic_load(mbox(c, min(wave + 4 * i, nrhs - 1), w, lane),
+                                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                for (int i = 0; i < JP; i++)
+#pragma unroll
+                    for (int w = 0; w < WPV; w++) ok = ok && (uint32_t)(got[i][w] >> 32) == epoch;
+                if (ok) {
+#pragma unroll
+                    for (int i = 0; i < JP; i++)
+                        if (wave + 4 * i < nrhs)
+                            Xs[sb][lane][wave + 4 * i] =
+                                tv_join<T>((uint32_t)got[i][0], (uint32_t)got[i][WPV - 1]);
+                    break;
+                }
+                // the flag and the clock only now and then: the next poll waits
+                // for their answer
+                if ((++it & 15u) == 0) {
+                    if (__hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                        s_abort[sb] = 1;
+                        break;
                     }
-                }
-                if (__all(ok)) break;
-                if (__hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                    ab = 1;
-                    break;
-                }
-                if (wall_clock64() - t0 > spin_limit) {
-                    __hip_atomic_store(abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    ab = 1;
-                    break;
+                    if (wall_clock64() - t0 > spin_limit) {
+                        __hip_atomic_store(abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        s_abort[sb] = 1;
+                        break;
+                    }
                 }
                 // workgroups far behind the chain poll less often
                 if (t - s > 4) __builtin_amdgcn_s_sleep(16);
-                else __builtin_amdgcn_s_sleep(1);
             }
-#pragma unroll
-            for (int j = 0; j < NR; j++)
-                Xs[lane][j] = (lane < crows && j < nrhs) ? tv_join<T>(got[j][0], got[j][WPV - 1])
-                                                         : T(0);
-            if (lane == 0) s_abort = ab;
         }
         __syncthreads();
-        if (s_abort) return;  // the whole workgroup leaves together
-        if (lane < rows) {
+        if (s_abort[sb]) return;  // the whole workgroup leaves together
+        if constexpr (MF) {
+            T xb[TV_PART];
 #pragma unroll
-            for (int kk = 0; kk < TV_PART; kk++) {
-                const T av = (T)a[kk];
-                const int k = wave * TV_PART + kk;
+            for (int kk = 0; kk < TV_PART; kk++) xb[kk] = Xs[sb][pk + kk][lr];
 #pragma unroll
-                for (int j = 0; j < NR; j++) part[j] = fma(av, Xs[k][j], part[j]);
-            }
+            for (int kk = 0; kk < TV_PART; kk++)
+                acc[kk & 3] = mfma16x4<T>((T)a[kk], xb[kk], acc[kk & 3]);
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < TV_PART; kk++) part = fma((T)a[kk], Xs[sb][pk + kk][0], part);
         }
         if (s + 1 < t) load_block(s + 1);
-        __syncthreads();  // Xs is reused by the next block
     }
+    if constexpr (MF) {
 #pragma unroll
-    for (int j = 0; j < NR; j++) Part[wave][lane][j] = part[j];
-    __syncthreads();
+        for (int r = 0; r < 4; r++)
+            Ys[lr][16 * wave + mfma_row<T>(lk, r)] =
+                rhs[r] - ((acc[0][r] + acc[1][r]) + (acc[2][r] + acc[3][r]));
+        __syncthreads();
+    } else {
+        Part[wave][lane] = part;
+        __syncthreads();
+        if (wave == 0)
+            Ys[0][lane] = rhs[0] - (((Part[0][lane] + Part[1][lane]) + Part[2][lane]) + Part[3][lane]);
+        __syncthreads();
+    }
 
-    if (wave == 0) {
-        T x[NR];
+    // The diagonal block: column j of the right-hand sides in a row of 16 lanes,
+    // lane l rows 16 i + l; four 16 x 16 triangles, each solved value going on to
+    // the rows below (above) its triangle at once.
+    const int j = 4 * wave + lk;
+    if (4 * wave < nrhs) {
+        const T *y = Ys[MF ? j : 0];
+        T bb[4];  // bb[0]: the rows of the current triangle, then those after it
 #pragma unroll
-        for (int j = 0; j < NR; j++) {
-            const T sum = ((Part[0][lane][j] + Part[1][lane][j]) + Part[2][lane][j]) + Part[3][lane][j];
-            x[j] = rhs[j] - sum;
-        }
-        // Column i of the triangle applied to x: element (lane, i) of the
-        // diagonal block, or (i, lane) for the transposed solves.
-        if (FORWARD) {
-            for (int i = 0; i < rows; i++) {
-                const T l = TRANS ? Ds[i][lane] : Ds[lane][i];
+        for (int i = 0; i < 4; i++) bb[i] = y[16 * (FORWARD ? i : 3 - i) + lr];
+        const uint64_t tag = (uint64_t)epoch << 32;
+#pragma unroll 1
+        for (int i = 0; i < 4; i++) {
+            const int r0 = 16 * (FORWARD ? i : 3 - i);
+            const T *e[4];  // rows r0, and those of bb[1] .. bb[3] (a row of the block if none)
 #pragma unroll
-                for (int j = 0; j < NR; j++) {
-                    if (!UNIT && lane == i) x[j] = x[j] * rdiag;
-                    const T xi = lane_read(x[j], i);
-                    if (lane > i) x[j] = fma(-l, xi, x[j]);
-                }
+            for (int q = 0; q < 4; q++)
+                e[q] = &Es[r0][(FORWARD ? min(r0 + 16 * q, TV_BS - 16) : max(r0 - 16 * q, 0)) + lr];
+            T x = T(0);
+            tv_steps<0, FORWARD, UNIT>(bb, x, e, rd + r0, lr);
+            if (j < nrhs && r0 + lr < rows) {
+#pragma unroll
+                for (int w = 0; w < WPV; w++)
+                    __hip_atomic_store(mbox(b, j, w, r0 + lr), tag | tv_half(x, w),
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                X[(size_t)(rb + r0 + lr) + (size_t)j * ldx] = x;
             }
-        } else {
-            for (int i = rows - 1; i >= 0; i--) {
-                const T u = TRANS ? Ds[i][lane] : Ds[lane][i];
-#pragma unroll
-                for (int j = 0; j < NR; j++) {
-                    if (!UNIT && lane == i) x[j] = x[j] * rdiag;
-                    const T xi = lane_read(x[j], i);
-                    if (lane < i) x[j] = fma(-u, xi, x[j]);
-                }
-            }
-        }
-        if (lane < rows) {
-            const uint64_t tag = (uint64_t)epoch << 32;
-#pragma unroll
-            for (int j = 0; j < NR; j++) {
-                if (j < nrhs) {
-#pragma unroll
-                    for (int w = 0; w < WPV; w++)
-                        __hip_atomic_store(mbox(b, j, w, lane), tag | tv_half(x[j], w),
-                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    X[(size_t)(rb + lane) + (size_t)j * ldx] = x[j];
-                }
-            }
+            bb[0] = bb[1];
+            bb[1] = bb[2];
+            bb[2] = bb[3];
         }
     }
 }
@@ -631,8 +703,6 @@ template void trsm_llnu<float>(int, int, const float *, int, float *, int, hipSt
 namespace {
 
 constexpr int TB_M = 512, TB_NC = 16, TB_LD = TB_NC + 1;
-typedef double bd4_t __attribute__((ext_vector_type(4)));
-typedef float bf4_t __attribute__((ext_vector_type(4)));
 
 template <typename T>
 __global__ __launch_bounds__(1024) void trsm_diag_inv_kernel(int m, const T *__restrict__ L,
@@ -654,21 +724,6 @@ __global__ __launch_bounds__(1024) void trsm_diag_inv_kernel(int m, const T *__r
         }
     }
     inv[(size_t)b * 1024 + (size_t)j * 32 + i] = x;
-}
-
-template <typename T>
-__device__ __forceinline__ auto mfma16x4(T a, T b, typename std::conditional<sizeof(T) == 8, bd4_t,
-                                                                            bf4_t>::type c)
-{
-    if constexpr (sizeof(T) == 8) return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    else return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-// row of accumulator element r of lane (lr, lk) within a 16 x 16 tile
-template <typename T>
-__device__ __forceinline__ int mfma_row(int lk, int r)
-{
-    return sizeof(T) == 8 ? lk + 4 * r : 4 * lk + r;
 }
 
 // MM: rows at most.  The panel's solves (MM <= 256) run beside the trailing
@@ -942,9 +997,7 @@ void trsv_persistent(TrsvOp op, int n, int nrhs, const TA *A, int lda, T *X, int
 #define SLA_TRSV_NR(FW, TR)                           \
     do {                                              \
         if (nrhs <= 1) SLA_TRSV(FW, TR, 1);           \
-        else if (nrhs <= 2) SLA_TRSV(FW, TR, 2);      \
         else if (nrhs <= 4) SLA_TRSV(FW, TR, 4);      \
-        else if (nrhs <= 8) SLA_TRSV(FW, TR, 8);      \
         else SLA_TRSV(FW, TR, 16);                    \
     } while (0)
     switch (op) {
