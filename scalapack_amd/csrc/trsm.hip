@@ -905,13 +905,12 @@ __global__ __launch_bounds__(TT_T) void trsm_tri_kernel(int m, int n, const T *_
             T an[8];
             load_tile(an, kr, t + NW, ntile);
             const int r0 = kr + 32 + 16 * t;
-            acc_t c;
+            // summed apart from X, which then takes one rounding a block and not eight
+            acc_t c[2] = {};
 #pragma unroll
-            for (int r = 0; r < 4; r++) c[r] = Xs[r0 + mfma_row<T>(lk, r)][lr];
+            for (int s = 0; s < 8; s++) c[s & 1] = mfma16x4<T>(a[s], xb[s], c[s & 1]);
 #pragma unroll
-            for (int s = 0; s < 8; s++) c = mfma16x4<T>(a[s], xb[s], c);
-#pragma unroll
-            for (int r = 0; r < 4; r++) Xs[r0 + mfma_row<T>(lk, r)][lr] = c[r];
+            for (int r = 0; r < 4; r++) Xs[r0 + mfma_row<T>(lk, r)][lr] += c[0][r] + c[1][r];
 #pragma unroll
             for (int s = 0; s < 8; s++) a[s] = an[s];
         }
