@@ -9,24 +9,34 @@
 // and two triangular solves (pdgetrs.f:255-266), skipped when INFO > 0
 // (pdgesv.f:231).
 //
-// Work distribution: workgroups (256 threads) take systems from a device
-// queue, largest first (the host sorts the sizes once), until the queue is
-// empty; every workgroup leaves when the ticket passes the batch size.
-// Inside a system the factorization is blocked right-looking with W-column
-// panels:
-//   panel    columns kb .. kb+W-1: while the panel has at most 256 RPT rows
-//            (RPT = 2 for FP64, 4 for FP32) it is held in registers and a
-//            column costs one workgroup barrier (panel_regs); taller panels
-//            run unblocked in memory (pivot search as a wave-shuffle argmax
-//            folded across the four waves in LDS, row interchange over all n
-//            columns, reciprocal scaling, rank-1 update, two barriers per
-//            column);
-//   U12      L11^{-1} A12, one thread per column of A12;
-//   update   A22 -= L21 U12 in 64 x 64 tiles, L21 / U12 staged through LDS,
-//            the products on the 16 x 16 x 4 MFMA of the storage precision.
-// The solves take 64-row blocks: one wave solves the diagonal block in
-// registers (lane = row, values broadcast by lane reads), then all four
-// waves update the rows below (above) with the 64 new values.
+// Work distribution: workgroups take systems from a device queue, largest first
+// (the host sorts the sizes once), until the queue is empty; every workgroup
+// leaves when the ticket passes the batch size.
+//
+// Factorization, 512 threads, blocked right-looking with W-column panels:
+//   panel    held in registers, a thread a row (two rows and 8 columns where more
+//            than 512 rows are left); a column costs one workgroup barrier
+//            (panel_regs);
+//   strips   of 16 columns right of the panel, a wave each with no barrier in
+//            between: the interchanges, U12 = L11^{-1} A12 in registers, then
+//            A22 -= L21 U12 on the 16 x 16 x 4 MFMA of the storage precision,
+//            the strip of A22 passing through registers once; strips left of the
+//            panel get their interchanges only, and only if there are any.
+// Bound: small systems by the chain of columns (about 1 us each, search, post,
+// barrier, fold, update), large ones by the passes over A22, n / W of them, since
+// the systems in flight (512 of n = 512 are 1 GB) do not stay in cache.  512
+// threads and at most 128 registers keep 16 waves on a CU with two workgroups,
+// where 256 threads with 196 registers kept eight.  Before, the interchanges of a
+// column were one after another in memory, U12 and A22 went through LDS with a
+// barrier around every 64 x 64 tile, and the search took eighteen lane exchanges.
+// Factorization and solve of 512 systems, us, before -> this: FP64 n = 64 273 ->
+// 165, 128 601 -> 350, 256 1918 -> 1329, 512 11095 -> 9332; FP32 257 -> 147, 559 ->
+// 299, 1666 -> 870, 8764 -> 5849.  2000 FP64 systems of 32 .. 512: factorization
+// 12.5 -> 6.0 ms.
+//
+// The solves take 16-row blocks: one wave solves the diagonal block in
+// registers (lane = row, values broadcast by lane reads), then all waves
+// update the rows below (above) with the new values.
 #include "sla_common.h"
 #include "sla_handle.h"
 #include "sla_batched.h"
@@ -46,429 +56,331 @@ namespace sla {
 
 namespace {
 
-constexpr int BT = 256;       // threads per workgroup
-constexpr int UT = 64;        // update tile edge
-
-// Kernel variants for comparisons: SLA_BATCHED_FLAGS (environment) sets the
-// flags of factor_system (default 3: register panels and MFMA updates).
-int batched_flags()
-{
-    static const int f = [] {
-        const char *e = getenv("SLA_BATCHED_FLAGS");
-        return e ? (atoi(e) & 3) : 3;
-    }();
-    return f;
-}
+constexpr int FT = 512, FW = FT / 64;  // threads and waves of a factorization's workgroup
+constexpr int BT = 256;                // threads of a solve's
+constexpr int SC = 16;                 // columns of a strip
 
 struct SysDesc {
     int n, nrhs, lda, ldb;
 };
 
-template <typename T>
-__device__ __forceinline__ void argmax_fold(T &v, int &i, T v2, int i2)
-{
-    if (v2 > v || (v2 == v && i2 < i)) {
-        v = v2;
-        i = i2;
-    }
-}
-// The same carrying the signed value at the winning row.
-template <typename T>
-__device__ __forceinline__ void argmax_fold3(T &v, int &i, T &sv, T v2, int i2, T sv2)
-{
-    if (v2 > v || (v2 == v && i2 < i)) {
-        v = v2;
-        i = i2;
-        sv = sv2;
-    }
-}
-
-// LDS of the register-resident panel: per column parity, the candidate row
-// of every wave (slots 0..3) and the row at the diagonal position (slot 4),
-// the wave maxima and their positions; the panel's pivots.
-template <typename T, int W>
-struct RegPanelLds {
-    T rows[2][5][W];
-    T val[2][4];
-    int pos[2][4];
-    int piv[W];
-};
-
-// Panel columns kb .. kb+w-1 of rows kb .. n-1 held in registers while they
-// are factored: thread t holds positions kb + t + 256 q (q < RPT), so this
-// path serves panels of at most 256 RPT rows.  Per column j: every thread
-// finds its largest |a| among the positions >= j (lowest position on ties),
-// a wave argmax, the owner of each wave's winner posts its whole panel row
-// and the owner of position j its row, ONE workgroup barrier, then every
-// thread folds the four posts in the same order: the owner of the pivot's
-// position takes the row from position j and the owner of position j the
-// pivot row (the interchange within the panel), the rows below j are scaled
-// by the reciprocal of the pivot and updated with the pivot row.  The
-// posts are double-buffered by column parity, so no second barrier is
-// needed.  The operations on every element are those of the unblocked
-// panel below (same interchange, reciprocal scaling, FMA), so both give the
-// same bits.  The interchanges reach the other columns after the panel,
-// replayed in order column by column.
-template <typename T, int W, int RPT>
-__device__ void panel_regs(int n, int kb, int w, T *__restrict__ a, int lda, int *__restrict__ piv,
-                           int &info, RegPanelLds<T, W> &sl)
-{
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    T v[RPT][W];
-#pragma unroll
-    for (int q = 0; q < RPT; q++) {
-        const int r = kb + tid + BT * q;
-#pragma unroll
-        for (int c = 0; c < W; c++)
-            v[q][c] = (r < n && c < w) ? a[(size_t)r + (size_t)(kb + c) * lda] : T(0);
-    }
-#pragma unroll
-    for (int jj = 0; jj < W; jj++) {
-        if (jj < w) {  // uniform
-        const int j = kb + jj, pb = jj & 1;
-        // the largest |a| of column j among this thread's positions >= j
-        T best = T(-1);
-        int bi = INT_MAX;
-#pragma unroll
-        for (int q = 0; q < RPT; q++) {
-            const int r = kb + tid + BT * q;
-            const T x = fabs(v[q][jj]);
-            if (r >= j && r < n && x > best) {  // a NaN never wins
-                best = x;
-                bi = r;
-            }
-        }
-        for (int o = 32; o > 0; o >>= 1) argmax_fold(best, bi, __shfl_xor(best, o), __shfl_xor(bi, o));
-        if (bi != INT_MAX && (bi - kb) % BT == tid) {  // this thread holds the wave's winner
-            const int qw = (bi - kb) / BT;
-#pragma unroll
-            for (int q = 0; q < RPT; q++)
-                if (q == qw)
-#pragma unroll
-                    for (int c = 0; c < W; c++) sl.rows[pb][wave][c] = v[q][c];
-        }
-        if (tid == jj)  // position j is (thread jj, q = 0)
-#pragma unroll
-            for (int c = 0; c < W; c++) sl.rows[pb][4][c] = v[0][c];
-        if (lane == 0) {
-            sl.val[pb][wave] = best;
-            sl.pos[pb][wave] = bi;
-        }
-        __syncthreads();
-        T fv = sl.val[pb][0];
-        int fi = sl.pos[pb][0], fw = 0;
-#pragma unroll
-        for (int q = 1; q < 4; q++) {
-            const T v2 = sl.val[pb][q];
-            const int i2 = sl.pos[pb][q];
-            if (v2 > fv || (v2 == fv && i2 < fi)) {
-                fv = v2;
-                fi = i2;
-                fw = q;
-            }
-        }
-        // no comparable entry (all NaN): keep row j
-        const int p = fi < n ? fi : j;
-        const T *prow = fi < n ? sl.rows[pb][fw] : sl.rows[pb][4];
-        const T pv = prow[jj];
-        if (tid == 0) {
-            piv[j] = p + 1;
-            sl.piv[jj] = p;
-        }
-        if (pv != T(0)) {
-            if (p != j) {
-                if ((p - kb) % BT == tid) {
-                    const int qp = (p - kb) / BT;
-#pragma unroll
-                    for (int q = 0; q < RPT; q++)
-                        if (q == qp)
-#pragma unroll
-                            for (int c = 0; c < W; c++) v[q][c] = sl.rows[pb][4][c];
-                }
-                if (tid == jj)
-#pragma unroll
-                    for (int c = 0; c < W; c++) v[0][c] = prow[c];
-            }
-            const T rcp = T(1) / pv;
-#pragma unroll
-            for (int q = 0; q < RPT; q++) {
-                const int r = kb + tid + BT * q;
-                if (r > j && r < n) v[q][jj] = v[q][jj] * rcp;
-            }
-        } else if (info == 0) {
-            info = j + 1;
-        }
-        // rank-1 update of the panel's columns right of j
-#pragma unroll
-        for (int q = 0; q < RPT; q++) {
-            const int r = kb + tid + BT * q;
-            if (r > j && r < n) {
-                const T l = v[q][jj];
-                // constant bounds, so the inner loop unrolls before the outer
-#pragma unroll
-                for (int c = 1; c < W; c++)
-                    if (c > jj && c < w) v[q][c] = fma(-l, prow[c], v[q][c]);
-            }
-        }
-        }  // jj < w
-    }
-#pragma unroll
-    for (int q = 0; q < RPT; q++) {
-        const int r = kb + tid + BT * q;
-        if (r < n)
-#pragma unroll
-            for (int c = 0; c < W; c++)
-                if (c < w) a[(size_t)r + (size_t)(kb + c) * lda] = v[q][c];
-    }
-    __syncthreads();  // sl.piv complete
-    // the panel's interchanges, in order, on every other column
-    for (int c = tid; c < n; c += BT) {
-        if (c >= kb && c < kb + w) continue;
-        T *cc = a + (size_t)c * lda;
-        for (int jj = 0; jj < w; jj++) {
-            const int p = sl.piv[jj];
-            if (p != kb + jj) {
-                const T t = cc[kb + jj];
-                cc[kb + jj] = cc[p];
-                cc[p] = t;
-            }
-        }
-    }
-}
-
-// C[rows x cols] -= Ls[0:rows, 0:w] Us[0:w, 0:cols] for one 64 x 64 tile on
-// the 16 x 16 x 4 MFMA of the storage precision: wave v owns rows
-// 32 (v & 1) .., columns 32 (v >> 1) .. as 2 x 2 blocks.  w is a multiple of
-// 4 (every update follows a full panel of width W in {8, 16, 32}).
-// D layouts: f64 16x16x4, element r of lane l = D[l/16 + 4 r][l % 16];
-// f32 16x16x4, element r of lane l = D[4 (l/16) + r][l % 16].
 typedef double bd4_t __attribute__((ext_vector_type(4)));
 typedef float bf4_t __attribute__((ext_vector_type(4)));
 
+// A barrier that waits for the workgroup's LDS traffic only: panel_regs stores to
+// global memory between barriers and nobody reads that before the panel's end.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_max(uint32_t x)
+{
+    // lanes the move does not reach combine with 0
+    const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
+    return x > y ? x : y;
+}
+
+// Wave-wide maximum, uniform.
+__device__ __forceinline__ uint32_t wave_max(uint32_t x)
+{
+    x = dpp_max<0x121, 0xf>(x);
+    x = dpp_max<0x122, 0xf>(x);
+    x = dpp_max<0x124, 0xf>(x);
+    x = dpp_max<0x128, 0xf>(x);
+    x = dpp_max<0x142, 0xa>(x);
+    x = dpp_max<0x143, 0xc>(x);
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+
+// The value of lane S of the quad, in all four lanes.
+template <int S, typename T>
+__device__ __forceinline__ T quad_lane(T v)
+{
+    if constexpr (sizeof(T) == 8) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, S * 0x55, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), S * 0x55, 0xf, 0xf, false);
+        return __builtin_bit_cast(T, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+    } else {
+        return __builtin_bit_cast(
+            T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), S * 0x55, 0xf, 0xf, false));
+    }
+}
+
+// A pivot candidate's rank, (hi, lo) compared as one number: 0 for no candidate,
+// then a NaN in row j (kept only if nothing is comparable), then |v|.
+__device__ __forceinline__ void rank_of(double v, bool act, bool top, uint32_t &hi, uint32_t &lo)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t h = (uint32_t)(u >> 32) & 0x7fffffffu;
+    const bool nan = v != v;
+    hi = act ? (nan ? (top ? 1u : 0u) : h + 2u) : 0u;
+    lo = nan ? 0u : (uint32_t)u;
+}
+__device__ __forceinline__ void rank_of(float v, bool act, bool top, uint32_t &hi, uint32_t &lo)
+{
+    hi = act ? (v != v ? (top ? 1u : 0u) : (__builtin_bit_cast(uint32_t, v) & 0x7fffffffu) + 2u) : 0u;
+    lo = 0u;
+}
+
+// LDS of a factorization.  Per column parity: every wave's candidate row with the
+// reciprocal of its pivot, its rank and position.
 template <typename T, int W>
-__device__ __forceinline__ void tile_update_mfma(int w, int rows, int cols, const T (*Ls)[W + 1],
-                                                 const T (*Us)[UT + 1], T *__restrict__ C, int ldc)
+struct FactorLds {
+    alignas(16) T rows[2][FW][W];
+    T rcp[2][FW];
+    uint32_t hi[2][FW], lo[2][FW];
+    int pos[2][FW];
+    T L11[W][W + 1];           // column k of the unit lower triangle in row k
+    T U[FW][W][SC + 1];        // a wave's strip of U12
+    int src[BATCHED_NMAX];     // the row that the panel moved to each position
+    int dst[W], ndst, moved;   // positions below the panel's rows that received one
+};
+
+// Panel columns kb .. kb + w - 1 of rows kb .. n - 1 held in registers while they
+// are factored: thread t holds rows kb + t + 512 q (q < RPT).  Rows stay with
+// their thread and carry their position.  Per column j: the wave's first largest
+// |a| among the positions >= j (its leading 32 bits decide unless they are
+// shared), the owner posts its row and its reciprocal, ONE barrier, every wave
+// folds the posts in the same order, the rows below are scaled by the reciprocal
+// and updated with the pivot row.  The posts alternate by column parity, so no
+// second barrier is needed.  The interchanges reach the other columns in the
+// strips that follow, from src and dst.
+template <typename T, int W, int RPT, int WL>
+__device__ __forceinline__ void panel_regs(int n, int kb, int w, T *a, int lda, int *__restrict__ piv,
+                                           int &info, FactorLds<T, WL> &sl)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int nw = min(FW, (n - kb + 63) / 64);  // waves that hold rows
+    T v[RPT][W];
+    int pos[RPT];
+#pragma unroll
+    for (int q = 0; q < RPT; q++) {
+        const int r = kb + tid + FT * q;
+        pos[q] = r < n ? r : -1;
+#pragma unroll
+        for (int c = 0; c < W; c++)
+            v[q][c] = (r < n && c < w) ? (a + (size_t)(kb + c) * lda)[(unsigned)r] : T(0);
+    }
+    if (tid == 0) sl.ndst = sl.moved = 0;
+#pragma unroll
+    for (int jj = 0; jj < W; jj++) {
+        if (jj < w) {  // uniform
+            const int j = kb + jj, pb = jj & 1;
+            if (wave < nw) {
+                uint32_t bh, bl;
+                int bq = 0, bp = pos[0];
+                rank_of(v[0][jj], pos[0] >= j, pos[0] == j, bh, bl);
+#pragma unroll
+                for (int q = 1; q < RPT; q++) {
+                    uint32_t h, l;
+                    rank_of(v[q][jj], pos[q] >= j, pos[q] == j, h, l);
+                    if (h > bh || (h == bh && (l > bl || (l == bl && pos[q] < bp)))) {
+                        bh = h, bl = l, bp = pos[q], bq = q;
+                    }
+                }
+                const uint32_t hm = wave_max(bh);
+                uint64_t in = __ballot(bh == hm);
+                if ((in & (in - 1)) && hm) {
+                    const uint32_t lm = wave_max(bh == hm ? bl : 0u);
+                    const bool eq = bh == hm && bl == lm;
+                    const uint32_t nm = wave_max(eq ? ~(uint32_t)bp : 0u);
+                    in = __ballot(eq && ~(uint32_t)bp == nm);
+                }
+                if (lane == __builtin_ctzll(in)) {
+#pragma unroll
+                    for (int c = jj; c < W; c++) {
+                        T x = v[0][c];
+#pragma unroll
+                        for (int q = 1; q < RPT; q++) x = bq == q ? v[q][c] : x;
+                        sl.rows[pb][wave][c] = x;
+                        if (c == jj) sl.rcp[pb][wave] = T(1) / x;
+                    }
+                    sl.hi[pb][wave] = bh;
+                    sl.lo[pb][wave] = bl;
+                    sl.pos[pb][wave] = bp;
+                }
+            }
+            lds_barrier();
+            const int i = lane & (FW - 1);
+            const uint32_t h = i < nw ? sl.hi[pb][i] : 0u;
+            const int wp = i < nw ? sl.pos[pb][i] : 0;
+            uint32_t hm = dpp_max<0x121, 0xf>(h);
+            hm = dpp_max<0x122, 0xf>(hm);
+            hm = dpp_max<0x124, 0xf>(hm);
+            uint32_t in = (uint32_t)__ballot(h == hm) & ((1u << FW) - 1u);
+            if (in & (in - 1)) {
+                const uint32_t l = sl.lo[pb][i];
+                const uint32_t lm = wave_max(h == hm ? l : 0u);
+                const bool eq = h == hm && l == lm;
+                const uint32_t nm = wave_max(eq ? ~(uint32_t)wp : 0u);
+                in = (uint32_t)__ballot(eq && ~(uint32_t)wp == nm) & ((1u << FW) - 1u);
+            }
+            const int fw = __builtin_ctz(in);
+            const int p = __builtin_amdgcn_readlane(wp, fw);
+            const T *prow = sl.rows[pb][fw];
+            const T pv = prow[jj], rcp = sl.rcp[pb][fw];
+            const bool nz = pv != T(0);
+            if (tid == 0) piv[j] = p + 1;
+            if (!nz && info == 0) info = j + 1;
+#pragma unroll
+            for (int q = 0; q < RPT; q++) {
+                if (nz) pos[q] = pos[q] == p ? j : pos[q] == j ? p : pos[q];
+                if (pos[q] > j) {
+                    const T l = nz ? v[q][jj] * rcp : v[q][jj];
+                    v[q][jj] = l;
+#pragma unroll
+                    for (int c = jj + 1; c < W; c++) v[q][c] = fma(-l, prow[c], v[q][c]);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < RPT; q++) {
+        const int r = kb + tid + FT * q;
+        if (r < n) {
+#pragma unroll
+            for (int c = 0; c < W; c++)
+                if (c < w) (a + (size_t)(kb + c) * lda)[(unsigned)pos[q]] = v[q][c];
+            if (pos[q] < kb + w)
+#pragma unroll
+                for (int c = 0; c < W; c++) sl.L11[c][pos[q] - kb] = v[q][c];
+            sl.src[pos[q]] = r;
+            if (pos[q] != r) {
+                sl.moved = 1;
+                if (pos[q] >= kb + w) sl.dst[atomicAdd(&sl.ndst, 1)] = pos[q];
+            }
+        }
+    }
+    __syncthreads();
+}
+
+// b <- L^{-1} b for a column in a quad of lanes, lane q rows 4 i + q.
+template <int K, int W, typename T, int WL>
+__device__ __forceinline__ void unit_steps(T (&b)[W / 4], const T (*Es)[WL], int q)
+{
+    if constexpr (K < W) {
+        const T x = quad_lane<K % 4>(b[K / 4]);
+        const T own = fma(-Es[K][K / 4 * 4 + q], x, b[K / 4]);
+        b[K / 4] = q > K % 4 ? own : b[K / 4];
+#pragma unroll
+        for (int i = K / 4 + 1; i < W / 4; i++) b[i] = fma(-Es[K][4 * i + q], x, b[i]);
+        unit_steps<K + 1, W>(b, Es, q);
+    }
+}
+
+// One wave takes the 16 columns c0 .. c0 + 15 through the panel kb .. kb + w - 1:
+// its interchanges (loads of the panel's rows and of what they displace, then the
+// stores), and with UPDATE, w = W, U12 = L11^{-1} A12 by substitution, a quad of
+// lanes a column, and A22 -= L21 U12 in 16-row tiles on MFMA.  The product is formed
+// transposed, so a load or store of A22 covers 16 consecutive rows of four columns
+// rather than four of sixteen.  Loads run one tile ahead.
+// D layouts: f64 16x16x4, element r of lane l = D[l/16 + 4 r][l % 16];
+// f32 16x16x4, element r of lane l = D[4 (l/16) + r][l % 16].
+template <bool UPDATE, typename T, int W, int WL>
+__device__ __forceinline__ void strip(int n, int kb, int w, int c0, int cend, T *a, int lda,
+                                      FactorLds<T, WL> &sl)
 {
     using acc_t = typename std::conditional<sizeof(T) == 8, bd4_t, bf4_t>::type;
+    constexpr int NI = W / 4;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wr = (wave & 1) * 32, wc = (wave >> 1) * 32, lr = lane & 15, lk = lane >> 4;
-    acc_t acc[2][2];
+    const int lr = lane & 15, lk = lane >> 4;
+    T b[NI];
+    const int q = lane & 3, c = lane >> 2;
+    {
+        const bool on = c0 + c < cend;
+        T *x = a + (size_t)(on ? c0 + c : c0) * lda;
+        T d[NI];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+        for (int i = 0; i < NI; i++)
+            b[i] = on && 4 * i + q < w ? x[sl.src[kb + 4 * i + q]] : T(0);
 #pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = acc_t{0, 0, 0, 0};
-    for (int k0 = 0; k0 < w; k0 += 4) {
-        T af[2], bf[2];
+        for (int i = 0; i < NI; i++)
+            if (4 * i + q < sl.ndst) d[i] = x[sl.src[sl.dst[4 * i + q]]];
 #pragma unroll
-        for (int i = 0; i < 2; i++) af[i] = Ls[wr + 16 * i + lr][k0 + lk];
+        for (int i = 0; i < NI; i++)
+            if (on && 4 * i + q < sl.ndst) x[sl.dst[4 * i + q]] = d[i];
+        if constexpr (UPDATE) unit_steps<0, W>(b, sl.L11, q);
 #pragma unroll
-        for (int j = 0; j < 2; j++) bf[j] = Us[k0 + lk][wc + 16 * j + lr];
+        for (int i = 0; i < NI; i++)
+            if (on && 4 * i + q < w) x[kb + 4 * i + q] = b[i];
+    }
+    if constexpr (UPDATE) {
+        T(*Us)[SC + 1] = sl.U[wave];
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+        for (int i = 0; i < NI; i++) Us[4 * i + q][c] = b[i];
+        __builtin_amdgcn_wave_barrier();
+        T u[NI];
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
+        for (int s = 0; s < NI; s++) u[s] = Us[4 * s + lk][lr];
+        __builtin_amdgcn_wave_barrier();
+        const int r0 = kb + W, ntile = (n - r0 + 15) / 16;
+        const T *L = a + (size_t)(r0 + lr) + (size_t)(kb + lk) * lda;
+        const int cc = c0 + (sizeof(T) == 8 ? lk : 4 * lk);
+        constexpr int CS = sizeof(T) == 8 ? 4 : 1;  // columns between a lane's elements
+        T *C = a + (size_t)(r0 + lr) + (size_t)cc * lda;
+        T l[NI], v[4];
+        auto load = [&](T(&l)[NI], T(&v)[4], int t) {
+            const bool ok = r0 + lr + 16 * t < n;
+#pragma unroll
+            for (int s = 0; s < NI; s++) l[s] = ok ? L[16 * t + (size_t)(4 * s) * lda] : T(0);
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                v[r] = ok && cc + CS * r < cend ? C[16 * t + (size_t)(CS * r) * lda] : T(0);
+        };
+        load(l, v, 0);
+        for (int t = 0; t < ntile; t++) {
+            T ln[NI], vn[4];
+            load(ln, vn, t + 1);  // nothing past the last tile: its rows are >= n
+            acc_t acc = acc_t{0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < NI; s++) {
                 if constexpr (sizeof(T) == 8)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i], bf[j], acc[i][j], 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(u[s], l[s], acc, 0, 0, 0);
                 else
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i], bf[j], acc[i][j], 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(u[s], l[s], acc, 0, 0, 0);
             }
-    }
+            const bool ok = r0 + lr + 16 * t < n;
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int c = wc + 16 * j + lr;
-        if (c >= cols) continue;
-        T *cc = C + (size_t)c * ldc;
+            for (int r = 0; r < 4; r++)
+                if (ok && cc + CS * r < cend) C[16 * t + (size_t)(CS * r) * lda] = v[r] - acc[r];
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+            for (int s = 0; s < NI; s++) l[s] = ln[s];
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int row = wr + 16 * i + (sizeof(T) == 8 ? lk + 4 * r : 4 * lk + r);
-                if (row < rows) cc[row] -= acc[i][j][r];
-            }
-    }
-}
-
-// The same with 4 x 4 outputs per thread on vector FMAs (thread t: rows
-// 4 (t % 16) .., columns 4 (t / 16) ..).
-template <typename T, int W>
-__device__ __forceinline__ void tile_update_valu(int w, int rows, int cols, const T (*Ls)[W + 1],
-                                                 const T (*Us)[UT + 1], T *__restrict__ C, int ldc)
-{
-    const int tr = threadIdx.x & 15, tc = threadIdx.x >> 4;
-    T acc[4][4];
-#pragma unroll
-    for (int x = 0; x < 4; x++)
-#pragma unroll
-        for (int y = 0; y < 4; y++) acc[x][y] = T(0);
-    for (int k = 0; k < w; k++) {
-        T l[4], u[4];
-#pragma unroll
-        for (int x = 0; x < 4; x++) l[x] = Ls[4 * tr + x][k];
-#pragma unroll
-        for (int y = 0; y < 4; y++) u[y] = Us[k][4 * tc + y];
-#pragma unroll
-        for (int x = 0; x < 4; x++)
-#pragma unroll
-            for (int y = 0; y < 4; y++) acc[x][y] = fma(l[x], u[y], acc[x][y]);
-    }
-#pragma unroll
-    for (int y = 0; y < 4; y++) {
-        const int c = 4 * tc + y;
-        if (c < cols) {
-            T *cc = C + (size_t)c * ldc;
-#pragma unroll
-            for (int x = 0; x < 4; x++)
-                if (4 * tr + x < rows) cc[4 * tr + x] -= acc[x][y];
+            for (int r = 0; r < 4; r++) v[r] = vn[r];
         }
     }
 }
 
-// flags: bit 0 -- panels of at most 256 RPT rows in registers (panel_regs);
-// bit 1 -- the trailing-update tiles on MFMA (else vector FMAs).
-template <typename T, int W>
-__device__ void factor_system(int n, T *__restrict__ a, int lda, int *__restrict__ piv, int &info,
-                              T (*Ls)[W + 1], T (*Us)[UT + 1], T (*L11s)[W + 1], T *s_v, int *s_i,
-                              RegPanelLds<T, W> &rp, int flags)
+// The panel of W columns at kb and its strips.
+template <int W, int RPT, typename T, int WL>
+__device__ __forceinline__ void factor_step(int n, int kb, T *a, int lda, int *__restrict__ piv,
+                                            int &info, FactorLds<T, WL> &sl)
 {
-    constexpr int RPT = sizeof(T) == 8 ? 2 : 4;  // rows per thread of the register panel
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int kb = 0; kb < n; kb += W) {
-        const int w = min(W, n - kb);
-        if ((flags & 1) && n - kb <= BT * RPT) {
-            panel_regs<T, W, RPT>(n, kb, w, a, lda, piv, info, rp);
-        } else {
-        // ---- panel (unblocked), columns kb .. kb+w-1.  Thread t owns rows
-        // j+1+t, j+1+t+256, ... of every step, so the rank-1 update of
-        // column j and the pivot search of column j+1 run in one pass over
-        // those rows with no barrier between them.  The search carries the
-        // signed value of the winning row, and the owner of row j (thread 0)
-        // publishes A(j, j) before the barrier, so after it no thread reads
-        // the two elements that the interchange then rewrites; the
-        // interchange of the other columns and the scaling of column j touch
-        // disjoint data: two workgroup barriers per column.
-        T best = T(-1), bsv = T(0);
-        int bi = INT_MAX;
-        {
-            const T *col = a + (size_t)kb * lda;
-            for (int i = kb + tid; i < n; i += BT) {
-                const T x = col[i], v = fabs(x);
-                if (v > best) {
-                    best = v;
-                    bi = i;
-                    bsv = x;
-                }
-            }
-            if (tid == 0) s_v[4] = col[kb];
-        }
-        for (int j = kb; j < kb + w; j++) {
-            T *cj = a + (size_t)j * lda;
-            for (int o = 32; o > 0; o >>= 1)
-                argmax_fold3(best, bi, bsv, __shfl_xor(best, o), __shfl_xor(bi, o), __shfl_xor(bsv, o));
-            if (lane == 0) {
-                s_v[wave] = best;
-                s_i[wave] = bi;
-                s_v[5 + wave] = bsv;
-            }
-            __syncthreads();
-            best = s_v[0];
-            bi = s_i[0];
-            bsv = s_v[5];
-            for (int q = 1; q < 4; q++) argmax_fold3(best, bi, bsv, s_v[q], s_i[q], s_v[5 + q]);
-            const T ajj = s_v[4];
-            const int p = bi < n ? bi : j;  // no comparable entry (all NaN): keep row j
-            const T pv = bi < n ? bsv : ajj;
-            if (tid == 0) piv[j] = p + 1;
-            if (pv != T(0)) {
-                if (p != j)
-                    for (int c = tid; c < n; c += BT) {
-                        if (c == j) continue;
-                        T *cc = a + (size_t)c * lda;
-                        const T t = cc[j];
-                        cc[j] = cc[p];
-                        cc[p] = t;
-                    }
-                const T r = T(1) / pv;
-                // column j: rows j+1.. scaled (row p receives the old A(j, j))
-                for (int i = j + 1 + tid; i < n; i += BT) cj[i] = (i == p ? ajj : cj[i]) * r;
-                if (tid == 0) cj[j] = pv;
-            } else if (info == 0) {
-                info = j + 1;
-            }
-            __syncthreads();  // row j (all columns) and column j are final
-            // rank-1 update of the panel's columns right of j, fused with the
-            // pivot search of column j + 1 over the same rows
-            best = T(-1);
-            bi = INT_MAX;
-            bsv = T(0);
-            const int cend = kb + w;
-            for (int i = j + 1 + tid; i < n; i += BT) {
-                const T l = cj[i];
-                for (int c = j + 1; c < cend; c++) {
-                    T *cc = a + (size_t)c * lda;
-                    cc[i] = fma(-l, cc[j], cc[i]);
-                }
-                if (j + 1 < cend) {
-                    const T x = a[(size_t)(j + 1) * lda + i], v = fabs(x);
-                    if (v > best) {
-                        best = v;
-                        bi = i;
-                        bsv = x;
-                    }
-                }
-            }
-            // row j+1 is owned by thread 0 in this pass: A(j+1, j+1) is final
-            if (tid == 0 && j + 1 < cend && j + 1 < n) s_v[4] = a[(size_t)(j + 1) * (lda + 1)];
-        }
-        }  // panel
-        __syncthreads();  // the panel is final before U12 reads L11
-        const int c0 = kb + w;
-        if (c0 >= n) break;
-        // ---- U12 = L11^{-1} A12 and A22 -= L21 U12, by 64-column chunks of
-        // the trailing columns: the chunk of A12 is staged in LDS once,
-        // solved there against L11 (one thread per column, the FMA sequence
-        // of a substitution) and written back as U12, then every 64-row tile
-        // of A22 below it is updated with it (L21 tiles staged in LDS, the
-        // products on MFMA or vector FMAs)
-        const int m2 = n - c0;
-        for (int idx = tid; idx < w * w; idx += BT) {
-            const int r = idx % w, k = idx / w;
-            L11s[r][k] = a[(size_t)(kb + r) + (size_t)(kb + k) * lda];
-        }
-        for (int u0 = 0; u0 < m2; u0 += UT) {
-            const int cols = min(UT, m2 - u0);
-            for (int idx = tid; idx < UT * w; idx += BT) {
-                const int k = idx % w, c = idx / w;
-                Us[k][c] = c < cols ? a[(size_t)(kb + k) + (size_t)(c0 + u0 + c) * lda] : T(0);
-            }
-            __syncthreads();
-            if (tid < cols) {
-                for (int r = 0; r < w; r++) {
-                    const T x = Us[r][tid];
-                    for (int r2 = r + 1; r2 < w; r2++) Us[r2][tid] = fma(-L11s[r2][r], x, Us[r2][tid]);
-                }
-            }
-            __syncthreads();
-            for (int idx = tid; idx < UT * w; idx += BT) {
-                const int k = idx % w, c = idx / w;
-                if (c < cols) a[(size_t)(kb + k) + (size_t)(c0 + u0 + c) * lda] = Us[k][c];
-            }
-            for (int t0 = 0; t0 < m2; t0 += UT) {
-                const int rows = min(UT, m2 - t0);
-                for (int idx = tid; idx < UT * w; idx += BT) {
-                    const int i = idx % UT, k = idx / UT;
-                    Ls[i][k] = i < rows ? a[(size_t)(c0 + t0 + i) + (size_t)(kb + k) * lda] : T(0);
-                }
-                __syncthreads();
-                if (flags & 2)
-                    tile_update_mfma<T, W>(w, rows, cols, Ls, Us,
-                                           a + (size_t)(c0 + u0) * lda + c0 + t0, lda);
-                else
-                    tile_update_valu<T, W>(w, rows, cols, Ls, Us,
-                                           a + (size_t)(c0 + u0) * lda + c0 + t0, lda);
-                __syncthreads();  // Ls is reloaded by the next tile, Us by the next chunk
-            }
-        }
-    }
+    const int wave = threadIdx.x >> 6, w = min(W, n - kb);
+    panel_regs<T, W, RPT>(n, kb, w, a, lda, piv, info, sl);
+    for (int c0 = kb + w + SC * wave; c0 < n; c0 += SC * FW)
+        strip<true, T, W>(n, kb, w, c0, n, a, lda, sl);
+    if (sl.moved)
+        for (int c0 = SC * (FW - 1 - wave); c0 < kb; c0 += SC * FW)
+            strip<false, T, W>(n, kb, w, c0, kb, a, lda, sl);
+    __syncthreads();  // the columns are final before the next panel, sl free
+}
+
+// P A = L U in place by panels of W columns; panels of more than 512 rows keep two
+// rows a thread and are 8 columns wide, which fits the registers.
+template <typename T, int W>
+__device__ void factor_system(int n, T *a, int lda, int *__restrict__ piv, int &info,
+                              FactorLds<T, W> &sl)
+{
+    constexpr int W2 = 8;
+    int kb = 0;
+    for (; n - kb > FT; kb += W2) factor_step<W2, 2>(n, kb, a, lda, piv, info, sl);
+    for (; kb < n; kb += W) factor_step<W, 1>(n, kb, a, lda, piv, info, sl);
 }
 
 // X = U^{-1} L^{-1} P B for all nrhs columns of B at once.
@@ -573,25 +485,16 @@ __device__ void solve_all(int n, const T *__restrict__ a, int lda, const int *__
 }
 
 template <typename T, int W>
-__global__ __launch_bounds__(BT) void gesv_batched_kernel(int batch, const int *__restrict__ order,
-                                                          const SysDesc *__restrict__ desc,
-                                                          T *const *__restrict__ A,
-                                                          int *const *__restrict__ ipiv,
-                                                          T *const *__restrict__ B,
-                                                          int *__restrict__ info, int *queue,
-                                                          int flags)
+__global__ __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(4))) void gesv_batched_kernel(
+    int batch, const int *__restrict__ order, const SysDesc *__restrict__ desc,
+    T *const *__restrict__ A, int *const *__restrict__ ipiv, int *__restrict__ info, int *queue)
 {
-    __shared__ T Ls[UT][W + 1];
-    __shared__ T Us[W][UT + 1];
-    __shared__ T s_v[9];  // [0..3] wave maxima, [4] A(j, j), [5..8] signed values
-    __shared__ int s_i[4];
     __shared__ int s_q;
-    __shared__ RegPanelLds<T, W> rp;
-    __shared__ T L11s[W][W + 1];
+    __shared__ FactorLds<T, W> sl;
     for (;;) {
         if (threadIdx.x == 0) s_q = atomicAdd(queue, 1);
         __syncthreads();
-        const int q = s_q;
+        const int q = __builtin_amdgcn_readfirstlane(s_q);  // uniform: bases in scalar registers
         __syncthreads();  // s_q is rewritten by the next ticket
         if (q >= batch) break;
         const int s = order[q];
@@ -600,7 +503,7 @@ __global__ __launch_bounds__(BT) void gesv_batched_kernel(int batch, const int *
         int *piv = ipiv[s];
         // n < 0 marks a system whose sizes the allocation-free entry rejected
         int inf = d.n < 0 ? -1 : 0;
-        if (d.n > 0) factor_system<T, W>(d.n, a, d.lda, piv, inf, Ls, Us, L11s, s_v, s_i, rp, flags);
+        if (d.n > 0) factor_system<T, W>(d.n, a, d.lda, piv, inf, sl);
         if (threadIdx.x == 0) info[s] = inf;
         __syncthreads();
     }
@@ -751,8 +654,8 @@ void launch(const BatchedPlan &p, int w, int wgs, int solve_wgs, T *const *A, in
 {
     hipLaunchKernelGGL(zero_queue_kernel, dim3(1), dim3(64), 0, s, p.d_queue);
 #define SLA_BATCHED(WV)                                                                          \
-    hipLaunchKernelGGL((gesv_batched_kernel<T, WV>), dim3(wgs), dim3(BT), 0, s, p.batch,         \
-                       p.d_order, p.d_desc, A, ipiv, B, info, p.d_queue, batched_flags())
+    hipLaunchKernelGGL((gesv_batched_kernel<T, WV>), dim3(wgs), dim3(FT), 0, s, p.batch,         \
+                       p.d_order, p.d_desc, A, ipiv, info, p.d_queue)
     switch (w) {
     case 8: SLA_BATCHED(8); break;
     case 16: SLA_BATCHED(16); break;
@@ -869,8 +772,8 @@ void gesv_batched_noalloc_device(Handle &h, int batch, const int *dn, const int 
     SLA_LAUNCH_CHECK();
     const int wgs = std::max(1, h.batched_wgs_per_cu) * h.num_cus;
 #define SLA_BATCHED(WV)                                                                          \
-    hipLaunchKernelGGL((gesv_batched_kernel<T, WV>), dim3(wgs), dim3(BT), 0, h.stream, batch,     \
-                       order, desc, dA, dipiv, dB, dinfo, queue, batched_flags())
+    hipLaunchKernelGGL((gesv_batched_kernel<T, WV>), dim3(wgs), dim3(FT), 0, h.stream, batch,     \
+                       order, desc, dA, dipiv, dinfo, queue)
     switch (h.batched_w) {
     case 8: SLA_BATCHED(8); break;
     case 16: SLA_BATCHED(16); break;
