@@ -13,26 +13,30 @@
 // (the host sorts the sizes once), until the queue is empty; every workgroup
 // leaves when the ticket passes the batch size.
 //
-// Factorization, 512 threads, blocked right-looking with W-column panels:
+// Factorization, 512 threads, blocked right-looking with blocks of 64 columns, each
+// of W-column panels:
 //   panel    held in registers, a thread a row (two rows and 8 columns where more
 //            than 512 rows are left); a column costs one workgroup barrier
 //            (panel_regs);
-//   strips   of 16 columns right of the panel, a wave each with no barrier in
-//            between: the interchanges, U12 = L11^{-1} A12 in registers, then
-//            A22 -= L21 U12 on the 16 x 16 x 4 MFMA of the storage precision,
-//            the strip of A22 passing through registers once; strips left of the
-//            panel get their interchanges only, and only if there are any.
-// Bound: small systems by the chain of columns (about 1 us each, search, post,
-// barrier, fold, update), large ones by the passes over A22, n / W of them, since
-// the systems in flight (512 of n = 512 are 1 GB) do not stay in cache.  512
-// threads and at most 128 registers keep 16 waves on a CU with two workgroups,
-// where 256 threads with 196 registers kept eight.  Before, the interchanges of a
-// column were one after another in memory, U12 and A22 went through LDS with a
-// barrier around every 64 x 64 tile, and the search took eighteen lane exchanges.
-// Factorization and solve of 512 systems, us, before -> this: FP64 n = 64 273 ->
-// 165, 128 601 -> 350, 256 1918 -> 1329, 512 11095 -> 9332; FP32 257 -> 147, 559 ->
-// 299, 1666 -> 870, 8764 -> 5849.  2000 FP64 systems of 32 .. 512: factorization
-// 12.5 -> 6.0 ms.
+//   strips   of 16 columns right of a panel or a block: the interchanges, U12 =
+//            L11^{-1} A12 in registers, A22 -= L21 U12 on the 16 x 16 x 4 MFMA of the
+//            storage precision, the strip of A22 passing through registers once.
+//            After a panel they end at the block and all waves share them; after
+//            the block a wave takes a strip by itself, with no barrier in between.
+//            Columns on the left get their interchanges only, if there are any.
+// Bound: small systems by the chain of columns (under 1 us each: search, post,
+// barrier, fold, update), large ones by the passes over A22, n / 64 of them, and over
+// L21, once a strip, since the systems in flight (512 of n = 512 are 1 GB) do not
+// stay in cache.  512 threads and at most 128 registers, none of them in scratch,
+// keep 16 waves on a CU with two workgroups, where 256 threads with 196 registers
+// kept eight.  Before, A22 was passed over n / W times, the interchanges of a column
+// were one after another in memory, U12 and A22 went through LDS with a barrier
+// around every 64 x 64 tile, and the search took eighteen lane exchanges.
+// Factorization and solve of 512 systems with interchanges, us, that -> strips behind
+// every panel -> blocks: FP64 n = 64 273 -> 165 -> 166, 128 601 -> 350 -> 335, 256
+// 1918 -> 1329 -> 973, 512 11095 -> 9332 -> 5310; FP32 257 -> 147 -> 147, 559 -> 299 ->
+// 292, 1666 -> 870 -> 703, 8764 -> 5849 -> 3468.  2000 FP64 systems of 32 .. 512, the
+// factorization: 12.5 -> 6.0 -> 3.9 ms.
 //
 // The solves take 16-row blocks: one wave solves the diagonal block in
 // registers (lane = row, values broadcast by lane reads), then all waves
@@ -59,10 +63,17 @@ namespace {
 constexpr int FT = 512, FW = FT / 64;  // threads and waves of a factorization's workgroup
 constexpr int BT = 256;                // threads of a solve's
 constexpr int SC = 16;                 // columns of a strip
+constexpr int KB = 64;                 // columns of a block
 
 struct SysDesc {
     int n, nrhs, lda, ldb;
 };
+
+// A pointer that was itself loaded from memory has no known address space, and
+// its accesses would be flat: no scalar base, and counted among the LDS accesses
+// that a barrier waits for.
+template <typename T>
+using Global = __attribute__((address_space(1))) T;
 
 typedef double bd4_t __attribute__((ext_vector_type(4)));
 typedef float bf4_t __attribute__((ext_vector_type(4)));
@@ -127,6 +138,14 @@ __device__ __forceinline__ void rank_of(float v, bool act, bool top, uint32_t &h
     lo = 0u;
 }
 
+// What the interchanges of the columns at kb do: row kb + i receives row src[i],
+// and its old contents go to row dst[i].
+template <int W>
+struct Moves {
+    int src[W], dst[W];
+    int any;
+};
+
 // LDS of a factorization.  Per column parity: every wave's candidate row with the
 // reciprocal of its pivot, its rank and position.
 template <typename T, int W>
@@ -135,10 +154,12 @@ struct FactorLds {
     T rcp[2][FW];
     uint32_t hi[2][FW], lo[2][FW];
     int pos[2][FW];
-    T L11[W][W + 1];           // column k of the unit lower triangle in row k
-    T U[FW][W][SC + 1];        // a wave's strip of U12
-    int src[BATCHED_NMAX];     // the row that the panel moved to each position
-    int dst[W], ndst, moved;   // positions below the panel's rows that received one
+    T L11[W][W + 1];             // column k of the panel's unit lower triangle in row k
+    T Lb[KB][KB + 1];            // and of the block's
+    T U[FW][16][SC + 1];         // 16 rows of a wave's strip of U12
+    int from[BATCHED_NMAX];      // the row that the block's panels moved to each position
+    Moves<W> pm;                 // the panel's interchanges
+    Moves<KB> bm;                // and the block's
 };
 
 // Panel columns kb .. kb + w - 1 of rows kb .. n - 1 held in registers while they
@@ -151,22 +172,23 @@ struct FactorLds {
 // second barrier is needed.  The interchanges reach the other columns in the
 // strips that follow, from src and dst.
 template <typename T, int W, int RPT, int WL>
-__device__ __forceinline__ void panel_regs(int n, int kb, int w, T *a, int lda, int *__restrict__ piv,
+__device__ __forceinline__ void panel_regs(int n, int kb, int w, bool first, Global<T> *a, int lda, Global<int> *piv,
                                            int &info, FactorLds<T, WL> &sl)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nw = min(FW, (n - kb + 63) / 64);  // waves that hold rows
     T v[RPT][W];
-    int pos[RPT];
+    int pos[RPT], from[RPT];  // from: the row at the block's start
 #pragma unroll
     for (int q = 0; q < RPT; q++) {
         const int r = kb + tid + FT * q;
         pos[q] = r < n ? r : -1;
+        from[q] = r < n && !first ? sl.from[r] : r;
 #pragma unroll
         for (int c = 0; c < W; c++)
             v[q][c] = (r < n && c < w) ? (a + (size_t)(kb + c) * lda)[(unsigned)r] : T(0);
     }
-    if (tid == 0) sl.ndst = sl.moved = 0;
+    if (tid == 0) sl.pm.any = 0;
 #pragma unroll
     for (int jj = 0; jj < W; jj++) {
         if (jj < w) {  // uniform
@@ -249,11 +271,10 @@ __device__ __forceinline__ void panel_regs(int n, int kb, int w, T *a, int lda, 
             if (pos[q] < kb + w)
 #pragma unroll
                 for (int c = 0; c < W; c++) sl.L11[c][pos[q] - kb] = v[q][c];
-            sl.src[pos[q]] = r;
-            if (pos[q] != r) {
-                sl.moved = 1;
-                if (pos[q] >= kb + w) sl.dst[atomicAdd(&sl.ndst, 1)] = pos[q];
-            }
+            sl.from[pos[q]] = from[q];
+            if (pos[q] < kb + w) sl.pm.src[pos[q] - kb] = r;
+            if (r < kb + w) sl.pm.dst[r - kb] = pos[q];
+            if (pos[q] != r) sl.pm.any = 1;
         }
     }
     __syncthreads();
@@ -269,118 +290,198 @@ __device__ __forceinline__ void unit_steps(T (&b)[W / 4], const T (*Es)[WL], int
         b[K / 4] = q > K % 4 ? own : b[K / 4];
 #pragma unroll
         for (int i = K / 4 + 1; i < W / 4; i++) b[i] = fma(-Es[K][4 * i + q], x, b[i]);
+        // or the reads of many steps ahead take the registers
+        if (W > 32 && (K < 32 || K % 2)) __builtin_amdgcn_sched_barrier(0);
         unit_steps<K + 1, W>(b, Es, q);
     }
 }
 
-// One wave takes the 16 columns c0 .. c0 + 15 through the panel kb .. kb + w - 1:
-// its interchanges (loads of the panel's rows and of what they displace, then the
-// stores), and with UPDATE, w = W, U12 = L11^{-1} A12 by substitution, a quad of
-// lanes a column, and A22 -= L21 U12 in 16-row tiles on MFMA.  The product is formed
-// transposed, so a load or store of A22 covers 16 consecutive rows of four columns
-// rather than four of sixteen.  Loads run one tile ahead.
+// One wave takes the 16 columns c0 .. c0 + 15 (those below cend) through the K
+// columns at kb (w of them, w = K with UPDATE): their interchanges (loads of rows
+// kb .. and of what they displace, then the stores), and with UPDATE U12 =
+// L11^{-1} A12 by substitution, a quad of lanes a column, and A22 -= L21 U12 in
+// 16-row tiles on MFMA.  With SPLIT nparts waves share the strip: each forms U12, the
+// first stores it, and they take the row tiles in turn; all waves of the workgroup
+// call it, those without a strip with c0 >= cend.
+// The product is formed transposed, so a load or store of A22 covers 16 consecutive
+// rows of four columns rather than four of sixteen.  Loads run ahead of the MFMA by
+// 32 columns of L21 and by a tile of A22.
 // D layouts: f64 16x16x4, element r of lane l = D[l/16 + 4 r][l % 16];
 // f32 16x16x4, element r of lane l = D[4 (l/16) + r][l % 16].
-template <bool UPDATE, typename T, int W, int WL>
-__device__ __forceinline__ void strip(int n, int kb, int w, int c0, int cend, T *a, int lda,
-                                      FactorLds<T, WL> &sl)
+template <bool UPDATE, bool SPLIT, int K, typename T, int LD>
+__device__ __forceinline__ void strip(int n, int kb, int w, int c0, int cend, Global<T> *a, int lda,
+                                      const int *src, const int *dst, bool moved, const T (*Es)[LD],
+                                      T (*Us)[SC + 1], int part, int nparts)
 {
     using acc_t = typename std::conditional<sizeof(T) == 8, bd4_t, bf4_t>::type;
-    constexpr int NI = W / 4;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int NI = K / 4, UR = K < 16 ? K : 16;  // rows of U12 that change layout at once
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));  // else a kernel's worth of offsets is kept, in scratch
     const int lr = lane & 15, lk = lane >> 4;
     T b[NI];
-    const int q = lane & 3, c = lane >> 2;
     {
+        const int q = lane & 3, c = lane >> 2;
         const bool on = c0 + c < cend;
-        T *x = a + (size_t)(on ? c0 + c : c0) * lda;
-        T d[NI];
+        // loads are clamped into the matrix, not predicated: what they bring from
+        // there stays in rows or columns that are not stored
+        Global<T> *x = a + (size_t)min(c0 + c, cend - 1) * lda;
+        if (moved) {
+            T d[NI];
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                const int k = UPDATE ? 4 * i + q : min(4 * i + q, w - 1);
+                b[i] = x[(unsigned)src[k]];
+                d[i] = x[kb + k];
+            }
+            if constexpr (SPLIT) __syncthreads();  // all parts have loaded
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                const int k = 4 * i + q;
+                if (on && k < w && (!SPLIT || part == 0)) {
+                    const int to = dst[k];
+                    if (to >= kb + w) x[(unsigned)to] = d[i];
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < NI; i++) b[i] = x[kb + (UPDATE ? 4 * i + q : min(4 * i + q, w - 1))];
+        }
+        if constexpr (SPLIT) __syncthreads();  // all have loaded; rows of other parts' tiles
+        if constexpr (UPDATE) unit_steps<0, K>(b, Es, q);
 #pragma unroll
         for (int i = 0; i < NI; i++)
-            b[i] = on && 4 * i + q < w ? x[sl.src[kb + 4 * i + q]] : T(0);
-#pragma unroll
-        for (int i = 0; i < NI; i++)
-            if (4 * i + q < sl.ndst) d[i] = x[sl.src[sl.dst[4 * i + q]]];
-#pragma unroll
-        for (int i = 0; i < NI; i++)
-            if (on && 4 * i + q < sl.ndst) x[sl.dst[4 * i + q]] = d[i];
-        if constexpr (UPDATE) unit_steps<0, W>(b, sl.L11, q);
-#pragma unroll
-        for (int i = 0; i < NI; i++)
-            if (on && 4 * i + q < w) x[kb + 4 * i + q] = b[i];
+            if (on && 4 * i + q < w && (!SPLIT || part == 0)) x[kb + 4 * i + q] = b[i];
     }
     if constexpr (UPDATE) {
-        T(*Us)[SC + 1] = sl.U[wave];
+        const int r0 = kb + K, ntile = c0 < cend ? (n - r0 + 15) / 16 : 0;
+        if (SPLIT && part >= ntile) return;
+        // b <- the B operand, row 4 s + lk of column lr
 #pragma unroll
-        for (int i = 0; i < NI; i++) Us[4 * i + q][c] = b[i];
-        __builtin_amdgcn_wave_barrier();
-        T u[NI];
+        for (int g = 0; g < K / UR; g++) {
 #pragma unroll
-        for (int s = 0; s < NI; s++) u[s] = Us[4 * s + lk][lr];
-        __builtin_amdgcn_wave_barrier();
-        const int r0 = kb + W, ntile = (n - r0 + 15) / 16;
-        const T *L = a + (size_t)(r0 + lr) + (size_t)(kb + lk) * lda;
+            for (int i = 0; i < UR / 4; i++) Us[4 * i + (lane & 3)][lane >> 2] = b[g * UR / 4 + i];
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int s = 0; s < UR / 4; s++) b[g * UR / 4 + s] = Us[4 * s + lk][lr];
+            __builtin_amdgcn_wave_barrier();
+        }
         const int cc = c0 + (sizeof(T) == 8 ? lk : 4 * lk);
         constexpr int CS = sizeof(T) == 8 ? 4 : 1;  // columns between a lane's elements
-        T *C = a + (size_t)(r0 + lr) + (size_t)cc * lda;
-        T l[NI], v[4];
-        auto load = [&](T(&l)[NI], T(&v)[4], int t) {
-            const bool ok = r0 + lr + 16 * t < n;
+        const Global<T> *L = a + (size_t)(kb + lk) * lda;
+        Global<T> *C[4];
 #pragma unroll
-            for (int s = 0; s < NI; s++) l[s] = ok ? L[16 * t + (size_t)(4 * s) * lda] : T(0);
+        for (int r = 0; r < 4; r++) C[r] = a + (size_t)min(cc + CS * r, cend - 1) * lda;
+        constexpr int NH = NI > 8 ? 8 : NI, H = NI / NH;  // loads of L21 in H pieces
+        T l[2][NH], v[4];
+        auto load_l = [&](T(&l)[NH], int t, int h) {
+            const Global<T> *Lt = L + min(r0 + lr + 16 * t, n - 1);
+            size_t ld = lda;
+            asm("" : "+s"(ld));  // else sixteen column addresses are kept, in scratch
 #pragma unroll
-            for (int r = 0; r < 4; r++)
-                v[r] = ok && cc + CS * r < cend ? C[16 * t + (size_t)(CS * r) * lda] : T(0);
+            for (int s = 0; s < NH; s++) l[s] = Lt[(size_t)(4 * (h * NH + s)) * ld];
         };
-        load(l, v, 0);
-        for (int t = 0; t < ntile; t++) {
-            T ln[NI], vn[4];
-            load(ln, vn, t + 1);  // nothing past the last tile: its rows are >= n
-            acc_t acc = acc_t{0, 0, 0, 0};
+        auto load_c = [&](T(&v)[4], int t) {
+            const int row = min(r0 + lr + 16 * t, n - 1);
 #pragma unroll
-            for (int s = 0; s < NI; s++) {
+            for (int r = 0; r < 4; r++) v[r] = C[r][row];
+        };
+        auto mm = [&](acc_t &acc, const T(&l)[NH], int h) {
+#pragma unroll
+            for (int s = 0; s < NH; s++) {
                 if constexpr (sizeof(T) == 8)
-                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(u[s], l[s], acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(b[h * NH + s], l[s], acc, 0, 0, 0);
                 else
-                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(u[s], l[s], acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(b[h * NH + s], l[s], acc, 0, 0, 0);
+            }
+        };
+        load_l(l[0], part, 0);
+        if constexpr (H == 1) load_c(v, part);
+        for (int t = part; t < ntile; t += nparts) {
+            T vn[4];
+            acc_t acc = acc_t{0, 0, 0, 0};
+            if constexpr (H == 2) {
+                load_c(v, t);
+                load_l(l[1], t, 1);
+                mm(acc, l[0], 0);
+                load_l(l[0], t + nparts, 0);
+                mm(acc, l[1], 1);
+            } else {
+                load_l(l[1], t + nparts, 0);
+                load_c(vn, t + nparts);
+                mm(acc, l[0], 0);
+#pragma unroll
+                for (int s = 0; s < NH; s++) l[0][s] = l[1][s];
             }
             const bool ok = r0 + lr + 16 * t < n;
 #pragma unroll
-            for (int r = 0; r < 4; r++)
-                if (ok && cc + CS * r < cend) C[16 * t + (size_t)(CS * r) * lda] = v[r] - acc[r];
-#pragma unroll
-            for (int s = 0; s < NI; s++) l[s] = ln[s];
-#pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = vn[r];
+            for (int r = 0; r < 4; r++) {
+                if (ok && cc + CS * r < cend) C[r][r0 + lr + 16 * t] = v[r] - acc[r];
+                if constexpr (H == 1) v[r] = vn[r];
+            }
         }
     }
 }
 
-// The panel of W columns at kb and its strips.
+// The panel at kp of the block kb .. ce - 1 and its strips inside the block; returns
+// its width.
 template <int W, int RPT, typename T, int WL>
-__device__ __forceinline__ void factor_step(int n, int kb, T *a, int lda, int *__restrict__ piv,
-                                            int &info, FactorLds<T, WL> &sl)
+__device__ __forceinline__ int inner_step(int n, int kb, int kp, int ce, Global<T> *a, int lda,
+                                          Global<int> *piv, int &info, FactorLds<T, WL> &sl)
 {
-    const int wave = threadIdx.x >> 6, w = min(W, n - kb);
-    panel_regs<T, W, RPT>(n, kb, w, a, lda, piv, info, sl);
-    for (int c0 = kb + w + SC * wave; c0 < n; c0 += SC * FW)
-        strip<true, T, W>(n, kb, w, c0, n, a, lda, sl);
-    if (sl.moved)
-        for (int c0 = SC * (FW - 1 - wave); c0 < kb; c0 += SC * FW)
-            strip<false, T, W>(n, kb, w, c0, kb, a, lda, sl);
-    __syncthreads();  // the columns are final before the next panel, sl free
+    const int wave = threadIdx.x >> 6, w = min(W, ce - kp);
+    panel_regs<T, W, RPT>(n, kp, w, kp == kb, a, lda, piv, info, sl);
+    const int ns = (ce - kp - w + SC - 1) / SC;
+    if (ns > 0) {
+        const int nparts = FW / ns, si = wave / nparts;
+        strip<true, true, W>(n, kp, w, si < ns ? kp + w + SC * si : ce, ce, a, lda, sl.pm.src,
+                             sl.pm.dst, sl.pm.any, (const T(*)[WL + 1])sl.L11, sl.U[wave], wave % nparts, nparts);
+    }
+    if (sl.pm.any)
+        for (int c0 = kb + SC * wave; c0 < kp; c0 += SC * FW)
+            strip<false, false, W>(n, kp, w, c0, kp, a, lda, sl.pm.src, sl.pm.dst,
+                                   true,
+                                   (const T(*)[WL + 1])sl.L11, sl.U[wave], 0, 1);
+    __syncthreads();  // the block's columns are final before the next panel, sl free
+    return w;
 }
 
-// P A = L U in place by panels of W columns; panels of more than 512 rows keep two
-// rows a thread and are 8 columns wide, which fits the registers.
+// P A = L U in place by blocks of 64 columns: panels of W columns (of 8 where more
+// than 512 rows are left and a thread keeps two: that fits the registers) and their
+// strips inside the block, then the block's strips outside.
 template <typename T, int W>
-__device__ void factor_system(int n, T *a, int lda, int *__restrict__ piv, int &info,
+__device__ __forceinline__ void factor_system(int n, Global<T> *a, int lda, Global<int> *piv, int &info,
                               FactorLds<T, W> &sl)
 {
-    constexpr int W2 = 8;
-    int kb = 0;
-    for (; n - kb > FT; kb += W2) factor_step<W2, 2>(n, kb, a, lda, piv, info, sl);
-    for (; kb < n; kb += W) factor_step<W, 1>(n, kb, a, lda, piv, info, sl);
+    const int tid = threadIdx.x, wave = tid >> 6;
+    for (int kb = 0; kb < n; kb += KB) {
+        const int wb = min(KB, n - kb), ce = kb + wb;
+        for (int kp = kb; kp < ce;) {
+            if (n - kp > FT) kp += inner_step<8, 2>(n, kb, kp, ce, a, lda, piv, info, sl);
+            else kp += inner_step<W, 1>(n, kb, kp, ce, a, lda, piv, info, sl);
+        }
+        if (kb == 0 && ce == n) break;
+        if (tid == 0) sl.bm.any = 0;
+        for (int i = tid; i < KB * KB; i += FT) {
+            const int r = i % KB, k = i / KB;
+            sl.Lb[k][r] = r < wb && k < wb ? a[(size_t)(kb + r) + (size_t)(kb + k) * lda] : T(0);
+        }
+        __syncthreads();
+        for (int r = kb + tid; r < n; r += FT) {
+            const int from = sl.from[r];
+            if (r < ce) sl.bm.src[r - kb] = from;
+            if (from < ce) sl.bm.dst[from - kb] = r;
+            if (from != r) sl.bm.any = 1;
+        }
+        __syncthreads();
+        for (int c0 = ce + SC * wave; c0 < n; c0 += SC * FW)
+            strip<true, false, KB>(n, kb, wb, c0, n, a, lda, sl.bm.src, sl.bm.dst, sl.bm.any,
+                                   (const T(*)[KB + 1])sl.Lb, sl.U[wave], 0, 1);
+        if (sl.bm.any)
+            for (int c0 = SC * (FW - 1 - wave); c0 < kb; c0 += SC * FW)
+                strip<false, false, KB>(n, kb, wb, c0, kb, a, lda, sl.bm.src, sl.bm.dst, true,
+                                        (const T(*)[KB + 1])sl.Lb, sl.U[wave], 0, 1);
+        __syncthreads();  // the columns are final before the next panel, sl free
+    }
 }
 
 // X = U^{-1} L^{-1} P B for all nrhs columns of B at once.
@@ -499,8 +600,8 @@ __global__ __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(4))) void ge
         if (q >= batch) break;
         const int s = order[q];
         const SysDesc d = desc[s];
-        T *a = A[s];
-        int *piv = ipiv[s];
+        Global<T> *a = (Global<T> *)A[s];
+        Global<int> *piv = (Global<int> *)ipiv[s];
         // n < 0 marks a system whose sizes the allocation-free entry rejected
         int inf = d.n < 0 ? -1 : 0;
         if (d.n > 0) factor_system<T, W>(d.n, a, d.lda, piv, inf, sl);
