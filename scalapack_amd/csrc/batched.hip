@@ -38,9 +38,14 @@
 // 292, 1666 -> 870 -> 703, 8764 -> 5849 -> 3468.  2000 FP64 systems of 32 .. 512, the
 // factorization: 12.5 -> 6.0 -> 3.9 ms.
 //
-// The solves take 16-row blocks: one wave solves the diagonal block in
-// registers (lane = row, values broadcast by lane reads), then all waves
-// update the rows below (above) with the new values.
+// The solves, 512 threads: the interchanges as one permutation, then blocks of 64
+// rows for all right-hand sides at once: the diagonal block by substitution on 16 x
+// 16 triangles, the rows outside it by MFMA in tiles of 16 rows (solve_triangle).
+// Bound by the chain of blocks, about 5 us each, for the systems of a CU in turn.
+// Before, blocks of 16 rows each waited for their triangle's row from memory, exchanged
+// values through LDS permutes and updated by dot products, and one thread composed
+// the interchanges.  2000 FP64 systems of 32 .. 512, one to eight right-hand sides:
+// 2.05 -> 0.33 ms; 4000 FP32 systems of 8 .. 160: 227 -> 146 us.
 #include "sla_common.h"
 #include "sla_handle.h"
 #include "sla_batched.h"
@@ -49,6 +54,7 @@
 #include <climits>
 #include <cstdlib>
 #include <cstring>
+#include <limits>
 #include <mutex>
 #include <numeric>
 #include <stdexcept>
@@ -60,8 +66,8 @@ namespace sla {
 
 namespace {
 
-constexpr int FT = 512, FW = FT / 64;  // threads and waves of a factorization's workgroup
-constexpr int BT = 256;                // threads of a solve's
+constexpr int FT = 512, FW = FT / 64;  // threads and waves of a workgroup
+constexpr int SOLVE_WGS = 2;           // workgroups a CU of the solves: what fits
 constexpr int SC = 16;                 // columns of a strip
 constexpr int KB = 64;                 // columns of a block
 
@@ -280,19 +286,26 @@ __device__ __forceinline__ void panel_regs(int n, int kb, int w, bool first, Glo
     __syncthreads();
 }
 
-// b <- L^{-1} b for a column in a quad of lanes, lane q rows 4 i + q.
+// b <- L^{-1} b for a column in a quad of lanes, lane q rows 4 i + q.  What 16 solved
+// values take from the rows after them is summed apart, in s.
 template <int K, int W, typename T, int WL>
-__device__ __forceinline__ void unit_steps(T (&b)[W / 4], const T (*Es)[WL], int q)
+__device__ __forceinline__ void unit_steps(T (&b)[W / 4], T (&s)[W / 4], const T (*Es)[WL], int q)
 {
     if constexpr (K < W) {
+        constexpr int I1 = (K / 16 + 1) * 4 < W / 4 ? (K / 16 + 1) * 4 : W / 4;
         const T x = quad_lane<K % 4>(b[K / 4]);
         const T own = fma(-Es[K][K / 4 * 4 + q], x, b[K / 4]);
         b[K / 4] = q > K % 4 ? own : b[K / 4];
 #pragma unroll
-        for (int i = K / 4 + 1; i < W / 4; i++) b[i] = fma(-Es[K][4 * i + q], x, b[i]);
+        for (int i = K / 4 + 1; i < I1; i++) b[i] = fma(-Es[K][4 * i + q], x, b[i]);
+#pragma unroll
+        for (int i = I1; i < W / 4; i++) {
+            s[i] = K % 16 ? fma(-Es[K][4 * i + q], x, s[i]) : -Es[K][4 * i + q] * x;
+            if (K % 16 == 15) b[i] += s[i];
+        }
         // or the reads of many steps ahead take the registers
         if (W > 32 && (K < 32 || K % 2)) __builtin_amdgcn_sched_barrier(0);
-        unit_steps<K + 1, W>(b, Es, q);
+        unit_steps<K + 1, W>(b, s, Es, q);
     }
 }
 
@@ -347,7 +360,10 @@ __device__ __forceinline__ void strip(int n, int kb, int w, int c0, int cend, Gl
             for (int i = 0; i < NI; i++) b[i] = x[kb + (UPDATE ? 4 * i + q : min(4 * i + q, w - 1))];
         }
         if constexpr (SPLIT) __syncthreads();  // all have loaded; rows of other parts' tiles
-        if constexpr (UPDATE) unit_steps<0, K>(b, Es, q);
+        if constexpr (UPDATE) {
+            T sum[NI];
+            unit_steps<0, K>(b, sum, Es, q);
+        }
 #pragma unroll
         for (int i = 0; i < NI; i++)
             if (on && 4 * i + q < w && (!SPLIT || part == 0)) x[kb + 4 * i + q] = b[i];
@@ -385,37 +401,48 @@ __device__ __forceinline__ void strip(int n, int kb, int w, int c0, int cend, Gl
 #pragma unroll
             for (int r = 0; r < 4; r++) v[r] = C[r][row];
         };
-        auto mm = [&](acc_t &acc, const T(&l)[NH], int h) {
+        // the sums of 16 products are formed apart, or a block's rounding errors grow
+        // above those of as many panels
+        auto mm = [&](acc_t(&acc)[NH > 4 ? 2 : 1], const T(&l)[NH], int h) {
 #pragma unroll
             for (int s = 0; s < NH; s++) {
+                acc_t &c = acc[s / 4];
                 if constexpr (sizeof(T) == 8)
-                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(b[h * NH + s], l[s], acc, 0, 0, 0);
+                    c = __builtin_amdgcn_mfma_f64_16x16x4f64(b[h * NH + s], l[s], c, 0, 0, 0);
                 else
-                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(b[h * NH + s], l[s], acc, 0, 0, 0);
+                    c = __builtin_amdgcn_mfma_f32_16x16x4f32(b[h * NH + s], l[s], c, 0, 0, 0);
             }
+        };
+        auto take = [&](T(&v)[4], const acc_t(&acc)[NH > 4 ? 2 : 1]) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] -= NH > 4 ? acc[0][r] + acc[NH > 4][r] : acc[0][r];
         };
         load_l(l[0], part, 0);
         if constexpr (H == 1) load_c(v, part);
         for (int t = part; t < ntile; t += nparts) {
             T vn[4];
-            acc_t acc = acc_t{0, 0, 0, 0};
+            acc_t acc[NH > 4 ? 2 : 1] = {};
             if constexpr (H == 2) {
                 load_c(v, t);
                 load_l(l[1], t, 1);
                 mm(acc, l[0], 0);
                 load_l(l[0], t + nparts, 0);
-                mm(acc, l[1], 1);
+                acc_t acc2[2] = {};
+                mm(acc2, l[1], 1);
+                take(v, acc);
+                take(v, acc2);
             } else {
                 load_l(l[1], t + nparts, 0);
                 load_c(vn, t + nparts);
                 mm(acc, l[0], 0);
+                take(v, acc);
 #pragma unroll
                 for (int s = 0; s < NH; s++) l[0][s] = l[1][s];
             }
             const bool ok = r0 + lr + 16 * t < n;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                if (ok && cc + CS * r < cend) C[r][r0 + lr + 16 * t] = v[r] - acc[r];
+                if (ok && cc + CS * r < cend) C[r][r0 + lr + 16 * t] = v[r];
                 if constexpr (H == 1) v[r] = vn[r];
             }
         }
@@ -484,105 +511,206 @@ __device__ __forceinline__ void factor_system(int n, Global<T> *a, int lda, Glob
     }
 }
 
-// X = U^{-1} L^{-1} P B for all nrhs columns of B at once.
-//   P: the interchanges composed once into a permutation in LDS (thread 0,
-//      pdlapv2.f:208-242's order), then every column gathered through LDS;
-//   L (unit lower) top down and U bottom up in 16-row blocks: the diagonal
-//      block by substitution in registers, lane = row of one of four
-//      columns per wave (four waves: sixteen columns at a time), the block's
-//      row of the triangle loaded before the substitution; then every thread
-//      updates rows outside the block for one column (dot product over the
-//      block).
+// LDS of a solve.
 template <typename T>
-__device__ void solve_all(int n, const T *__restrict__ a, int lda, const int *__restrict__ piv,
-                          T *__restrict__ B, int ldb, int nrhs, int *s_perm, int *s_piv, T *s_x)
+struct SolveLds {
+    T Es[KB][KB + 1];  // the diagonal block, column k in row k
+    T Xs[KB][SC + 1];  // its solution
+    T rd[KB];          // reciprocals of U's diagonal
+    alignas(16) int piv[BATCHED_NMAX];
+    int moved;
+};
+
+// The value of lane K of every row of 16 lanes, in all of them.
+template <int K, typename T>
+__device__ __forceinline__ T row_lane(T v)
 {
-    constexpr int SB = 16;  // rows per diagonal block
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int lr = lane & (SB - 1), grp = lane / SB;  // row in the block, column of the wave
-    for (int i = tid; i < n; i += BT) {
-        s_perm[i] = i;
-        s_piv[i] = piv[i] - 1;
+    if constexpr (sizeof(T) == 8) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, 0x150 + K, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), 0x150 + K, 0xf, 0xf, false);
+        return __builtin_bit_cast(T, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+    } else {
+        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                                                 0x150 + K, 0xf, 0xf, false));
+    }
+}
+
+// Steps of a 16 x 16 triangle, top down (L, unit) or bottom up (U): lane l of a row
+// of 16 lanes holds row l of b[0], and in b[1] .. b[3] what the solved values take
+// from a row each of the triangles after it; e[i][k (KB + 1)] is column k of those
+// rows.  A
+// quotient is the product with the reciprocal and one correction by its residual;
+// where that is not finite it is divided out.
+template <int S, bool FWD, typename T>
+__device__ __forceinline__ void solve_steps(T (&b)[4], T &x, const T *const (&e)[4], const T *rd, int l)
+{
+    if constexpr (S < 16) {
+        constexpr int K = FWD ? S : 15 - S;
+        T v = b[0];
+        if (!FWD) {
+            const T d = e[0][K * (KB + 1) + K - l], r = rd[K], y = v * r;
+            v = fma(fma(-d, y, v), r, y);
+            if (!(fabs(v) <= std::numeric_limits<T>::max())) v = b[0] / d;
+        }
+        v = row_lane<K>(v);
+        x = l == K ? v : x;
+#pragma unroll
+        for (int i = 0; i < 4; i++) b[i] = fma(-e[i][K * (KB + 1)], v, b[i]);
+        solve_steps<S + 1, FWD>(b, x, e, rd, l);
+    }
+}
+
+// X <- L^{-1} X (FWD) or U^{-1} X for all nrhs <= 16 columns at once, right-looking in
+// blocks of 64 rows: the diagonal block as four 16 x 16 triangles, a column in each
+// row of 16 lanes of waves 0 .. 3, then the rows below (above) in tiles of 16 on MFMA,
+// formed transposed like the strips of the factorization.
+template <bool FWD, typename T>
+__device__ __forceinline__ void solve_triangle(int n, const Global<T> *a, int lda, Global<T> *X, int ldx,
+                                               int nrhs, SolveLds<T> &sl)
+{
+    using acc_t = typename std::conditional<sizeof(T) == 8, bd4_t, bf4_t>::type;
+    constexpr int NE = KB * KB / FT, NS = KB / 4;
+    constexpr int CS = sizeof(T) == 8 ? 4 : 1;  // columns between a lane's elements
+    const int wave = threadIdx.x >> 6, nblk = (n + KB - 1) / KB;
+    int lane = threadIdx.x & 63;
+    // blocks count from the end they start at: only the last one can be short
+    auto first_row = [&](int s) { return FWD ? KB * s : max(n - KB * (s + 1), 0); };
+    T en[NE];  // the next diagonal block: row lane, columns wave + 8 i
+    auto load_diag = [&](int rb) {
+#pragma unroll
+        for (int i = 0; i < NE; i++)
+            en[i] = a[(size_t)min(rb + lane, n - 1) + (size_t)min(rb + wave + FW * i, n - 1) * lda];
+    };
+    load_diag(first_row(0));
+    for (int s = 0; s < nblk; s++) {
+        const int rb = first_row(s), rows = min(KB, FWD ? n - rb : n - KB * s);
+        asm volatile("" : "+v"(lane));  // else all offsets of a block are kept, in scratch
+        const int lr = lane & 15, lk = lane >> 4;
+#pragma unroll
+        for (int i = 0; i < NE; i++) {
+            const int k = wave + FW * i;
+            const bool in = lane < rows && k < rows;
+            sl.Es[k][lane] = in ? en[i] : T(0);
+            if (!FWD && lane == k) sl.rd[k] = in ? T(1) / en[i] : T(1);
+        }
+        const int j = 4 * wave + lk;
+        T y[4];
+        if (4 * wave < nrhs) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int r = 16 * (FWD ? i : 3 - i) + lr;
+                y[i] = X[(size_t)min(rb + r, n - 1) + (size_t)min(j, nrhs - 1) * ldx];
+                y[i] = r < rows ? y[i] : T(0);
+            }
+        }
+        __syncthreads();  // Es
+        if (4 * wave < nrhs) {
+#pragma unroll 1
+            for (int i = 0; i < 4; i++) {
+                const int r0 = 16 * (FWD ? i : 3 - i);
+                T bb[4] = {y[0], T(0), T(0), T(0)};
+                const T *e[4];  // rows r0, and those of bb[1] .. bb[3] (a row of the block if none)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    e[q] = &sl.Es[r0][(FWD ? min(r0 + 16 * q, KB - 16) : max(r0 - 16 * q, 0)) + lr];
+                T x = T(0);
+                if (r0 < rows) solve_steps<0, FWD>(bb, x, e, sl.rd + r0, lr);
+                sl.Xs[r0 + lr][j] = r0 + lr < rows ? x : T(0);
+                if (r0 + lr < rows && j < nrhs) X[(size_t)(rb + r0 + lr) + (size_t)j * ldx] = x;
+                y[0] = y[1] + bb[1], y[1] = y[2] + bb[2], y[2] = y[3] + bb[3];
+            }
+        }
+        __syncthreads();  // Xs; Es is free
+        if (s + 1 == nblk) break;
+        const int r0 = FWD ? rb + KB : 0, rend = FWD ? n : rb;
+        const int ntile = (rend - r0 + 15) / 16;
+        if (wave < ntile) {
+            T u[NS];  // columns without a right-hand side hold anything: theirs alone
+#pragma unroll
+            for (int i = 0; i < NS; i++) u[i] = sl.Xs[4 * i + lk][lr];
+            const int cc = sizeof(T) == 8 ? lk : 4 * lk;
+            for (int t = wave; t < ntile; t += FW) {
+                const int row = r0 + 16 * t + lr, lrow = min(row, rend - 1);
+                T l[NS], v[4];
+                size_t ld = lda;
+                asm("" : "+s"(ld));
+                const Global<T> *Lt = a + lrow + (size_t)(rb + lk) * lda;
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    v[r] = X[(size_t)lrow + (size_t)min(cc + CS * r, nrhs - 1) * ldx];
+#pragma unroll
+                for (int i = 0; i < NS; i++) l[i] = Lt[(size_t)(4 * i) * ld];  // a full block
+                acc_t acc[4] = {};  // as in the strips
+#pragma unroll
+                for (int i = 0; i < NS; i++) {
+                    acc_t &c = acc[i / 4];
+                    if constexpr (sizeof(T) == 8)
+                        c = __builtin_amdgcn_mfma_f64_16x16x4f64(u[i], l[i], c, 0, 0, 0);
+                    else
+                        c = __builtin_amdgcn_mfma_f32_16x16x4f32(u[i], l[i], c, 0, 0, 0);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (row < rend && cc + CS * r < nrhs)
+                        X[(size_t)row + (size_t)(cc + CS * r) * ldx] =
+                            v[r] - ((acc[0][r] + acc[1][r]) + (acc[2][r] + acc[3][r]));
+            }
+        }
+        load_diag(first_row(s + 1));          // on its way while the stores of X are
+        __syncthreads();                     // X, before the next block reads it
+    }
+}
+
+// X = U^{-1} L^{-1} P B for all nrhs columns of B at once.  The interchanges: each
+// thread follows its rows through all of them (n steps on registers, four pivots a
+// read of LDS), then the rows move at once.
+template <typename T>
+__device__ __forceinline__ void solve_all(int n, const Global<T> *a, int lda, const Global<int> *piv,
+                                          Global<T> *B, int ldb, int nrhs, SolveLds<T> &sl)
+{
+    constexpr int RPT = BATCHED_NMAX / FT, NC = 4;
+    const int tid = threadIdx.x, n4 = (n + 3) & ~3;
+    if (tid == 0) sl.moved = 0;
+    __syncthreads();
+    for (int i = tid; i < n4; i += FT) {
+        const int p = i < n ? piv[i] - 1 : i;
+        sl.piv[i] = p;
+        if (p != i) sl.moved = 1;
     }
     __syncthreads();
-    if (tid == 0)
-        for (int j = 0; j < n; j++) {
-            const int p = s_piv[j];
-            if (p != j) {
-                const int t = s_perm[j];
-                s_perm[j] = s_perm[p];
-                s_perm[p] = t;
-            }
-        }
-    __syncthreads();
-    for (int c = 0; c < nrhs; c++) {
-        T *x = B + (size_t)c * ldb;
-        for (int i = tid; i < n; i += BT) s_x[i] = x[s_perm[i]];
-        __syncthreads();
-        for (int i = tid; i < n; i += BT) x[i] = s_x[i];
-        __syncthreads();
-    }
-    // L, 16-row blocks top down
-    for (int b0 = 0; b0 < n; b0 += SB) {
-        const int rows = min(SB, n - b0);
-        for (int c = 4 * wave + grp; c - grp < nrhs; c += 16) {
-            const bool on = c < nrhs && lr < rows;
-            T *x = B + (size_t)(on ? c : 0) * ldb;
-            const T *ar = a + (size_t)(b0 + lr) + (size_t)b0 * lda;
-            T lrow[SB];
+    if (sl.moved) {
+        int to[RPT];
 #pragma unroll
-            for (int i = 0; i < SB; i++) lrow[i] = (on && i < lr) ? ar[(size_t)i * lda] : T(0);
-            T v = on ? x[b0 + lr] : T(0);
+        for (int q = 0; q < RPT; q++) to[q] = tid + FT * q;
+        for (int j = 0; j < n4; j += 4) {
+            const int4 p4 = *reinterpret_cast<const int4 *>(&sl.piv[j]);
+            const int p[4] = {p4.x, p4.y, p4.z, p4.w};
 #pragma unroll
-            for (int i = 0; i < SB; i++) {
-                const T xi = __shfl(v, i + SB * grp);
-                if (lr > i) v = fma(-lrow[i], xi, v);
-            }
-            if (on) x[b0 + lr] = v;
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int q = 0; q < RPT; q++)
+                    to[q] = to[q] == j + i ? p[i] : to[q] == p[i] ? j + i : to[q];
         }
-        __syncthreads();
-        const int below = n - b0 - rows;
-        for (int idx = tid; idx < below * nrhs; idx += BT) {
-            const int i = b0 + rows + idx % below, c = idx / below;
-            T *x = B + (size_t)c * ldb;
-            T acc = T(0);
-            for (int k = 0; k < rows; k++) acc = fma(a[(size_t)i + (size_t)(b0 + k) * lda], x[b0 + k], acc);
-            x[i] -= acc;
+        for (int c0 = 0; c0 < nrhs; c0 += NC) {
+            T v[RPT][NC];
+#pragma unroll
+            for (int q = 0; q < RPT; q++)
+#pragma unroll
+                for (int c = 0; c < NC; c++)
+                    v[q][c] = B[(size_t)min(tid + FT * q, n - 1) + (size_t)min(c0 + c, nrhs - 1) * ldb];
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < RPT; q++)
+#pragma unroll
+                for (int c = 0; c < NC; c++)
+                    if (tid + FT * q < n && c0 + c < nrhs)
+                        B[(size_t)to[q] + (size_t)(c0 + c) * ldb] = v[q][c];
         }
         __syncthreads();
     }
-    // U (non-unit), 16-row blocks bottom up
-    const int nb = (n + SB - 1) / SB;
-    for (int bb = nb - 1; bb >= 0; bb--) {
-        const int b0 = bb * SB, rows = min(SB, n - b0);
-        for (int c = 4 * wave + grp; c - grp < nrhs; c += 16) {
-            const bool on = c < nrhs && lr < rows;
-            T *x = B + (size_t)(on ? c : 0) * ldb;
-            const T *ar = a + (size_t)(b0 + lr) + (size_t)b0 * lda;
-            T urow[SB];
-#pragma unroll
-            for (int i = 0; i < SB; i++)
-                urow[i] = (on && i > lr && i < rows) ? ar[(size_t)i * lda] : T(0);
-            const T d = on ? ar[(size_t)lr * lda] : T(1);
-            T v = on ? x[b0 + lr] : T(0);
-#pragma unroll
-            for (int i = SB - 1; i >= 0; i--) {
-                if (lr == i && i < rows) v = v / d;
-                const T xi = __shfl(v, i + SB * grp);
-                if (lr < i && i < rows) v = fma(-urow[i], xi, v);
-            }
-            if (on) x[b0 + lr] = v;
-        }
-        __syncthreads();
-        for (int idx = tid; idx < b0 * nrhs; idx += BT) {
-            const int i = idx % b0, c = idx / b0;
-            T *x = B + (size_t)c * ldb;
-            T acc = T(0);
-            for (int k = 0; k < rows; k++) acc = fma(a[(size_t)i + (size_t)(b0 + k) * lda], x[b0 + k], acc);
-            x[i] -= acc;
-        }
-        __syncthreads();
-    }
+    solve_triangle<true>(n, a, lda, B, ldb, nrhs, sl);
+    solve_triangle<false>(n, a, lda, B, ldb, nrhs, sl);
 }
 
 template <typename T, int W>
@@ -614,26 +742,24 @@ __global__ __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(4))) void ge
 // persistent queue (queue[1]), after the factorization launch: a kernel of
 // its own keeps its registers out of the factorization's.
 template <typename T>
-__global__ __launch_bounds__(BT) void getrs_batched_kernel(int batch, const int *__restrict__ order,
-                                                           const SysDesc *__restrict__ desc,
-                                                           T *const *__restrict__ A,
-                                                           int *const *__restrict__ ipiv,
-                                                           T *const *__restrict__ B,
-                                                           const int *__restrict__ info, int *queue)
+__global__ __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(4))) void getrs_batched_kernel(
+    int batch, const int *__restrict__ order, const SysDesc *__restrict__ desc,
+    T *const *__restrict__ A, int *const *__restrict__ ipiv, T *const *__restrict__ B,
+    const int *__restrict__ info, int *queue)
 {
     __shared__ int s_q;
-    __shared__ int s_perm[BATCHED_NMAX], s_piv[BATCHED_NMAX];
-    __shared__ T s_x[BATCHED_NMAX];
+    __shared__ SolveLds<T> sl;
     for (;;) {
         if (threadIdx.x == 0) s_q = atomicAdd(queue + 1, 1);
         __syncthreads();
-        const int q = s_q;
+        const int q = __builtin_amdgcn_readfirstlane(s_q);
         __syncthreads();
         if (q >= batch) break;
         const int s = order[q];
         const SysDesc d = desc[s];
         if (d.n > 0 && d.nrhs > 0 && info[s] == 0)
-            solve_all<T>(d.n, A[s], d.lda, ipiv[s], B[s], d.ldb, d.nrhs, s_perm, s_piv, s_x);
+            solve_all<T>(d.n, (const Global<T> *)A[s], d.lda, (const Global<int> *)ipiv[s],
+                         (Global<T> *)B[s], d.ldb, d.nrhs, sl);
         __syncthreads();
     }
 }
@@ -765,7 +891,7 @@ void launch(const BatchedPlan &p, int w, int wgs, int solve_wgs, T *const *A, in
     }
 #undef SLA_BATCHED
     SLA_LAUNCH_CHECK();
-    hipLaunchKernelGGL(getrs_batched_kernel<T>, dim3(solve_wgs), dim3(BT), 0, s, p.batch,
+    hipLaunchKernelGGL(getrs_batched_kernel<T>, dim3(solve_wgs), dim3(FT), 0, s, p.batch,
                        p.d_order, p.d_desc, (T *const *)A, ipiv, B, info, p.d_queue);
     SLA_LAUNCH_CHECK();
 }
@@ -883,7 +1009,7 @@ void gesv_batched_noalloc_device(Handle &h, int batch, const int *dn, const int 
     }
 #undef SLA_BATCHED
     SLA_LAUNCH_CHECK();
-    hipLaunchKernelGGL(getrs_batched_kernel<T>, dim3(4 * h.num_cus), dim3(BT), 0, h.stream, batch,
+    hipLaunchKernelGGL(getrs_batched_kernel<T>, dim3(SOLVE_WGS * h.num_cus), dim3(FT), 0, h.stream, batch,
                        order, desc, (T *const *)dA, (int *const *)dipiv, dB, dinfo, queue);
     SLA_LAUNCH_CHECK();
 }
@@ -905,7 +1031,7 @@ void gesv_batched_device(Handle &h, int batch, const int *n, const int *nrhs, T 
     const int wgs = std::max(1, h.batched_wgs_per_cu) * h.num_cus;
     const int prec = sizeof(T) == 8 ? 0 : 1;
     if (!h.batched_graph) {
-        launch<T>(p, w, wgs, 4 * h.num_cus, dA, dipiv, dB, dinfo, h.stream);
+        launch<T>(p, w, wgs, SOLVE_WGS * h.num_cus, dA, dipiv, dB, dinfo, h.stream);
         SLA_HIP(hipStreamSynchronize(h.stream));
         return;
     }
@@ -925,7 +1051,7 @@ void gesv_batched_device(Handle &h, int batch, const int *n, const int *nrhs, T 
         hipGraph_t g = nullptr;
         SLA_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
         try {
-            launch<T>(p, w, wgs, 4 * h.num_cus, dA, dipiv, dB, dinfo, cs);
+            launch<T>(p, w, wgs, SOLVE_WGS * h.num_cus, dA, dipiv, dB, dinfo, cs);
         } catch (...) {
             (void)hipStreamEndCapture(cs, &g);
             if (g) (void)hipGraphDestroy(g);
@@ -1001,7 +1127,7 @@ BatchedTune tune_batched_device(Handle &h, int batch, const int *n, const int *n
                 hipLaunchKernelGGL(fill_synthetic_kernel<T>, dim3(64, std::min(batch, 65535)), dim3(256), 0, h.stream,
                                    batch, p.d_desc, dA, dB);
                 SLA_HIP(hipEventRecord(e0, h.stream));
-                launch<T>(p, w, k * h.num_cus, 4 * h.num_cus, dA, dP, dB, info, h.stream);
+                launch<T>(p, w, k * h.num_cus, SOLVE_WGS * h.num_cus, dA, dP, dB, info, h.stream);
                 SLA_HIP(hipEventRecord(e1, h.stream));
                 SLA_HIP(hipEventSynchronize(e1));
                 float ms = 0.f;
