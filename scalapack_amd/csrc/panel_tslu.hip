@@ -32,11 +32,6 @@
 
 #include <climits>
 
-// wavefront-wide maximum of the ROCm device library (declared by the HIP
-// headers only with their optional 64-bit warp-sync types)
-extern "C" __device__ __attribute__((const)) unsigned long long __ockl_wfred_max_u64(
-    unsigned long long);
-
 namespace sla {
 
 namespace {
@@ -44,72 +39,115 @@ namespace {
 constexpr int TPT = 512;         // threads per workgroup
 constexpr int TNW = TPT / 64;    // waves per workgroup
 constexpr int TW = 32;           // leaf width
-constexpr int TMR = 2;           // candidate rows per thread in the tournament
+constexpr int TMR = 2;           // candidate rows per thread in the tournament at most
 constexpr int TGMAX = TPT * TMR / TW;  // workgroups per launch at most (32)
 // candidate values are stored column by column (value c of candidate sid at
 // c * TCAND + sid), so the tournament's loads are contiguous across lanes
 constexpr int TCAND = TGMAX * TW;
 
-// Pivot key of a row: |v| as float bits (monotone for |v| >= 0; a NaN counts
-// as zero) in the upper half, INT_MAX - row in the lower, so the larger key
-// is the larger magnitude and, on a tie, the lower row; 0 = no row.
-__device__ __forceinline__ uint64_t piv_key(float v, int row)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_max(uint32_t x)
+{
+    // lanes the move does not reach combine with 0
+    const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
+    return x > y ? x : y;
+}
+
+// Wave-wide maximum, uniform.
+__device__ __forceinline__ uint32_t wave_max(uint32_t x)
+{
+    x = dpp_max<0x121, 0xf>(x);
+    x = dpp_max<0x122, 0xf>(x);
+    x = dpp_max<0x124, 0xf>(x);
+    x = dpp_max<0x128, 0xf>(x);
+    x = dpp_max<0x142, 0xa>(x);
+    x = dpp_max<0x143, 0xc>(x);
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+
+// A barrier that waits for the workgroup's LDS traffic only.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Rank of a pivot candidate: 0 for no row, else 1 + |v|'s bits (monotone; a NaN
+// counts as zero).  Equal ranks are decided by the lower row.
+__device__ __forceinline__ uint32_t piv_rank(float v, bool act)
 {
     const float a = fabsf(v);
-    const uint32_t ab = (a == a) ? __float_as_uint(a) : 0u;
-    return row == INT_MAX ? 0ull : (((uint64_t)ab << 32) | (uint32_t)(INT_MAX - row));
+    return act ? ((a == a) ? __float_as_uint(a) : 0u) + 1u : 0u;
 }
 
 // Partial-pivoting elimination over the rows a whole workgroup holds (NR
 // per thread; key = row identity and tie-break, INT_MAX = no row; pid =
 // payload id).  Selects up to wa pivots in order: out_key[j], out_pid[j]
-// (written by thread 0); with s_u, row j of U (columns j..) goes to s_u[j].
-// Per column: one wave max over the packed pivot keys, the winning lane of
-// every wave posts its row to LDS, one workgroup barrier, every thread folds
-// the 8 posts in the same order and applies the rank-1 update with the
-// winner's row.  The posts are double-buffered by column parity: a buffer is
-// rewritten two columns later, after a barrier every reader has passed.
+// (written by the row's owner); with s_u, row j of U (columns j..) goes to s_u[j].
+// Per column: one wave maximum of the ranks, the winning lane of every wave
+// posts its row and the reciprocal of its pivot to LDS, one workgroup barrier,
+// every wave folds the 8 posts in the same order by lane moves and applies the
+// rank-1 update with the winner's row.  The posts are double-buffered by column
+// parity: a buffer is rewritten two columns later, after a barrier every reader
+// has passed.
 //
 // The columns rotate through the registers: at step j, register column 0
 // holds matrix column j, and the update writes column c+1's new value into
 // register column c, so every register index is a compile-time constant while
 // the step loop stays rolled.
+//
+// Bound: the chain of a column (search, post, barrier, fold, row, update), of
+// which a leaf has 2 W; beside the trailing update, which shares the SIMDs, every
+// part of it takes about half as long again.  Of the parts the LDS takes most:
+// sixteen 16-byte accesses a wave for a row of 32 columns.  So the steps run on 32,
+// 24, 16 and 8 columns, as many as are left (four copies of the loop; unrolling
+// all steps would be fetched cold at every launch).  Reading one element a lane and
+// passing the rest by DPP was 6 % slower.  Maxima of 32-bit ranks by lane moves
+// replace a 64-bit reduction and a fold of eight keys one after another, and a
+// thread takes one candidate in the tournament when there are at most 512.
+// A leaf of m rows alone, us, before -> this: m = 4000 103 -> 76, 26000 131 -> 97;
+// a factorization step is 1.1 -> 0.75 us.
 struct alignas(16) GeppLds {
-    uint64_t wkey[2][TNW];
     float wrow[2][TNW][TW];
-    int wpid[2][TNW];
+    uint32_t wrank[2][TNW];
+    int wkey[2][TNW];
+    float wrcp[2][TNW];
 };
 typedef float f4_t __attribute__((ext_vector_type(4)));
-typedef unsigned long long u2_t __attribute__((ext_vector_type(2)));
 
-template <typename T, int NR, bool FULL>
-__device__ __forceinline__ void wg_gepp(T (&v)[NR][TW], const int (&key)[NR], const int (&pid)[NR],
-                                        int wa, int *out_key, int *out_pid, GeppLds &sl,
-                                        T (*s_u)[TW + 1])
+// Steps j0 .. j1 - 1, in which the rows have at most NC columns left.
+template <int NC, typename T, int NR>
+__device__ __forceinline__ void gepp_steps(T (&v)[NR][TW], const int (&key)[NR], const int (&pid)[NR],
+                                           bool (&act)[NR], int j0, int j1, int *out_key,
+                                           int *out_pid, GeppLds &sl, T (*s_u)[TW + 1])
 {
-    static_assert(sizeof(T) == 4, "the packed pivot key holds a float magnitude");
+    static_assert(sizeof(T) == 4, "the rank holds a float magnitude");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    bool act[NR];
-#pragma unroll
-    for (int q = 0; q < NR; q++) act[q] = key[q] != INT_MAX;
-    const int steps = FULL ? TW : wa;
 #pragma unroll 1
-    for (int j = 0; j < steps; j++) {
+    for (int j = j0; j < j1; j++) {
         const int pb = j & 1;
-        uint64_t bk = 0;
-        int bq = 0;
+        uint32_t bk = piv_rank(v[0][0], act[0]);
+        int bq = 0, bkey = key[0];
 #pragma unroll
-        for (int q = 0; q < NR; q++) {
-            const uint64_t k = act[q] ? piv_key(v[q][0], key[q]) : 0ull;
-            if (k > bk) {
+        for (int q = 1; q < NR; q++) {
+            const uint32_t k = piv_rank(v[q][0], act[q]);
+            if (k > bk || (k == bk && key[q] < bkey)) {
                 bk = k;
                 bq = q;
+                bkey = key[q];
             }
         }
-        const uint64_t wmax = __ockl_wfred_max_u64(bk);
-        if (wmax != 0 && bk == wmax) {  // the one lane holding the wave's winner
+        const uint32_t wmax = wave_max(bk);
+        uint64_t in = __ballot(bk == wmax);
+        if (in & (in - 1)) {  // shared: the lowest row (rows are below INT_MAX)
+            const uint32_t nm = wave_max(bk == wmax ? ~(uint32_t)bkey : 0u);
+            in = __ballot(bk == wmax && ~(uint32_t)bkey == nm);
+        }
+        const int wl = __builtin_ctzll(in);
+        if (lane == wl) {
 #pragma unroll
-            for (int c4 = 0; c4 < TW; c4 += 4) {
+            for (int c4 = 0; c4 < NC; c4 += 4) {
                 f4_t sel4;
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
@@ -119,51 +157,49 @@ __device__ __forceinline__ void wg_gepp(T (&v)[NR][TW], const int (&key)[NR], co
                     sel4[e] = sel;
                 }
                 *reinterpret_cast<f4_t *>(&sl.wrow[pb][wave][c4]) = sel4;
+                if (c4 == 0) sl.wrcp[pb][wave] = sel4[0] != T(0) ? T(1) / sel4[0] : T(0);
             }
-            int sp = pid[0];
-#pragma unroll
-            for (int q = 1; q < NR; q++) sp = (bq == q) ? pid[q] : sp;
-            sl.wpid[pb][wave] = sp;
+            sl.wrank[pb][wave] = bk;
+            sl.wkey[pb][wave] = bkey;
         }
-        if (lane == 0) sl.wkey[pb][wave] = wmax;
-        __syncthreads();
-        u2_t kk[TNW / 2];
-#pragma unroll
-        for (int w = 0; w < TNW / 2; w++) kk[w] = reinterpret_cast<const u2_t *>(sl.wkey[pb])[w];
-        uint64_t fk = kk[0][0];
-        int fw = 0;
-#pragma unroll
-        for (int w = 1; w < TNW; w++) {
-            const uint64_t k = kk[w / 2][w % 2];
-            if (k > fk) {
-                fk = k;
-                fw = w;
-            }
+        lds_barrier();
+        const uint32_t fr = sl.wrank[pb][lane & (TNW - 1)];
+        const int fkey = sl.wkey[pb][lane & (TNW - 1)];
+        uint32_t fm = dpp_max<0x121, 0xf>(fr);
+        fm = dpp_max<0x122, 0xf>(fm);
+        fm = dpp_max<0x124, 0xf>(fm);
+        uint32_t fin = (uint32_t)__ballot(fr == fm) & ((1u << TNW) - 1u);
+        if (fin & (fin - 1)) {
+            const uint32_t nm = wave_max(fr == fm ? ~(uint32_t)fkey : 0u);
+            fin = (uint32_t)__ballot(fr == fm && ~(uint32_t)fkey == nm) & ((1u << TNW) - 1u);
         }
-        // fk == 0 (uniform): no rows left -- no pivot, and every multiplier
+        const int fw = __builtin_ctz(fin);
+        // rank 0 (uniform): no rows left -- no pivot, and every multiplier
         // below is 0 because no row is active
-        const bool any = fk != 0;
-        if (any && bk == fk) {  // the owner of the pivot row retires it
-#pragma unroll
-            for (int q = 0; q < NR; q++)
-                if (bq == q) act[q] = false;
-        }
+        const bool any = __builtin_amdgcn_readlane((int)fr, fw) != 0;
         const float *prow = sl.wrow[pb][fw];
-        if (tid == 0) {
-            out_key[j] = any ? INT_MAX - (int)(uint32_t)fk : INT_MAX;
-            out_pid[j] = any ? sl.wpid[pb][fw] : -1;
-        }
-        if (any && s_u != nullptr && tid < TW - j) s_u[j][j + tid] = prow[tid];
-        T pr[TW];
+        const T rcp = sl.wrcp[pb][fw];
+        const T ux = prow[lane & (TW - 1)];  // waited for with the row
+        T pr[NC];
 #pragma unroll
-        for (int c4 = 0; c4 < TW; c4 += 4) {
+        for (int c4 = 0; c4 < NC; c4 += 4) {
             const f4_t x = reinterpret_cast<const f4_t *>(prow)[c4 / 4];
 #pragma unroll
             for (int e = 0; e < 4; e++) pr[c4 + e] = x[e];
         }
-        const T pj = pr[0];
-        const bool nz = pj != T(0);
-        const T rcp = nz ? T(1) / pj : T(0);
+        if (wave == fw && lane == wl) {  // the owner of the pivot row retires it
+            out_key[j] = any ? bkey : INT_MAX;
+            int sp = -1;
+#pragma unroll
+            for (int q = 0; q < NR; q++)
+                if (any && bq == q) {
+                    act[q] = false;
+                    sp = pid[q];
+                }
+            out_pid[j] = sp;
+        }
+        if (any && s_u != nullptr && tid < TW - j) s_u[j][j + tid] = ux;
+        const bool nz = pr[0] != T(0);
         // every row rotates (a retired row with multiplier 0: its values are
         // never read again), so the registers need no copies between steps
 #pragma unroll
@@ -172,10 +208,25 @@ __device__ __forceinline__ void wg_gepp(T (&v)[NR][TW], const int (&key)[NR], co
             if (nz) l = l * rcp;
             l = act[q] ? l : T(0);
 #pragma unroll
-            for (int c = 1; c < TW; c++) v[q][c - 1] = fma(-l, pr[c], v[q][c]);
-            v[q][TW - 1] = T(0);
+            for (int c = 1; c < NC; c++) v[q][c - 1] = fma(-l, pr[c], v[q][c]);
+            v[q][NC - 1] = T(0);
         }
     }
+}
+
+template <typename T, int NR, bool FULL>
+__device__ __forceinline__ void wg_gepp(T (&v)[NR][TW], const int (&key)[NR], const int (&pid)[NR],
+                                        int wa, int *out_key, int *out_pid, GeppLds &sl,
+                                        T (*s_u)[TW + 1])
+{
+    bool act[NR];
+#pragma unroll
+    for (int q = 0; q < NR; q++) act[q] = key[q] != INT_MAX;
+    const int steps = FULL ? TW : wa;
+    gepp_steps<32>(v, key, pid, act, 0, min(steps, 8), out_key, out_pid, sl, s_u);
+    gepp_steps<24>(v, key, pid, act, 8, min(steps, 16), out_key, out_pid, sl, s_u);
+    gepp_steps<16>(v, key, pid, act, 16, min(steps, 24), out_key, out_pid, sl, s_u);
+    gepp_steps<8>(v, key, pid, act, 24, steps, out_key, out_pid, sl, s_u);
     __syncthreads();  // out_* and s_u complete before anyone reads them
 }
 
@@ -186,7 +237,7 @@ __device__ __forceinline__ int colx(int c, int wa)
 }
 
 // FULL: the leaf is TW columns wide (no column predicates).
-template <typename T, int RPT, bool FULL>
+template <typename T, int RPT, int MR, bool FULL>
 __global__ __launch_bounds__(TPT) void panel_tslu_kernel(
     T *__restrict__ A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0,
     int *__restrict__ ipiv, TsluSlots<T> slots, unsigned *ctr, unsigned target, int *abort_flag,
@@ -248,10 +299,10 @@ __global__ __launch_bounds__(TPT) void panel_tslu_kernel(
     __syncthreads();
     {
         const int total = G * TW;
-        T v[TMR][TW];
-        int key[TMR], pid[TMR];
+        T v[MR][TW];
+        int key[MR], pid[MR];
 #pragma unroll
-        for (int q = 0; q < TMR; q++) {
+        for (int q = 0; q < MR; q++) {
             const int sid = q * TPT + tid;
             const bool ok = sid < total;
             const int r = ok ? coherent_load(&slots.cand_r[sid]) : INT_MAX;
@@ -261,7 +312,7 @@ __global__ __launch_bounds__(TPT) void panel_tslu_kernel(
 #pragma unroll
             for (int c = 0; c < TW; c++) v[q][c] = coherent_load(&slots.cand_v[(size_t)c * TCAND + sv]);
         }
-        wg_gepp<T, TMR, FULL>(v, key, pid, wa, s_k2, s_p2, s_gl, s_lu);
+        wg_gepp<T, MR, FULL>(v, key, pid, wa, s_k2, s_p2, s_gl, s_lu);
     }
     if (wave == 0 && lane < wa) {
         // L11: lane r solves its pivot row's original values against U11
@@ -401,16 +452,19 @@ unsigned panel_tslu(T *A, int lda, int m, int wa, int lcols, int rcols, int row0
         G = ceil_div(m, TPT * rpt);
     }
     const unsigned target = base + (unsigned)G;
-#define SLA_TSLU(RV, FV)                                                                      \
-    hipLaunchKernelGGL((panel_tslu_kernel<T, RV, FV>), dim3(G), dim3(TPT), 0, s, A, lda, m, wa, \
+    const bool one = G * TW <= TPT;  // a candidate a thread
+#define SLA_TSLU(RV, MV, FV)                                                                  \
+    hipLaunchKernelGGL((panel_tslu_kernel<T, RV, MV, FV>), dim3(G), dim3(TPT), 0, s, A, lda, m, wa, \
                        lcols, rcols, row0, col0, ipiv, slots, pw.ctr, target, pw.abort_flag,   \
                        pw.zero_col, pw.spin_limit)
     if (wa == TW) {
-        if (rpt == 1) SLA_TSLU(1, true);
-        else SLA_TSLU(2, true);
+        if (rpt == 2) SLA_TSLU(2, 2, true);
+        else if (one) SLA_TSLU(1, 1, true);
+        else SLA_TSLU(1, 2, true);
     } else {
-        if (rpt == 1) SLA_TSLU(1, false);
-        else SLA_TSLU(2, false);
+        if (rpt == 2) SLA_TSLU(2, 2, false);
+        else if (one) SLA_TSLU(1, 1, false);
+        else SLA_TSLU(1, 2, false);
     }
 #undef SLA_TSLU
     SLA_LAUNCH_CHECK();
