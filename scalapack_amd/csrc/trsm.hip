@@ -228,12 +228,13 @@ __device__ __forceinline__ T row_lane(T v)
     }
 }
 
-// Steps of a 16 x 16 triangle: lane l holds row l of b[0] and a row each of what
-// the solved values are to be subtracted from, b[1] .. b[3]; e[q][k (TV_BS + 1)]
-// is column k of the triangle and of those rows, rd the reciprocals of a non-unit
-// diagonal.  Lane l's solved value goes to x.  (Lanes already solved go on
-// subtracting; only x counts.)  The chain of a step is a product, a DPP move and
-// an fma; the other rows' are off it.
+// Steps of a 16 x 16 triangle: lane l holds row l of b[0], and in b[1] .. b[3] what
+// the solved values take from a row each of the triangles after it (summed apart:
+// one rounding of their size a triangle, not sixteen); e[q][k (TV_BS + 1)] is
+// column k of those rows, rd the reciprocals of a non-unit diagonal.  Lane l's
+// solved value goes to x.  (Lanes already solved go on subtracting; only x counts.)
+// The chain of a step is a product, a DPP move and an fma; the other rows' are off
+// it.
 template <int S, bool FORWARD, bool UNIT, typename T>
 __device__ __forceinline__ void tv_steps(T (&b)[4], T &x, const T *const (&e)[4], const T *rd, int l)
 {
@@ -401,18 +402,18 @@ __global__ __launch_bounds__(256) void trsv_persistent_kernel(
     const int j = 4 * wave + lk;
     if (4 * wave < nrhs) {
         const T *y = Ys[MF ? j : 0];
-        T bb[4];  // bb[0]: the rows of the current triangle, then those after it
+        T yy[4];  // the rows of the current triangle, then those after it
 #pragma unroll
-        for (int i = 0; i < 4; i++) bb[i] = y[16 * (FORWARD ? i : 3 - i) + lr];
+        for (int i = 0; i < 4; i++) yy[i] = y[16 * (FORWARD ? i : 3 - i) + lr];
         const uint64_t tag = (uint64_t)epoch << 32;
 #pragma unroll 1
         for (int i = 0; i < 4; i++) {
             const int r0 = 16 * (FORWARD ? i : 3 - i);
-            const T *e[4];  // rows r0, and those of bb[1] .. bb[3] (a row of the block if none)
+            const T *e[4];  // rows r0, and those of yy[1] .. yy[3] (a row of the block if none)
 #pragma unroll
             for (int q = 0; q < 4; q++)
                 e[q] = &Es[r0][(FORWARD ? min(r0 + 16 * q, TV_BS - 16) : max(r0 - 16 * q, 0)) + lr];
-            T x = T(0);
+            T x = T(0), bb[4] = {yy[0], T(0), T(0), T(0)};
             tv_steps<0, FORWARD, UNIT>(bb, x, e, rd + r0, lr);
             if (j < nrhs && r0 + lr < rows) {
 #pragma unroll
@@ -421,9 +422,7 @@ __global__ __launch_bounds__(256) void trsv_persistent_kernel(
                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 X[(size_t)(rb + r0 + lr) + (size_t)j * ldx] = x;
             }
-            bb[0] = bb[1];
-            bb[1] = bb[2];
-            bb[2] = bb[3];
+            yy[0] = yy[1] + bb[1], yy[1] = yy[2] + bb[2], yy[2] = yy[3] + bb[3];
         }
     }
 }
