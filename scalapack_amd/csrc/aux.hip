@@ -79,26 +79,43 @@ __global__ __launch_bounds__(256) void lange_max_kernel(int m, int n, const doub
     if ((threadIdx.x & 63) == 0) atomic_max_nonneg(out, v);
 }
 
-// Column sums of |A| in the reference's order: one wave per 64 columns; each
-// 64 x 64 tile is read down its columns (coalesced) into LDS, then lane c adds
-// the tile's rows of column c one after another.
-__global__ __launch_bounds__(64) void lange_colsum_kernel(int m, int n, const double *__restrict__ A,
-                                                          int lda, double *__restrict__ colsum)
+// Column sums of |A| in the reference's order: 16 columns a workgroup, tiles of 256
+// rows read down their columns (coalesced) into LDS, then lane c adds the tile's
+// rows of column c one after another while the next tile is on its way.  Bound by
+// the chain of m additions.  One wave per 64 columns, which read and added in turn,
+// took 562 us at 2003 x 2003; PDGESVX there went from 11.42 to 10.89 ms.
+constexpr int CS_C = 16, CS_R = 256;
+__global__ __launch_bounds__(CS_R) void lange_colsum_kernel(int m, int n, const double *__restrict__ A,
+                                                            int lda, double *__restrict__ colsum)
 {
-    __shared__ double T[64][65];
-    const int lane = threadIdx.x, c0 = blockIdx.x * 64;
-    const int cols = min(64, n - c0);
+    __shared__ alignas(16) double T[CS_C][CS_R + 2];
+    typedef double d2_t __attribute__((ext_vector_type(2)));
+    const int tid = threadIdx.x, c0 = blockIdx.x * CS_C;
+    double v[CS_C];
+    auto load = [&](int r0) {
+#pragma unroll
+        for (int c = 0; c < CS_C; c++)
+            v[c] = r0 + tid < m ? A[(size_t)(r0 + tid) + (size_t)min(c0 + c, n - 1) * lda] : 0.0;
+    };
+    load(0);
     double sum = 0.0;
-    for (int r0 = 0; r0 < m; r0 += 64) {
-        const int rows = min(64, m - r0);
-        for (int c = 0; c < cols; c++)
-            T[c][lane] = lane < rows ? fabs(A[(size_t)(r0 + lane) + (size_t)(c0 + c) * lda]) : 0.0;
+    for (int r0 = 0; r0 < m; r0 += CS_R) {
+#pragma unroll
+        for (int c = 0; c < CS_C; c++) T[c][tid] = fabs(v[c]);
         __syncthreads();
-        if (lane < cols)
-            for (int k = 0; k < rows; k++) sum += T[lane][k];
+        load(r0 + CS_R);
+        if (tid < CS_C) {  // rows from m on are zeros, which change no sum
+            const d2_t *t = reinterpret_cast<const d2_t *>(T[tid]);
+#pragma unroll 16
+            for (int k = 0; k < CS_R / 2; k++) {
+                const d2_t x = t[k];
+                sum += x[0];
+                sum += x[1];
+            }
+        }
         __syncthreads();
     }
-    if (lane < cols) colsum[c0 + lane] = sum;
+    if (tid < CS_C && c0 + tid < n) colsum[c0 + tid] = sum;
 }
 
 // Row sums of |A| in the reference's order: thread i adds row i from column 0
@@ -790,7 +807,7 @@ double dlange_device(Handle &h, char norm, int m, int n, const double *dA, int l
     }
     if (c == 'O' || c == '1') {
         AuxWork a(h, n, 0);
-        hipLaunchKernelGGL(lange_colsum_kernel, dim3(ceil_div(n, 64)), dim3(64), 0, h.stream, m, n, dA,
+        hipLaunchKernelGGL(lange_colsum_kernel, dim3(ceil_div(n, CS_C)), dim3(CS_R), 0, h.stream, m, n, dA,
                            lda, a.x);
         SLA_LAUNCH_CHECK();
         a.maxabs(a.x, n, 0);
