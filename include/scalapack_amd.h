@@ -134,7 +134,10 @@ int sla_destroy(sla_handle_t h);
  * Calls return after the stream has drained. */
 int sla_set_stream(sla_handle_t h, void *stream);
 /* Tuning knobs: "nb" (block column width, 1..512), "leaf_w" (panel leaf width,
- * <= 32), "panel_wgs" (workgroups per panel leaf, 1..128), "profile" (0/1); for the
+ * <= 32), "panel_wgs" (workgroups per panel leaf, 1..128), "panel_patience" (us,
+ * 0..1000000, default 200: a panel leaf of more than 8192 rows on one die of the
+ * GPU waits that long for all its workgroups to run, then gives way to what keeps
+ * them out and runs spread over the dies; same factors), "profile" (0/1); for the
  * mixed-precision solve "ir_max_iter" (3..1000, default 30), "ir_gmres_on_stall"
  * (0/1, default 1), "ir_accept_stall" (0/1, default 1: a refinement that
  * stalls with scaled residual < 16 returns its X; 0: only DSGESV's

@@ -1068,7 +1068,7 @@ int sla_set_param(sla_handle_t h, const char *name, int value)
                                   "pivoting", "lookahead", "update_cus", "lacon_lapack",
                                   "batched_w", "batched_wgs_per_cu", "batched_graph",
                                   "update_lds_kb", "ir_accept_stall", "trsv_blockinv",
-                                  "ir_fallback", "trsm_mfma"};
+                                  "ir_fallback", "trsm_mfma", "panel_patience"};
     if (std::find_if(std::begin(known), std::end(known), [&](const char *x) { return k == x; }) ==
         std::end(known)) {
         g_last_error = "sla_set_param: unknown parameter " + k;
@@ -1080,6 +1080,7 @@ int sla_set_param(sla_handle_t h, const char *name, int value)
     if (k == "nb" && value >= 1 && value <= 512) H->nb = value;
     else if (k == "leaf_w" && value >= 1 && value <= 32) H->leaf_w = value;
     else if (k == "panel_wgs" && value >= 1 && value <= 128) H->panel_wgs = value;
+    else if (k == "panel_patience" && value >= 0 && value <= 1000000) H->panel_patience = value;
     else if (k == "profile") H->profile = value != 0;
     else if (k == "ir_max_iter" && value >= 3 && value <= 1000) H->ir_max_iter = value;
     else if (k == "gmres_m" && value >= 1 && value <= 1000) H->gmres_m = value;
@@ -1112,6 +1113,7 @@ int sla_get_param(sla_handle_t h, const char *name, int *value)
     if (k == "nb") *value = H->nb;
     else if (k == "leaf_w") *value = H->leaf_w;
     else if (k == "panel_wgs") *value = H->panel_wgs;
+    else if (k == "panel_patience") *value = H->panel_patience;
     else if (k == "profile") *value = H->profile ? 1 : 0;
     else if (k == "ir_max_iter") *value = H->ir_max_iter;
     else if (k == "gmres_m") *value = H->gmres_m;

@@ -110,6 +110,8 @@ PanelWork<T> Handle::panel_work()
     pw.abort_flag = abort_flag;
     pw.zero_col = zero_col;
     pw.spin_limit = spin_limit;
+    pw.yield = reinterpret_cast<unsigned *>(ctl + 6);
+    pw.patience = (uint64_t)(panel_patience * (wall_khz / 1000.0));
     pw.target_wgs = panel_wgs;
     pw.num_cus = num_cus;
     return pw;

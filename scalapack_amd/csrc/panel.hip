@@ -40,7 +40,11 @@
 // path 440 ns within an XCD and 500 - 620 ns between two (ping-pong of two
 // workgroups).  So a leaf of at most 32 workgroups puts them all on one XCD, a
 // different one from leaf to leaf, because the trailing update beside it is
-// dealt evenly over all of them.  The pivot row is fetched once the pivot is
+// dealt evenly over all of them.  Where that takes more than a quarter of the XCD,
+// leaves of several handles could keep each other from getting all their
+// workgroups to run; there the leaf gives way after 200 us in column 0 and a second
+// launch, over all XCDs, does the work (sla_panel_plan.h).  That launch costs a
+// leaf that did not give way 6 us.  The pivot row is fetched once the pivot is
 // known: gathering all G candidate rows in one trip, to LDS, took 85 us at m =
 // 2000 where this takes 77, and 57 KB of LDS where this takes 13.
 //
@@ -51,8 +55,8 @@
 //
 // Measured on 32 FP64 columns, alone on the GPU, us per leaf, before (all
 // columns unrolled, rows interchanged in registers, the workgroups spread over
-// the XCDs) and now: m = 100: 125, 36; 1000: 136, 79; 4000: 149, 80; 8192: 158,
-// 81; 16384: 165, 101; 32768: 183, 126.
+// the XCDs) and now: m = 100: 120, 36; 1000: 130, 73; 4096: 149, 79; 8192: 157,
+// 82; 16384: 165, 108; 32768: 182, 132.
 //
 // Mailbox: two regions of 32 column blocks; launch L uses region L & 1 and
 // refills the words launch L - 1 wrote in region (L + 1) & 1 -- that launch
@@ -60,6 +64,7 @@
 // region empty.
 #include "sla_common.h"
 #include "sla_kernels.h"
+#include "sla_panel_plan.h"
 
 #include <algorithm>
 #include <climits>
@@ -69,8 +74,6 @@ namespace sla {
 namespace {
 
 constexpr int NWV = 8;           // waves per workgroup at most
-constexpr int LEAF_GMAX = 128;   // workgroups per leaf launch at most
-constexpr int XCDS = 8, XCD_CUS = 32;  // the dies of the GPU and the CUs of one
 static_assert(LEAF_GMAX <= PANEL_MAIL_GMAX, "mailbox too small for the leaf's grid");
 
 constexpr uint64_t MAIL_EMPTY = ~0ull;  // no position or value word has this pattern
@@ -203,6 +206,10 @@ struct LeafArgs {
     uint64_t *box;  // this launch's mailbox region
     int *abort_flag;
     uint64_t spin_limit, t0;
+    unsigned *yield;    // where the leaf says that it gives way (null: it does not)
+    unsigned yield_id;  // by this number
+    uint64_t patience;  // ticks it waits in column 0 before it does
+    unsigned look;      // a wait looks at flags and clock when its count has none of these bits
     int G, g;       // workgroups of the leaf, this one
     uint32_t xcd;   // the die it runs on
 };
@@ -233,13 +240,22 @@ __device__ __forceinline__ void publish(const LeafArgs &ar, uint64_t *cb, bool l
     }
 }
 
-// Whether a wait goes on: false after spin_limit or when another wait gave up.
-__device__ __forceinline__ bool keep_waiting(const LeafArgs &ar, unsigned &it, int *s_abort)
+// Whether a wait of column j goes on: false after spin_limit, when another wait gave
+// up, or when the leaf gives way.  A leaf gives way only in column 0: a workgroup
+// that leaves there posts nothing more, so no other one gets past column 1, and
+// since nothing but the mailbox is written before the last column, all leave the
+// matrix as it was.  Once column 0 is through, every workgroup runs.
+__device__ __forceinline__ bool keep_waiting(const LeafArgs &ar, int j, unsigned &it, int *s_abort)
 {
-    if ((++it & 15u) != 0) return true;
+    if ((++it & ar.look) != 0) return true;
     bool on = true;
+    const uint64_t dt = wall_clock64() - ar.t0;
     if (coherent_load(ar.abort_flag)) on = false;
-    else if (wall_clock64() - ar.t0 > ar.spin_limit) {
+    else if (ar.yield && coherent_load(ar.yield) == ar.yield_id) on = false;
+    else if (ar.yield && j == 0 && dt > ar.patience) {
+        coherent_store(ar.yield, ar.yield_id);
+        on = false;
+    } else if (dt > ar.spin_limit) {
         coherent_store(ar.abort_flag, 1);
         on = false;
     }
@@ -345,8 +361,12 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
     }
     if (!found && lane == 0) sl.wpos[pb][wave] = INT_MAX;
     __syncthreads();
-    // a wait of the column before that gave up: all waves see it here
-    if (!SOLO) dead = sl.s_abort[pb ^ 1] != 0;
+    // a wait of the column before that gave up: all waves see it here, before the
+    // workgroup posts anything of this column
+    if constexpr (!SOLO) {
+        dead = sl.s_abort[pb ^ 1] != 0;
+        if (dead) return;
+    }
     // the workgroup's: lane x looks at the candidate of wave x % 8
     int p, fw;
     bool nonzero = true;
@@ -395,7 +415,7 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
             }
         } while ((kv[0] == MAIL_EMPTY || kp[0] == MAIL_EMPTY || kv[1] == MAIL_EMPTY ||
                   kp[1] == MAIL_EMPTY) &&
-                 keep_waiting(ar, it, &sl.s_abort[pb]));
+                 keep_waiting(ar, j, it, &sl.s_abort[pb]));
         int xp = lane < G ? (int)kp[0] : INT_MAX;
         T xv = mail_value<T>(kv[0]);
         const uint32_t h = xp != INT_MAX ? mag_hi(xv) : 0u;
@@ -435,7 +455,7 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
         // through the wave's own slot in LDS
         const uint64_t *rw = cb + (size_t)gw * PANEL_MAIL_CW + lane % (4 * NC);
         uint64_t w;
-        while ((w = coherent_load(rw)) == MAIL_EMPTY && keep_waiting(ar, it, &sl.s_abort[pb])) {
+        while ((w = coherent_load(rw)) == MAIL_EMPTY && keep_waiting(ar, j, it, &sl.s_abort[pb])) {
         }
         if (lane < 4 * NC) sl.prow[wave][lane] = mail_value<T>(w);
         prow = sl.prow[wave];
@@ -482,11 +502,14 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
 // stride: the leaf's workgroups are every stride-th of the launch (the others
 // leave at once): with 8, the number of XCDs over which consecutive workgroups
 // are dealt, they share one XCD and its L2 (checked in column 0).
+// yield_id: number by which the leaf gives way in *yield (0: it does not);
+// after_id: the leaf runs only if the launch of that number did (0: always).
 template <typename T, int NC, int NQ, bool SOLO, int PT, int WPE>
 __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(WPE))) void panel_leaf_kernel(
     T *__restrict__ A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0,
     int *__restrict__ ipiv, uint64_t *__restrict__ mail, int region, int prev_wa, int prev_g,
-    int *abort_flag, int *zero_col, uint64_t spin_limit, int stride, int first)
+    int *abort_flag, int *zero_col, uint64_t spin_limit, int stride, int first, unsigned *yield,
+    unsigned yield_id, unsigned after_id, uint64_t patience)
 {
     if (!SOLO && (int)blockIdx.x % stride != first) return;
     const int G = SOLO ? 1 : gridDim.x / stride, g = SOLO ? 0 : blockIdx.x / stride;
@@ -511,6 +534,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
                                        ? PANEL_MAIL_VAL + e - prev_g * PANEL_MAIL_CW
                                        : PANEL_MAIL_POS + e - prev_g * (PANEL_MAIL_CW + 1))],
                                MAIL_EMPTY);
+        if (after_id != 0 && coherent_load(yield) != after_id) return;
     }
 
     // column 4 i + cg of the leaf in register i; columns right of a narrow
@@ -527,7 +551,9 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
             a[q][i] = (r < m && c < wa) ? A[r + (size_t)c * lda] : T(0);
         }
     }
-    const LeafArgs ar{mail + (size_t)region * PANEL_MAIL_REGION, abort_flag, spin_limit, (uint64_t)wall_clock64(), G, g,
+    const LeafArgs ar{mail + (size_t)region * PANEL_MAIL_REGION, abort_flag, spin_limit, (uint64_t)wall_clock64(),
+                      yield_id != 0 ? yield : nullptr, yield_id, patience,
+                      yield_id != 0 && patience == 0 ? 0u : 15u, G, g,
                       SOLO ? 0u : (uint32_t)__builtin_amdgcn_s_getreg(63508) & 0xffffu};  // XCC_ID
     bool local = false;
     __syncthreads();
@@ -622,7 +648,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
 
 template <typename T, int NC, int NQ, bool SOLO, int PT, int WPE>
 void launch_leaf(T *A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0, int *ipiv,
-                 const PanelWork<T> &pw, int threads, int G, hipStream_t s)
+                 const PanelWork<T> &pw, int threads, int G, LeafPlace place, hipStream_t s)
 {
     PanelMailState &ms = *pw.mail_state;
     if (threads > PT) throw std::logic_error("panel leaf: workgroup larger than its kernel's");
@@ -630,52 +656,48 @@ void launch_leaf(T *A, int lda, int m, int wa, int lcols, int rcols, int row0, i
         // the mailbox and its record stay as the last exchanging launch left them
         hipLaunchKernelGGL((panel_leaf_kernel<T, NC, NQ, true, PT, WPE>), dim3(1), dim3(threads), 0,
                            s, A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw.mail, 0, 0, 0,
-                           pw.abort_flag, pw.zero_col, pw.spin_limit, 1, 0);
+                           pw.abort_flag, pw.zero_col, pw.spin_limit, 1, 0, pw.yield, 0u, 0u,
+                           (uint64_t)0);
         SLA_LAUNCH_CHECK();
     } else {
-        // One XCD for all only on the whole GPU, and if each of its CUs takes one at
-        // most: beside a trailing update a CU has room for one.
-        const int stride = G <= XCD_CUS && pw.num_cus == XCDS * XCD_CUS ? XCDS : 1;
-        const int first = stride == 1 ? 0 : (int)(ms.launches % XCDS);
-        hipLaunchKernelGGL((panel_leaf_kernel<T, NC, NQ, false, PT, WPE>), dim3(G * stride),
-                           dim3(threads), 0, s, A, lda, m, wa, lcols, rcols, row0, col0, ipiv,
-                           pw.mail, (int)(ms.launches & 1u), ms.prev_wa, ms.prev_g, pw.abort_flag,
-                           pw.zero_col, pw.spin_limit, stride, first);
-        SLA_LAUNCH_CHECK();
-        ms.launches++;
-        ms.prev_wa = wa;
-        ms.prev_g = G;
+        auto go = [&](int stride, unsigned yield_id, unsigned after_id) {
+            const int first = stride == 1 ? 0 : (int)(ms.launches % XCDS);
+            hipLaunchKernelGGL((panel_leaf_kernel<T, NC, NQ, false, PT, WPE>), dim3(G * stride),
+                               dim3(threads), 0, s, A, lda, m, wa, lcols, rcols, row0, col0, ipiv,
+                               pw.mail, (int)(ms.launches & 1u), ms.prev_wa, ms.prev_g,
+                               pw.abort_flag, pw.zero_col, pw.spin_limit, stride, first, pw.yield,
+                               yield_id, after_id, pw.patience);
+            SLA_LAUNCH_CHECK();
+            ms.launches++;
+            ms.prev_wa = wa;
+            ms.prev_g = G;
+        };
+        const unsigned id = std::max(1u, ms.launches + 1);
+        if (place == LEAF_ONE_XCD_YIELDS && wa < 2)
+            throw std::logic_error("panel leaf: a leaf of one column cannot give way");
+        go(place == LEAF_SPREAD ? 1 : XCDS, place == LEAF_ONE_XCD_YIELDS ? id : 0u, 0u);
+        if (place == LEAF_ONE_XCD_YIELDS) go(1, 0u, id);
     }
 }
 
-// Rows per quad (V / NC) for V values a thread.
+// NC: registers per row and lane.
 template <typename T, int NC>
 void leaf_of_width(T *A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0,
                    int *ipiv, const PanelWork<T> &pw, hipStream_t s)
 {
-    // V values a thread: 32 take at most 128 registers, 64 up to 256.
-    constexpr int V = NC == 2 ? 16 : 32;
-    auto grid = [&](int v, int waves) { return ceil_div(m, 16 * (v / NC) * waves); };
-#define SLA_LEAF(V, SOLO, PTV, WPE, threads, G)                                                     \
-    launch_leaf<T, NC, (V) / NC, SOLO, PTV, WPE>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, \
-                                                 threads, G, s)
-    // One workgroup while it holds the leaf: 78 us at m = 1000 and without the
-    // other streams' kernels in the way of an exchange.  (16 waves of 32 values
-    // instead of 8 of 64: 80 us; a SIMD's four waves wait for each other.)
-    if (grid(V, 8) == 1) return SLA_LEAF(V, true, 512, 4, 64 * grid(V, 1), 1);
-    if (grid(64, 8) == 1) return SLA_LEAF(64, true, 512, 2, 64 * grid(64, 1), 1);
-    // Then as many as one XCD runs, of the smallest kind: 82 us at m = 8192 with
-    // four waves.  Beside a long trailing update only those find room, so there
-    // they go on, across the XCDs: m = 16384 alone 139 us, with eight waves 95 us,
-    // but these wait for the end of the update.  The caller's preferred grid
-    // counts the largest kind.
-    const int target = std::min(pw.target_wgs, XCD_CUS);
-    if (grid(V, 4) <= (pw.beside ? std::min(4 * pw.target_wgs, LEAF_GMAX) : target))
-        return SLA_LEAF(V, false, 256, 4, 256, grid(V, 4));
-    if (grid(V, 8) <= target) return SLA_LEAF(V, false, 512, 4, 512, grid(V, 8));
-    if (grid(64, 8) > LEAF_GMAX)
+    const LeafPlan p = leaf_plan(m, wa, pw.target_wgs, pw.beside, pw.num_cus == XCDS * XCD_CUS);
+    constexpr int V = leaf_values(NC);
+    if (p.wgs > LEAF_GMAX)
         throw std::runtime_error("panel leaf: panel too tall for the leaf's workgroup limit");
-    SLA_LEAF(64, false, 512, 2, 512, grid(64, 8));
+#define SLA_LEAF(V, SOLO, PTV, WPE)                                                                 \
+    launch_leaf<T, NC, (V) / NC, SOLO, PTV, WPE>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, \
+                                                 64 * p.waves, p.wgs, p.place, s)
+    if (p.wgs == 1) {
+        if (p.values == V) SLA_LEAF(V, true, 512, 4);
+        else SLA_LEAF(64, true, 512, 2);
+    } else if (p.values != V) SLA_LEAF(64, false, 512, 2);
+    else if (p.waves == 4) SLA_LEAF(V, false, 256, 4);
+    else SLA_LEAF(V, false, 512, 4);
 #undef SLA_LEAF
 }
 
@@ -685,15 +707,12 @@ template <typename T>
 unsigned panel_leaf(T *A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0,
                     int *ipiv, const PanelWork<T> &pw, hipStream_t s)
 {
-    // registers per row and lane by the leaf's width
-    if (wa <= 8)
-        leaf_of_width<T, 2>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, s);
-    else if (wa <= 16)
-        leaf_of_width<T, 4>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, s);
-    else if (wa <= 32)
-        leaf_of_width<T, 8>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, s);
-    else
-        throw std::runtime_error("panel leaf: width above 32");
+    if (wa > 32) throw std::runtime_error("panel leaf: width above 32");
+    switch (leaf_nc(wa)) {
+    case 2: leaf_of_width<T, 2>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, s); break;
+    case 4: leaf_of_width<T, 4>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, s); break;
+    default: leaf_of_width<T, 8>(A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw, s);
+    }
     return 0;  // the mailbox exchange adds no barrier arrivals
 }
 

@@ -135,7 +135,7 @@ struct Handle {
 
     // device control block: [0] barrier counter, [1] abort flag,
     // [2] first zero-pivot column (INT_MAX: none), [3] ticket, [4] pair count,
-    // [5] pivot-row-out-of-range flag
+    // [5] pivot-row-out-of-range flag, [6] last panel leaf that gave way
     int *ctl = nullptr;
     unsigned *ctr = nullptr;
     int *abort_flag = nullptr, *zero_col = nullptr, *ticket = nullptr, *pair_count = nullptr;
@@ -171,6 +171,8 @@ struct Handle {
     int nb = 256;          // block column width of the outer factorization
     int leaf_w = 32;       // panel leaf width (columns per device-wide-barrier kernel)
     int panel_wgs = 32;    // preferred workgroups per leaf launch
+    int panel_patience = 200;  // us a leaf that takes most of an XCD waits for its
+                               // workgroups to run before it gives way
     int pivoting = 1;      // FP32-storage factorization: 0 partial, 1 tournament
     int lookahead = 1;     // factor block column p+1 on a second stream during p's update
     int update_cus = 0;    // > 0: the trailing update runs on at most this many CUs' worth

@@ -100,6 +100,8 @@ struct PanelWork {
     int *abort_flag;     // set by a wait that lasted past spin_limit
     int *zero_col;       // min over zero pivots of the 1-based column (INT_MAX: none)
     uint64_t spin_limit; // wall-clock ticks a barrier may wait
+    unsigned *yield;     // number of the last leaf launch that gave way to other kernels
+    uint64_t patience;   // ticks such a launch waits for all its workgroups to run
     int target_wgs;      // preferred number of workgroups per leaf launch
     int num_cus;         // CUs of the device
     bool beside = false; // a long trailing update runs on another stream meanwhile

@@ -1,0 +1,66 @@
+// sla_panel_plan.h -- how a panel leaf (panel.hip) of m rows and wa columns is cut
+// into workgroups, and where they run.  Host code only.
+#pragma once
+
+#include <algorithm>
+
+namespace sla {
+
+constexpr int LEAF_GMAX = 128;         // workgroups per leaf launch at most
+constexpr int XCDS = 8, XCD_CUS = 32;  // the dies of the GPU and the CUs of one
+
+// Where the workgroups go: dealt over all XCDs, all on one, or all on one with a
+// second launch, dealt over all, that does the work if the first gave way.
+enum LeafPlace { LEAF_SPREAD, LEAF_ONE_XCD, LEAF_ONE_XCD_YIELDS };
+
+struct LeafPlan {
+    int values;  // matrix elements a thread holds: 16 or 32 take at most 128 registers, 64 up to 256
+    int waves;   // of a workgroup
+    int wgs;     // workgroups (above LEAF_GMAX: the leaf is too tall)
+    LeafPlace place;
+};
+
+// Registers per row and lane by the leaf's width (a row lies in four lanes).
+constexpr int leaf_nc(int wa) { return wa <= 8 ? 2 : wa <= 16 ? 4 : 8; }
+// Elements a thread holds in the smaller kinds.
+constexpr int leaf_values(int nc) { return nc == 2 ? 16 : 32; }
+// Quarters of a CU that a workgroup's registers take.
+constexpr int leaf_quarters(const LeafPlan &p) { return (p.values == 64 ? 2 : 1) * (p.waves > 4 ? 2 : 1); }
+
+// panel_wgs: the caller's preferred grid, counted in the largest kind.  beside: a
+// long trailing update runs on another stream meanwhile.  xcds: the GPU has all
+// its XCDs' CUs.
+inline LeafPlan leaf_plan(int m, int wa, int panel_wgs, bool beside, bool xcds)
+{
+    const int nc = leaf_nc(wa), v = leaf_values(nc);
+    auto grid = [&](int values, int waves) {
+        const int rows = 16 * (values / nc) * waves;
+        return (m + rows - 1) / rows;
+    };
+    const int g1 = grid(v, 4), g2 = grid(v, 8), g3 = grid(64, 8);
+    // One workgroup while it holds the leaf: 78 us at m = 1000 and without the
+    // other streams' kernels in the way of an exchange.  (16 waves of 32 values
+    // instead of 8 of 64: 80 us; a SIMD's four waves wait for each other.)
+    if (g2 == 1) return {v, grid(v, 1), 1, LEAF_SPREAD};
+    if (g3 == 1) return {64, grid(64, 1), 1, LEAF_SPREAD};
+    // Then as many as one XCD runs, of the smallest kind: 82 us at m = 8192 with
+    // four waves.  Beside a long trailing update only those find room, so there
+    // they go on, across the XCDs: m = 16384 alone 139 us, with eight waves 95 us,
+    // but these wait for the end of the update.
+    //
+    // Workgroups that wait for one another have to run together, whatever else runs.
+    // The smallest kind takes a quarter of a CU, so an XCD holds four leaves of it
+    // at once: as many as HIP's four hardware queues run of a process's handles.
+    // The larger kinds take half a CU and a whole one.  On one XCD two leaves
+    // of theirs could keep each other out, each with a part of its workgroups
+    // running, so these give way (keep_waiting in panel.hip): a launch over all
+    // XCDs, where eight of them find room, follows and does the work instead.
+    const int target = std::min(panel_wgs, XCD_CUS);
+    const LeafPlace tall = xcds && wa > 1 ? LEAF_ONE_XCD_YIELDS : LEAF_SPREAD;
+    if (g1 <= (beside ? std::min(4 * panel_wgs, LEAF_GMAX) : target))
+        return {v, 4, g1, xcds && g1 <= XCD_CUS ? LEAF_ONE_XCD : LEAF_SPREAD};
+    if (g2 <= target) return {v, 8, g2, tall};
+    return {64, 8, g3, g3 <= XCD_CUS ? tall : LEAF_SPREAD};
+}
+
+}  // namespace sla
