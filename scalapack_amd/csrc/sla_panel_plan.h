@@ -42,11 +42,15 @@ inline LeafPlan leaf_plan(int m, int wa, int panel_wgs, bool beside, bool xcds)
     // other streams' kernels in the way of an exchange.  (16 waves of 32 values
     // instead of 8 of 64: 80 us; a SIMD's four waves wait for each other.)
     if (g2 == 1) return {v, grid(v, 1), 1, LEAF_SPREAD};
-    if (g3 == 1) return {64, grid(64, 1), 1, LEAF_SPREAD};
+    if (nc == 8 && g3 == 1) return {64, grid(64, 1), 1, LEAF_SPREAD};
     // Then as many as one XCD runs, of the smallest kind: 82 us at m = 8192 with
     // four waves.  Beside a long trailing update only those find room, so there
     // they go on, across the XCDs: m = 16384 alone 139 us, with eight waves 95 us,
-    // but these wait for the end of the update.
+    // but these wait for the end of the update.  Leaves of at most 16 columns go on
+    // there always: their steps are short, 64 values of so few columns are many rows
+    // a quad, and those come one after another (8 columns, m = 2000: one workgroup
+    // 55 us, eight 25; m = 50000: 13 workgroups 117 us, 98 of the smallest kind 45; 16
+    // columns: 66, 48; 100, 83).
     //
     // Workgroups that wait for one another have to run together, whatever else runs.
     // The smallest kind takes a quarter of a CU, so an XCD holds four leaves of it
@@ -57,10 +61,14 @@ inline LeafPlan leaf_plan(int m, int wa, int panel_wgs, bool beside, bool xcds)
     // XCDs, where eight of them find room, follows and does the work instead.
     const int target = std::min(panel_wgs, XCD_CUS);
     const LeafPlace tall = xcds && wa > 1 ? LEAF_ONE_XCD_YIELDS : LEAF_SPREAD;
-    if (g1 <= (beside ? std::min(4 * panel_wgs, LEAF_GMAX) : target))
+    if (g1 <= (beside || nc < 8 ? std::min(4 * panel_wgs, LEAF_GMAX) : target))
         return {v, 4, g1, xcds && g1 <= XCD_CUS ? LEAF_ONE_XCD : LEAF_SPREAD};
-    if (g2 <= target) return {v, 8, g2, tall};
-    return {64, 8, g3, g3 <= XCD_CUS ? tall : LEAF_SPREAD};
+    if (nc == 8 && g2 <= target) return {v, 8, g2, tall};
+    if (nc == 8 && g3 <= target) return {64, 8, g3, tall};
+    // Over the XCDs the middle kind is the faster one (32 columns, m = 65536: 174 us
+    // against 179 with half as many of the largest kind; 16 columns, 131072: 99, 115)
+    if (g2 <= LEAF_GMAX) return {v, 8, g2, LEAF_SPREAD};
+    return {64, 8, g3, LEAF_SPREAD};
 }
 
 }  // namespace sla

@@ -78,3 +78,10 @@ def test_waiting_workgroups_find_room(plans):
             leaves = 8 if p["wgs"] <= 32 else 2
             per_xcd = -(-p["wgs"] // XCDS)
             assert leaves * per_xcd * p["quarters"] <= 4 * XCD_CUS, p
+
+
+def test_narrow_leaves_hold_few_rows_a_quad(plans):
+    """At most 16 columns: 64 values a thread only where nothing else holds the rows."""
+    for p in plans:
+        if p["nc"] < 8 and p["m"] <= GMAX * 16 * ((16 if p["nc"] == 2 else 32) // p["nc"]) * 8:
+            assert p["values"] < 64, p
