@@ -134,8 +134,9 @@ int sla_destroy(sla_handle_t h);
  * Calls return after the stream has drained. */
 int sla_set_stream(sla_handle_t h, void *stream);
 /* Tuning knobs: "nb" (block column width, 1..512), "leaf_w" (panel leaf width,
- * <= 32), "panel_wgs" (workgroups per panel leaf, 1..128), "panel_patience" (us,
- * 0..1000000, default 200: a panel leaf of more than 8192 rows on one die of the
+ * <= 32), "panel_wgs" (1..128, default 32: workgroups per panel leaf at most, as
+ * far as its height allows; above 32 they run over all dies of the GPU),
+ * "panel_patience" (us, 0..1000000, default 200: a panel leaf of more than 8192 rows on one die of the
  * GPU waits that long for all its workgroups to run, then gives way to what keeps
  * them out and runs spread over the dies; same factors), "profile" (0/1); for the
  * mixed-precision solve "ir_max_iter" (3..1000, default 30), "ir_gmres_on_stall"

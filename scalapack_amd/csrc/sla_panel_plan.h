@@ -27,8 +27,8 @@ constexpr int leaf_values(int nc) { return nc == 2 ? 16 : 32; }
 // Quarters of a CU that a workgroup's registers take.
 constexpr int leaf_quarters(const LeafPlan &p) { return (p.values == 64 ? 2 : 1) * (p.waves > 4 ? 2 : 1); }
 
-// panel_wgs: the caller's preferred grid, counted in the largest kind.  beside: a
-// long trailing update runs on another stream meanwhile.  xcds: the GPU has all
+// panel_wgs: the workgroups that the caller prefers at most; four times as many of
+// the smallest kind beside an update and for narrow leaves.  beside: a long trailing update runs on another stream meanwhile.  xcds: the GPU has all
 // its XCDs' CUs.
 inline LeafPlan leaf_plan(int m, int wa, int panel_wgs, bool beside, bool xcds)
 {
@@ -59,12 +59,11 @@ inline LeafPlan leaf_plan(int m, int wa, int panel_wgs, bool beside, bool xcds)
     // of theirs could keep each other out, each with a part of its workgroups
     // running, so these give way (keep_waiting in panel.hip): a launch over all
     // XCDs, where eight of them find room, follows and does the work instead.
-    const int target = std::min(panel_wgs, XCD_CUS);
-    const LeafPlace tall = xcds && wa > 1 ? LEAF_ONE_XCD_YIELDS : LEAF_SPREAD;
-    if (g1 <= (beside || nc < 8 ? std::min(4 * panel_wgs, LEAF_GMAX) : target))
+    auto tall = [&](int g) { return xcds && wa > 1 && g <= XCD_CUS ? LEAF_ONE_XCD_YIELDS : LEAF_SPREAD; };
+    if (g1 <= (beside || nc < 8 ? std::min(4 * panel_wgs, LEAF_GMAX) : panel_wgs))
         return {v, 4, g1, xcds && g1 <= XCD_CUS ? LEAF_ONE_XCD : LEAF_SPREAD};
-    if (nc == 8 && g2 <= target) return {v, 8, g2, tall};
-    if (nc == 8 && g3 <= target) return {64, 8, g3, tall};
+    if (nc == 8 && g2 <= panel_wgs) return {v, 8, g2, tall(g2)};
+    if (nc == 8 && g3 <= panel_wgs) return {64, 8, g3, tall(g3)};
     // Over the XCDs the middle kind is the faster one (32 columns, m = 65536: 174 us
     // against 179 with half as many of the largest kind; 16 columns, 131072: 99, 115)
     if (g2 <= LEAF_GMAX) return {v, 8, g2, LEAF_SPREAD};

@@ -85,3 +85,14 @@ def test_narrow_leaves_hold_few_rows_a_quad(plans):
     for p in plans:
         if p["nc"] < 8 and p["m"] <= GMAX * 16 * ((16 if p["nc"] == 2 else 32) // p["nc"]) * 8:
             assert p["values"] < 64, p
+
+
+def test_preferred_workgroups(plans):
+    """panel_wgs over its whole range, wide leaves with no update beside them: at most
+    that many where a kind allows it, and more of them where the caller asks for more
+    than one die runs."""
+    by = {(p["m"], p["wa"], p["panel_wgs"]): p for p in plans if not p["beside"] and p["xcds"]}
+    for (m, wa, wgs), p in by.items():
+        if p["nc"] == 8 and m <= wgs * 16 * 8 * 8:
+            assert p["wgs"] <= wgs, p
+    assert [by[30011, 32, w]["wgs"] for w in (32, 64, 128)] == [30, 59, 118]
