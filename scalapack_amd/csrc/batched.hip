@@ -253,7 +253,8 @@ __device__ __forceinline__ void panel_regs(int n, int kb, int w, bool first, Glo
             const T *prow = sl.rows[pb][fw];
             const T pv = prow[jj], rcp = sl.rcp[pb][fw];
             const bool nz = pv != T(0);
-            if (tid == 0) piv[j] = p + 1;
+            // no interchange without a pivot (p != j if row j holds a NaN and others zeros)
+            if (tid == 0) piv[j] = (nz ? p : j) + 1;
             if (!nz && info == 0) info = j + 1;
 #pragma unroll
             for (int q = 0; q < RPT; q++) {
