@@ -76,12 +76,18 @@ __device__ __forceinline__ void tile_of(int id, int tm, int tn, int &im, int &in
     }
 }
 
-// TRAILING distinguishes the launches of the outer trailing update (1) from
-// every other use (0) in kernel traces.  The grid may be smaller than the tile
-// count (a persistent launch that leaves CUs free): workgroup b takes tiles b,
+// USE distinguishes the launches of the outer trailing update from the others in
+// kernel traces, and those of the solves, whose sums are of at most FOLD steps
+// (128 products) each and subtracted from C one after another: of 256 products in
+// one sum, PDGETRS's backward error was up to 1.2 times what it had been with four
+// sums side by side (n = 700).  The trailing update's grid may be smaller than the
+// tile count (a persistent launch that leaves CUs free): workgroup b takes tiles b,
 // b + grid, ...; grid is then a multiple of 8, so a tile index keeps its XCD.
 // O: type of the byte offsets within a tile's operands.
-template <typename T, typename O, bool TA, int BN, int TRAILING>
+enum Use { PLAIN = 0, TRAILING = 1, SOLVE = 2 };
+constexpr int FOLD = 8;
+
+template <typename T, typename O, bool TA, int BN, int USE>
 __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(4))) void gemm_tile_kernel(
     int m, int n, int k, const T *__restrict__ A, int lda, const T *__restrict__ B, int ldb,
     T *__restrict__ C, int ldc, unsigned long long *stamp)
@@ -92,13 +98,13 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(4))) void ge
     constexpr int LA = GM * GK / GT, LB = BN * GK / GT;  // loads of a thread and step
     __shared__ T As[2][GK][GM + 1];
     __shared__ T Bs[2][GK][BN + 1];
-    if (TRAILING) launch_stamp_begin(stamp);
+    if (USE == TRAILING) launch_stamp_begin(stamp);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, lk = lane >> 4;
     const int wm = BN == 64 ? (wave & 1) * 32 : wave * 16, wn = BN == 64 ? (wave >> 1) * 32 : 0;
     // column of C of accumulator element r within a 16 x 16 block
     auto ccol = [&](int r) { return sizeof(T) == 8 ? lk + 4 * r : 4 * lk + r; };
     const int tm = (m + GM - 1) / GM, tn = (n + BN - 1) / BN;
-    for (int tile = blockIdx.x; tile < tm * tn; tile += TRAILING ? gridDim.x : tm * tn) {
+    for (int tile = blockIdx.x; tile < tm * tn; tile += USE == TRAILING ? gridDim.x : tm * tn) {
     int im, in;
     tile_of(tile, tm, tn, im, in);
     const int bm = im * GM, bn = in * BN;
@@ -190,6 +196,15 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(4))) void ge
                 for (int j = 0; j < NB; j++)
                     acc[i][j] = mfma(b[j], a[i], acc[i][j]);
         }
+        if (USE == SOLVE && (t + 1) % FOLD == 0) {
+#pragma unroll
+            for (int i = 0; i < NA; i++)
+#pragma unroll
+                for (int j = 0; j < NB; j++) {
+                    c[i][j] -= acc[i][j];
+                    acc[i][j] = acc_t{0, 0, 0, 0};
+                }
+        }
         if (t + 1 < nk) store(buf ^ 1);
         __syncthreads();
     }
@@ -204,7 +219,7 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(4))) void ge
                     C[(size_t)row + (size_t)col * ldc] = c[i][j][r] - acc[i][j][r];
             }
     }  // tile loop
-    if (TRAILING) launch_stamp_end(stamp);
+    if (USE == TRAILING) launch_stamp_end(stamp);
 }
 
 }  // namespace
@@ -212,10 +227,11 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(4))) void ge
 template <typename T>
 void gemm_tile_sub(bool ta, int m, int n, int k, const T *A, int lda, const T *B, int ldb, T *C,
                    int ldc, hipStream_t s, bool trailing, int max_wgs, bool beside,
-                   unsigned long long *stamp)
+                   unsigned long long *stamp, bool solve)
 {
     if (m <= 0 || n <= 0 || k <= 0) return;
-    if (trailing && ta) throw std::logic_error("gemm: a trailing update is not transposed");
+    if (solve ? trailing || sizeof(T) != 8 : ta)
+        throw std::logic_error("gemm: only the solves' products, in FP64, are transposed");
     // n <= 32 would leave half of a 64-wide tile empty
     const int tiles = ceil_div(m, GM) * ceil_div(n, n <= 32 ? 32 : 64);
     const int grid = max_wgs >= 8 && tiles > max_wgs ? max_wgs / 8 * 8 : tiles;
@@ -228,33 +244,38 @@ void gemm_tile_sub(bool ta, int m, int n, int k, const T *A, int lda, const T *B
     const unsigned lds = beside ? 8000 : 0;
     // offsets of 64 columns and a step in 32 bits, but for extreme leading dimensions
     const bool small = (size_t)(64 + GK) * std::max(lda, ldb) * sizeof(T) < (size_t)UINT32_MAX;
-#define SLA_TILE(TAV, BNV, TR)                                                                      \
-    do {                                                                                            \
-        if (small)                                                                                  \
-            hipLaunchKernelGGL((gemm_tile_kernel<T, uint32_t, TAV, BNV, TR>), dim3(grid), dim3(GT), \
-                               lds, s, m, n, k, A, lda, B, ldb, C, ldc, stamp);                \
-        else                                                                                        \
-            hipLaunchKernelGGL((gemm_tile_kernel<T, uint64_t, TAV, BNV, TR>), dim3(grid), dim3(GT), \
-                               lds, s, m, n, k, A, lda, B, ldb, C, ldc, stamp);                \
+#define SLA_TILE(TAV, BNV, USEV)                                                                \
+    do {                                                                                        \
+        if (small)                                                                              \
+            hipLaunchKernelGGL((gemm_tile_kernel<T, uint32_t, TAV, BNV, USEV>), dim3(grid),     \
+                               dim3(GT), lds, s, m, n, k, A, lda, B, ldb, C, ldc, stamp);       \
+        else                                                                                    \
+            hipLaunchKernelGGL((gemm_tile_kernel<T, uint64_t, TAV, BNV, USEV>), dim3(grid),     \
+                               dim3(GT), lds, s, m, n, k, A, lda, B, ldb, C, ldc, stamp);       \
     } while (0)
     if (trailing) {
-        if (n <= 32) SLA_TILE(false, 32, 1);
-        else SLA_TILE(false, 64, 1);
-    } else if (n <= 32) {
-        if (ta) SLA_TILE(true, 32, 0);
-        else SLA_TILE(false, 32, 0);
-    } else {
-        if (ta) SLA_TILE(true, 64, 0);
-        else SLA_TILE(false, 64, 0);
+        if (n <= 32) SLA_TILE(false, 32, TRAILING);
+        else SLA_TILE(false, 64, TRAILING);
+    } else if (!solve) {
+        if (n <= 32) SLA_TILE(false, 32, PLAIN);
+        else SLA_TILE(false, 64, PLAIN);
+    } else if constexpr (sizeof(T) == 8) {
+        if (n <= 32) {
+            if (ta) SLA_TILE(true, 32, SOLVE);
+            else SLA_TILE(false, 32, SOLVE);
+        } else {
+            if (ta) SLA_TILE(true, 64, SOLVE);
+            else SLA_TILE(false, 64, SOLVE);
+        }
     }
 #undef SLA_TILE
     SLA_LAUNCH_CHECK();
 }
 template void gemm_tile_sub<double>(bool, int, int, int, const double *, int, const double *, int,
                                     double *, int, hipStream_t, bool, int, bool,
-                                    unsigned long long *);
+                                    unsigned long long *, bool);
 template void gemm_tile_sub<float>(bool, int, int, int, const float *, int, const float *, int,
                                    float *, int, hipStream_t, bool, int, bool,
-                                   unsigned long long *);
+                                   unsigned long long *, bool);
 
 }  // namespace sla

@@ -10,11 +10,12 @@ namespace sla {
 // outer trailing update (a kernel symbol of its own in traces); max_wgs > 0 caps
 // its workgroups (a persistent grid that leaves CUs to the panel running beside
 // it); beside: a panel runs on another stream meanwhile, so three workgroups a CU
-// instead of four; stamp: launch_stamp pair of a trailing update, or null.
+// instead of four; stamp: launch_stamp pair of a trailing update, or null; solve: a
+// product of the triangular solves, in sums of at most 128 terms.
 template <typename T>
 void gemm_tile_sub(bool ta, int m, int n, int k, const T *A, int lda, const T *B, int ldb, T *C,
                    int ldc, hipStream_t s, bool trailing = false, int max_wgs = 0, bool beside = false,
-                   unsigned long long *stamp = nullptr);
+                   unsigned long long *stamp = nullptr, bool solve = false);
 constexpr int GEMM_TILE_WGS_PER_CU = 4;  // workgroups that share a CU
 
 // ---- low-precision Schur-complement updates (FP32 storage) -----------------

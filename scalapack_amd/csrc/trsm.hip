@@ -947,7 +947,8 @@ void trsm_solve(TrsvOp op, int n, int nrhs, const double *A, int lda, double *X,
         SLA_LAUNCH_CHECK();
         const int r0 = fwd ? k1 : 0, r1 = fwd ? n : k0;  // rows still to be solved
         const double *off = trans ? A + (size_t)k0 + (size_t)r0 * lda : A + (size_t)r0 + (size_t)k0 * lda;
-        gemm_tile_sub<double>(trans, r1 - r0, nrhs, kb, off, lda, X + k0, ldx, X + r0, ldx, s);
+        gemm_tile_sub<double>(trans, r1 - r0, nrhs, kb, off, lda, X + k0, ldx, X + r0, ldx, s, false, 0,
+                              false, nullptr, true);
     }
 }
 
