@@ -234,7 +234,8 @@ void gemm_tile_sub(bool ta, int m, int n, int k, const T *A, int lda, const T *B
         throw std::logic_error("gemm: only the solves' products, in FP64, are transposed");
     // n <= 32 would leave half of a 64-wide tile empty
     const int tiles = ceil_div(m, GM) * ceil_div(n, n <= 32 ? 32 : 64);
-    const int grid = max_wgs >= 8 && tiles > max_wgs ? max_wgs / 8 * 8 : tiles;
+    // only the trailing update's kernel takes several tiles a workgroup
+    const int grid = trailing && max_wgs >= 8 && tiles > max_wgs ? max_wgs / 8 * 8 : tiles;
     // Beside a panel: LDS beyond the kernel's own, so that three workgroups (41 KB
     // each) share a CU and a fourth does not fit.  37 KB of LDS and a quarter of
     // the registers stay free for the panel's kernels, which otherwise wait until
