@@ -27,7 +27,7 @@ ARCH = os.environ.get("SLA_OFFLOAD_ARCH", "gfx950")
 # (source, object stem, extra flags): the panel leaf's two storage types are
 # separate objects of one source so that they compile in parallel
 HIP_SOURCES = [(f, f[:-4], []) for f in
-               ["gemm_tile.hip", "gemm_lowp.hip", "panel_tslu.hip", "swap.hip",
+               ["gemm_tile.hip", "gemm_wide.hip", "gemm_lowp.hip", "panel_tslu.hip", "swap.hip",
                 "trsm.hip", "lu.hip", "mixed.hip", "aux.hip", "batched.hip", "mlp.hip", "capi.hip"]]
 HIP_SOURCES += [("panel.hip", "panel_f64", ["-DSLA_PANEL_TYPE=64"]),
                 ("panel.hip", "panel_f32", ["-DSLA_PANEL_TYPE=32"])]

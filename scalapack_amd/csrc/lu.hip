@@ -261,6 +261,7 @@ struct Lu {
     PanelWork<T> pw;
     int schur = SCHUR_NATIVE;  // precision of the outer trailing update
     bool beside = false;       // the next trailing update runs beside a panel
+    bool outlasts = false;     // and for longer than it
     bool l_packed = false;     // L21 of the current block column is packed
     hipStream_t s_main = nullptr, s_panel = nullptr;  // update stream, panel stream
     const T *inv_of[2] = {nullptr, nullptr};  // L11 whose inverses each stream's area holds
@@ -360,6 +361,18 @@ struct Lu {
         panel(r0 + n1, c0 + n1, n - n1, pc0, pc1, s);
     }
 
+    // What the look-ahead expects of the two streams, in us.  A trailing update of
+    // this precision (flops per us measured at m = n = 16128, k = 512; FP64 with
+    // three workgroups a CU), and a panel of n columns beside one: a leaf and what
+    // lies between it and the next take 290 us at m = 16384, NB = 256 and 400 - 460 at
+    // m = 32768, NB = 512.
+    double update_us(double m, double n, double k) const
+    {
+        static const double low[] = {95e6, 400e6, 400e6, 210e6, 110e6, 210e6};  // by enum Schur
+        return 2.0 * m * n * k / (std::is_same<T, double>::value ? 48e6 : low[schur]);
+    }
+    double panel_us(int n) const { return 400.0 * ceil_div(n, h.leaf_w); }
+
     // Right-looking blocked LU (SRC/pdgetrf.f:227-295) with a look-ahead of
     // one block column.  Main stream S0, step of block column p = [j, jn):
     //   apply p's interchanges to the next block column and to the kept row
@@ -398,6 +411,7 @@ struct Lu {
                 break;
             }
             l_packed = false;
+            const int c = jn + jb2, rest = N - c;
             if (has_next) {
                 trsm(jb, jb2, at(j, j), at(j, jn), s0);
                 update(M - jn, jb2, jb, at(jn, j), at(j, jn), at(jn, jn), s0);
@@ -405,20 +419,20 @@ struct Lu {
                 SLA_HIP(hipStreamWaitEvent(s1, h.ev_next, 0));
                 // a trailing update that outlasts a leaf: the leaf has to start
                 // beside it, not after it
-                const double update_us = 2.0 * (M - jn) * (N - jn - jb2) * jb / 50e6;
+                const double rest_us = update_us(M - jn, rest, jb);
                 beside = s0 != s1;
-                pw.beside = beside && update_us > 100.0;
+                pw.beside = beside && rest_us > 100.0;
+                outlasts = beside && rest_us > 1.2 * panel_us(jb2);
                 panel(jn, jn, jb2, jn, jn + jb2, s1);
                 make_pairs(jn, jn + jb2, q ^ 1, s1);
                 SLA_HIP(hipEventRecord(h.ev_panel, s1));
             }
-            const int c = jn + jb2, rest = N - c;
             swap_block(j, jn, q, 0, j, s0);
             swap_block(j, jn, q, c, rest, s0);
             if (rest > 0) {
                 trsm(jb, rest, at(j, j), at(j, c), s0);
                 if (jn < M) update(M - jn, rest, jb, at(jn, j), at(j, c), at(jn, c), s0);
-                beside = false;
+                beside = outlasts = false;
             }
             if (has_next) SLA_HIP(hipStreamWaitEvent(s0, h.ev_panel, 0));
         }
@@ -443,8 +457,13 @@ void Lu<double>::update(int m, int n, int k, const double *l21, const double *u1
     if (m <= 0 || n <= 0 || k <= 0) return;
     h.timing_begin(CAT_GEMM, s);
     unsigned long long *st = h.next_kstamp(2.0 * m * n * k);
-    gemm_tile_sub<double>(false, m, n, k, l21, lda, u12, lda, c, lda, s, true,
-                          GEMM_TILE_WGS_PER_CU * h.update_cus, beside, st);
+    // An update that outlasts its panel is what the factorization waits for, so it
+    // takes the kernel that is the faster one on its own; at least 1.2 times as long
+    // (N = 20480, 24576, 32768 and 39936, NB = 512: 183.2 -> 181.6, 277.1 -> 272.5, 564.5 ->
+    // 547.7, 969 -> 926 ms; from 0.7 times on the first two gain nothing).
+    if (!outlasts || !gemm_wide_sub(m, n, k, l21, lda, u12, lda, c, lda, s, h.update_cus, st))
+        gemm_tile_sub<double>(false, m, n, k, l21, lda, u12, lda, c, lda, s, true,
+                              GEMM_TILE_WGS_PER_CU * h.update_cus, beside, st);
     h.timing_end(2.0 * m * n * k, s);
 }
 

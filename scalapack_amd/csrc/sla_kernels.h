@@ -17,6 +17,11 @@ void gemm_tile_sub(bool ta, int m, int n, int k, const T *A, int lda, const T *B
                    int ldc, hipStream_t s, bool trailing = false, int max_wgs = 0, bool beside = false,
                    unsigned long long *stamp = nullptr, bool solve = false);
 constexpr int GEMM_TILE_WGS_PER_CU = 4;  // workgroups that share a CU
+// C[m x n] -= A * B in FP64 for a trailing update that outlasts its panel
+// (gemm_wide.hip), at most max_wgs > 0 workgroups of the whole CU each; false, and
+// nothing done, where shape or alignment do not allow it.
+bool gemm_wide_sub(int m, int n, int k, const double *A, int lda, const double *B, int ldb,
+                   double *C, int ldc, hipStream_t s, int max_wgs, unsigned long long *stamp);
 
 // ---- low-precision Schur-complement updates (FP32 storage) -----------------
 // C[m x n] -= A[m x k] * B[k x n], FP32 operands on FP32 MFMA.
