@@ -363,8 +363,13 @@ __global__ __launch_bounds__(256) void trsv_persistent_kernel(
                         break;
                     }
                 }
-                // workgroups far behind the chain poll less often
-                if (t - s > 4) __builtin_amdgcn_s_sleep(16);
+                // Workgroups far behind the chain poll less often.  The transposed solves
+                // read down columns, which is slow enough at large n for the others'
+                // polls to be in the way (one right-hand side, n = 28000, U^T and L^T
+                // together: 5.28 ms with 16, 5.12 so; n = 4096 539, 526 us; the same in
+                // the other two, n = 4096: 542, 545 us).
+                if (TRANS && t - s > 32) __builtin_amdgcn_s_sleep(127);
+                else if (t - s > 4) __builtin_amdgcn_s_sleep(16);
             }
         }
         __syncthreads();
