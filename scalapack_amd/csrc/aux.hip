@@ -83,7 +83,9 @@ __global__ __launch_bounds__(256) void lange_max_kernel(int m, int n, const doub
 // rows read down their columns (coalesced) into LDS, then lane c adds the tile's
 // rows of column c one after another while the next tile is on its way.  Bound by
 // the chain of m additions.  One wave per 64 columns, which read and added in turn,
-// took 562 us at 2003 x 2003; PDGESVX there went from 11.42 to 10.89 ms.
+// took 562 us at 2003 x 2003; PDGESVX there went from 11.42 to 10.89 ms.  The
+// last tile's additions go only as far as there are rows, or one row costs what 256
+// do (1 x 1000000: 190 us, so 132; 132 with the 64 columns a wave too).
 constexpr int CS_C = 16, CS_R = 256;
 __global__ __launch_bounds__(CS_R) void lange_colsum_kernel(int m, int n, const double *__restrict__ A,
                                                             int lda, double *__restrict__ colsum)
@@ -106,11 +108,18 @@ __global__ __launch_bounds__(CS_R) void lange_colsum_kernel(int m, int n, const 
         load(r0 + CS_R);
         if (tid < CS_C) {  // rows from m on are zeros, which change no sum
             const d2_t *t = reinterpret_cast<const d2_t *>(T[tid]);
-#pragma unroll 16
-            for (int k = 0; k < CS_R / 2; k++) {
+            auto add = [&](int k) {
                 const d2_t x = t[k];
                 sum += x[0];
                 sum += x[1];
+            };
+            if (m - r0 >= CS_R) {
+#pragma unroll 16
+                for (int k = 0; k < CS_R / 2; k++) add(k);
+            } else {
+                for (int k0 = 0; k0 < (m - r0 + 1) / 2; k0 += 8)
+#pragma unroll
+                    for (int k = 0; k < 8; k++) add(k0 + k);
             }
         }
         __syncthreads();
