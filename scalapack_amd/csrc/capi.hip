@@ -163,7 +163,7 @@ struct Bounce {
     bool open(int ld, int n)
     {
         cols = (int)std::min<size_t>(n, HALF / 8 / (size_t)ld);
-        if (cols < 1) return false;
+        if (n < 2 || cols < 1) return false;
         for (int i = 0; i < (cols < n ? 2 : 1); i++) {
             if (hipHostMalloc((void **)&p[i], (size_t)ld * cols * 8, hipHostMallocDefault) != hipSuccess) {
                 (void)hipGetLastError();
@@ -199,11 +199,25 @@ struct Bounce {
 // hipMemcpy2D between a pageable array and the device moves it row by row of its
 // own, at 9 us a column: 13.9 ms in and 10.7 ms out for 1500 x 1500.  Packed to
 // the device's leading dimension and sent as contiguous pieces the same takes
-// 0.5 ms each way.  A column longer than a half of the pinned memory goes by
-// itself at the full rate either way.
+// 0.5 ms each way.  A single column, or one longer than a half of the pinned memory,
+// goes by itself at the full rate either way.  Up to 1 MB the pieces are packed in ordinary
+// memory, which the runtime stages itself: 12 - 50 us, where allocating pinned memory
+// takes 13 - 25 us each time, and 280 for some sequences of small sizes.  PDGETRS
+// from host arrays, us, column by column, all pinned, now: N = 1, one right-hand
+// side 146, 259, 146; N = 20, six 401, 805, 154.
+constexpr size_t PACK_BYTES = (size_t)1 << 20;
+
 void to_device(double *dst, int ldd, const double *src, int lds, int m, int n)
 {
     if (m <= 0 || n <= 0) return;
+    const size_t words = (size_t)(n - 1) * ldd + m;
+    if (n > 1 && words * 8 <= PACK_BYTES) {
+        std::unique_ptr<double[]> h(new double[words]);
+        for (int c = 0; c < n; c++)
+            std::memcpy(h.get() + (size_t)c * ldd, src + (size_t)c * lds, (size_t)m * 8);
+        SLA_HIP(hipMemcpy(dst, h.get(), words * 8, hipMemcpyHostToDevice));
+        return;
+    }
     Bounce b;
     if (!b.open(ldd, n)) {
         SLA_HIP(hipMemcpy2D(dst, (size_t)ldd * 8, src, (size_t)lds * 8, (size_t)m * 8, n,
@@ -225,6 +239,14 @@ void to_device(double *dst, int ldd, const double *src, int lds, int m, int n)
 void to_host(double *dst, int ldd, const double *src, int lds, int m, int n)
 {
     if (m <= 0 || n <= 0) return;
+    const size_t words = (size_t)(n - 1) * lds + m;
+    if (n > 1 && words * 8 <= PACK_BYTES) {
+        std::unique_ptr<double[]> h(new double[words]);
+        SLA_HIP(hipMemcpy(h.get(), src, words * 8, hipMemcpyDeviceToHost));
+        for (int c = 0; c < n; c++)
+            std::memcpy(dst + (size_t)c * ldd, h.get() + (size_t)c * lds, (size_t)m * 8);
+        return;
+    }
     Bounce b;
     if (!b.open(lds, n)) {
         SLA_HIP(hipMemcpy2D(dst, (size_t)ldd * 8, src, (size_t)lds * 8, (size_t)m * 8, n,
