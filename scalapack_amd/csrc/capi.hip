@@ -1423,7 +1423,7 @@ int sla_dgemm_sub(sla_handle_t h, int m, int n, int k, const double *dA, int lda
     SLA_TRY({
         auto &H = *reinterpret_cast<sla::Handle *>(h);
         H.timing_begin(sla::CAT_GEMM);
-        sla::gemm_tile_sub<double>(false, m, n, k, dA, lda, dB, ldb, dC, ldc, H.stream);
+        sla::dgemm_alone_sub(m, n, k, dA, lda, dB, ldb, dC, ldc, H.stream, H.num_cus);
         H.timing_end(2.0 * m * n * k);
         SLA_HIP(hipStreamSynchronize(H.stream));
         H.timing_collect();

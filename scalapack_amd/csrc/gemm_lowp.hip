@@ -103,8 +103,7 @@ __global__ __launch_bounds__(256, 2) void sgemm_nn_sub_direct_kernel(
     int ldb, float *__restrict__ C, int ldc, unsigned long long *stamp)
 {
     launch_stamp_begin(stamp);
-    // persistent when the grid is smaller than the tile count (see
-    // dgemm_nn_sub_direct_kernel)
+    // persistent when the grid is smaller than the tile count (as in gemm_tile.hip)
     for (int tile = blockIdx.x; tile < (m / 128) * (n / 128); tile += gridDim.x) {
     int tmi, tni;
     tile_coords_lp(tile, m / 128, n / 128, tmi, tni);
@@ -752,10 +751,14 @@ void sgemm_nn_sub(int m, int n, int k, const float *A, int lda, const float *B, 
                   unsigned long long *stamp)
 {
     if (m <= 0 || n <= 0 || k <= 0) return;
-    const int mf = (m / 128) * 128, nf = (n / 128) * 128;
-    if (trailing && mf > 0 && nf > 0 && k % 16 == 0 && lda % 4 == 0 && ldb % 4 == 0 &&
-        ldc % 4 == 0 && aligned16(A) && aligned16(B) && aligned16(C)) {
-        const int tiles = (mf / 128) * (nf / 128);
+    const int mf = (m / 128) * 128, nf = (n / 128) * 128, tiles = (mf / 128) * (nf / 128);
+    // Alone on the GPU 64 x 64 tiles are the faster ones (m = n = 1024, k = 512: 1.39 times;
+    // 4096: 1.09; 8192: 1.12), except where a tile of 128 x 128 is had by most CUs and
+    // none has two, and k is long: 2048, k = 512: 59 against 69 us, k = 4096: 296, 411; 1536,
+    // k = 2048: 159, 171; k = 512: 58, 57
+    const bool one_each = tiles >= 128 && tiles <= 256 && tiles * (size_t)k >= 256 * 512;
+    if ((trailing || one_each) && mf > 0 && nf > 0 && k % 16 == 0 && lda % 4 == 0 &&
+        ldb % 4 == 0 && ldc % 4 == 0 && aligned16(A) && aligned16(B) && aligned16(C)) {
         const int grid = (max_wgs >= 8 && tiles > max_wgs) ? (max_wgs / 8) * 8 : tiles;
         // reserve_lds: LDS the kernel does not use, reserved so that at most
         // floor(LDS per CU / reserve_lds) workgroups share a CU and registers
@@ -769,15 +772,19 @@ void sgemm_nn_sub(int m, int n, int k, const float *A, int lda, const float *B, 
                 attr_set = reserve_lds;
             }
         }
-        hipLaunchKernelGGL(sgemm_nn_sub_direct_kernel<1>, dim3(grid), dim3(256),
-                           (unsigned)std::max(0, reserve_lds), s, mf, nf, k, A, lda, B, ldb, C, ldc,
-                           stamp);
+        if (trailing)
+            hipLaunchKernelGGL(sgemm_nn_sub_direct_kernel<1>, dim3(grid), dim3(256),
+                               (unsigned)std::max(0, reserve_lds), s, mf, nf, k, A, lda, B, ldb, C,
+                               ldc, stamp);
+        else
+            hipLaunchKernelGGL(sgemm_nn_sub_direct_kernel<0>, dim3(tiles), dim3(256), 0, s, mf, nf,
+                               k, A, lda, B, ldb, C, ldc, (unsigned long long *)nullptr);
         SLA_LAUNCH_CHECK();
         if (m > mf)
-            gemm_tile_sub<float>(false, m - mf, n, k, A + mf, lda, B, ldb, C + mf, ldc, s, true);
+            gemm_tile_sub<float>(false, m - mf, n, k, A + mf, lda, B, ldb, C + mf, ldc, s, trailing);
         if (n > nf)
             gemm_tile_sub<float>(false, mf, n - nf, k, A, lda, B + (size_t)nf * ldb, ldb,
-                                 C + (size_t)nf * ldc, ldc, s, true);
+                                 C + (size_t)nf * ldc, ldc, s, trailing);
         return;
     }
     gemm_tile_sub<float>(false, m, n, k, A, lda, B, ldb, C, ldc, s, trailing, max_wgs, false, stamp);

@@ -1,5 +1,6 @@
-// gemm_wide.hip -- C[m x n] -= A[m x k] * B[k x n] in FP64 with a larger tile than
-// gemm_tile.hip's, for the trailing updates that outlast the panel beside them.
+// gemm_wide.hip -- C[m x n] -= A[m x k] * B[k x n] in FP64 with larger tiles than
+// gemm_tile.hip's, for the trailing updates that outlast the panel beside them and
+// for large products alone on the GPU.
 //
 // Bound by the matrix cores.  A 512-thread workgroup, one a CU, takes a 128 x 256 tile,
 // two waves a SIMD, so per flop it moves a third of what 64 x 64 tiles move through
@@ -133,15 +134,96 @@ __global__ __launch_bounds__(XT, 1) void dgemm_nn_sub_wide_kernel(
     launch_stamp_end(stamp);
 }
 
+// No LDS and no workgroup barrier: a 128 x 128 tile per 256-thread workgroup, one a
+// CU, each wave a 64 x 64 part whose operands it loads itself, three 16-deep K steps in
+// flight.  Two index permutations make every lane's operands 32 contiguous bytes:
+//   rows : MFMA block i, operand row lr  <->  C row wm + 4 lr + i
+//   K    : operand k-lane lk, step s     <->  k = k0 + 4 lk + s
+// A and B use the same K permutation; D element r of lane l (block row l / 16 + 4 r) is C
+// row wm + 4 (l / 16 + 4 r) + i, four consecutive rows for i = 0 .. 3.  Requires m, n
+// multiples of 128, k of 16, and 32-byte aligned columns.
+constexpr int DEPTH = 3;
+
+__global__ __launch_bounds__(256, 1) void dgemm_nn_sub_direct_kernel(
+    int m, int n, int k, const double *__restrict__ A, int lda,
+    const double *__restrict__ B, int ldb, double *__restrict__ C, int ldc)
+{
+    int tmi, tni;
+    tile_coords(blockIdx.x, m / 128, n / 128, tmi, tni);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = tmi * 128 + (wave & 1) * 64, wn = tni * 128 + (wave >> 1) * 64;
+    const int lr = lane & 15, lk = lane >> 4;
+    const double *Ap = A + (wm + 4 * lr) + (size_t)(4 * lk) * lda;
+    const double *Bp = B + (size_t)(wn + lr) * ldb + 4 * lk;
+    const size_t bstep = (size_t)16 * ldb;
+
+    d4_t a[DEPTH][4], b[DEPTH][4];
+    auto load = [&](int t, int q) {
+        const size_t k0 = (size_t)16 * t;
+#pragma unroll
+        for (int s = 0; s < 4; s++) a[q][s] = *(const d4_t *)(Ap + (k0 + s) * lda);
+#pragma unroll
+        for (int j = 0; j < 4; j++) b[q][j] = *(const d4_t *)(Bp + j * bstep + k0);
+    };
+    d4_t acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[i][j] = d4_t{0.0, 0.0, 0.0, 0.0};
+
+    const int nk = k / 16;
+#pragma unroll
+    for (int q = 0; q < DEPTH - 1; q++)
+        if (q < nk) load(q, q);
+    for (int t = 0; t < nk; t += DEPTH) {
+#pragma unroll
+        for (int q = 0; q < DEPTH; q++) {
+            if (t + q < nk) {
+                const int nt = t + q + DEPTH - 1;
+                if (nt < nk) load(nt, (q + DEPTH - 1) % DEPTH);
+#pragma unroll
+                for (int s = 0; s < 4; s++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+#pragma unroll
+                        for (int j = 0; j < 4; j++)
+                            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q][s][i], b[q][j][s],
+                                                                            acc[i][j], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        double *Cc = C + (size_t)(wn + 16 * j + lr) * ldc;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            d4_t *cp = (d4_t *)(Cc + wm + 4 * (lk + 4 * r));
+            d4_t c = *cp;
+            c[0] -= acc[0][j][r];
+            c[1] -= acc[1][j][r];
+            c[2] -= acc[2][j][r];
+            c[3] -= acc[3][j][r];
+            *cp = c;
+        }
+    }
+}
+
+// What both kernels require of the operands.
+bool aligned32(int k, const double *A, int lda, const double *B, int ldb, const double *C, int ldc)
+{
+    auto ok = [](const double *p, int ld) {
+        return (reinterpret_cast<uintptr_t>(p) & 31) == 0 && ld % 4 == 0;
+    };
+    return k > 0 && k % 16 == 0 && ok(A, lda) && ok(B, ldb) && ok(C, ldc);
+}
+
 }  // namespace
 
 bool gemm_wide_sub(int m, int n, int k, const double *A, int lda, const double *B, int ldb,
                    double *C, int ldc, hipStream_t s, int max_wgs, unsigned long long *stamp)
 {
-    auto aligned = [](const double *p, int ld) { return (reinterpret_cast<uintptr_t>(p) & 31) == 0 && ld % 4 == 0; };
     const int mw = m / XM * XM, nw = n / XN * XN;
-    if (mw <= 0 || nw <= 0 || k <= 0 || k % XK != 0 || !aligned(A, lda) || !aligned(B, ldb) || !aligned(C, ldc))
-        return false;
+    if (mw <= 0 || nw <= 0 || !aligned32(k, A, lda, B, ldb, C, ldc)) return false;
     const int tiles = (mw / XM) * (nw / XN);
     const int grid = max_wgs >= 8 && tiles > max_wgs ? max_wgs / 8 * 8 : tiles;
     hipLaunchKernelGGL(dgemm_nn_sub_wide_kernel<1>, dim3(grid), dim3(XT), 0, s, mw, nw, k, A, lda, B,
@@ -154,6 +236,32 @@ bool gemm_wide_sub(int m, int n, int k, const double *A, int lda, const double *
                           C + (size_t)nw * ldc, ldc, s, true, GEMM_TILE_WGS_PER_CU * max_wgs, false,
                           stamp);
     return true;
+}
+
+void dgemm_alone_sub(int m, int n, int k, const double *A, int lda, const double *B, int ldb,
+                     double *C, int ldc, hipStream_t s, int cus)
+{
+    // The larger tiles are worth their while for long sums and where a tile a CU
+    // leaves hardly any CU idle in the last round.  TF/s with tiles of 64 x 64, 128 x
+    // 128, 128 x 256: m = n = 2048, k = 512 41, 44, 27; k = 4096 53, 63, 33; 3072, k =
+    // 4096 (2.25 rounds) 55, 50, 37; 4096, k = 512 54, 56, 56; k = 4096 60, 65, 65; 6144, k =
+    // 512 55, 52, 50; k = 2048 59, 63, 58; 12288, k = 512 57, 54, 57; k = 1024 59, 60, 62.
+    auto full = [&](int t) { return t >= 0.95 * cus * ceil_div(t, cus); };
+    const int md = m / 128 * 128, nd = n / 128 * 128;
+    const int wide = (m / XM) * (n / XN), direct = (md / 128) * (nd / 128);
+    if (k >= 1024 && wide > 0 && full(wide) && gemm_wide_sub(m, n, k, A, lda, B, ldb, C, ldc, s, 0, nullptr))
+        return;
+    if (direct > 0 && full(direct) && (k >= 1024 || (k >= 512 && direct <= 4 * cus)) &&
+        aligned32(k, A, lda, B, ldb, C, ldc)) {
+        hipLaunchKernelGGL(dgemm_nn_sub_direct_kernel, dim3(direct), dim3(256), 0, s, md, nd, k, A,
+                           lda, B, ldb, C, ldc);
+        SLA_LAUNCH_CHECK();
+        gemm_tile_sub<double>(false, m - md, n, k, A + md, lda, B, ldb, C + md, ldc, s);
+        gemm_tile_sub<double>(false, md, n - nd, k, A, lda, B + (size_t)nd * ldb, ldb,
+                              C + (size_t)nd * ldc, ldc, s);
+        return;
+    }
+    gemm_tile_sub<double>(false, m, n, k, A, lda, B, ldb, C, ldc, s);
 }
 
 }  // namespace sla

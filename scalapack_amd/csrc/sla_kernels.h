@@ -22,6 +22,9 @@ constexpr int GEMM_TILE_WGS_PER_CU = 4;  // workgroups that share a CU
 // nothing done, where shape or alignment do not allow it.
 bool gemm_wide_sub(int m, int n, int k, const double *A, int lda, const double *B, int ldb,
                    double *C, int ldc, hipStream_t s, int max_wgs, unsigned long long *stamp);
+// The same alone on a GPU of `cus` CUs, any shape and alignment.
+void dgemm_alone_sub(int m, int n, int k, const double *A, int lda, const double *B, int ldb,
+                     double *C, int ldc, hipStream_t s, int cus);
 
 // ---- low-precision Schur-complement updates (FP32 storage) -----------------
 // C[m x n] -= A[m x k] * B[k x n], FP32 operands on FP32 MFMA.
