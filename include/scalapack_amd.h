@@ -191,7 +191,9 @@ int sla_reset_stats(sla_handle_t h);
  * HBM.  dipiv: device int[min(m,n)], 1-based pivot rows (PDGETRF's IPIV for
  * IA = JA = 1).  *info as PDGETRF's INFO (> 0: exactly zero pivot). */
 int sla_dgetrf(sla_handle_t h, int m, int n, double *dA, int lda, int *dipiv, int *info);
-/* Solve A X = B with the factors of sla_dgetrf (TRANS = 'N'). */
+/* Solve A X = B with the factors of sla_dgetrf (TRANS = 'N').  The handle keeps a
+ * workspace of n x min(nrhs, 1024) doubles (fewer columns at a time, 16 at least, if
+ * the device has no memory for as many). */
 int sla_dgetrs(sla_handle_t h, int n, int nrhs, const double *dA, int lda, const int *dipiv,
                double *dB, int ldb);
 int sla_dgesv(sla_handle_t h, int n, int nrhs, double *dA, int lda, int *dipiv, double *dB,

@@ -24,6 +24,7 @@
 #include <cstring>
 #include <string>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 namespace sla {
@@ -141,18 +142,31 @@ TrsvWork Handle::trsv_work(int n)
 void Handle::ensure_perm(int m)
 {
     if (m <= perm_cap) return;
-    if (perm) SLA_HIP(hipFree(perm));
+    if (perm) SLA_HIP(hipFree(std::exchange(perm, nullptr)));
+    perm_cap = 0;
     perm = alloc_dev<int>((size_t)m);
     perm_cap = m;
 }
 
+bool Handle::try_work(size_t bytes)
+{
+    if (bytes <= work_cap) return true;
+    SLA_HIP(hipStreamSynchronize(stream));
+    if (work) SLA_HIP(hipFree(std::exchange(work, nullptr)));
+    work_cap = 0;
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes + 256) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    work = static_cast<char *>(p);
+    work_cap = bytes;
+    return true;
+}
+
 void Handle::ensure_work(size_t bytes)
 {
-    if (bytes <= work_cap) return;
-    SLA_HIP(hipStreamSynchronize(stream));
-    if (work) SLA_HIP(hipFree(work));
-    work = alloc_dev<char>(bytes);
-    work_cap = bytes;
+    if (!try_work(bytes)) throw std::runtime_error("device memory: no room for the workspace");
 }
 
 void *Handle::buffer(int id, size_t bytes)
@@ -161,7 +175,8 @@ void *Handle::buffer(int id, size_t bytes)
     if (bytes > b.cap) {
         SLA_HIP(hipStreamSynchronize(stream));
         SLA_HIP(hipStreamSynchronize(stream2));
-        if (b.p) SLA_HIP(hipFree(b.p));
+        if (b.p) SLA_HIP(hipFree(std::exchange(b.p, nullptr)));
+        b.cap = 0;
         b.p = alloc_dev<char>(bytes);
         b.cap = bytes;
     }
@@ -658,9 +673,11 @@ void getrs_perm_device(Handle &h, bool trans, int n, int nrhs, const double *dA,
     // blocked solves whose products run on the matrix cores (n = 5000, 400
     // right-hand sides: 96 ms sixteen at a time, 2.9 ms blocked), in chunks that
     // bound the copy.
-    const bool many = nrhs > 16;
-    const int chunk = std::min(nrhs, many ? 1024 : 16);
+    int chunk = std::min(nrhs, nrhs > 16 ? 1024 : 16);
+    // fewer columns at a time where the device has no memory for as many
+    while (!h.try_work((size_t)n * chunk * sizeof(double)) && chunk > 16) chunk = std::max(16, chunk / 2);
     h.ensure_work((size_t)n * chunk * sizeof(double));
+    const bool many = chunk > 16;
     double *W = reinterpret_cast<double *>(h.work);
     TrsvWork tw = h.trsv_work(n);
     auto solve = [&](TrsvOp op, int nr) {

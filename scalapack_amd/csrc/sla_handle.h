@@ -237,6 +237,7 @@ struct Handle {
     PanelWork<T> panel_work();
     TrsvWork trsv_work(int n);  // mailbox sized for triangles of order n
     void ensure_perm(int m);
+    bool try_work(size_t bytes);  // false: no memory, and no workspace held
     void ensure_work(size_t bytes);
 };
 
