@@ -27,9 +27,10 @@
 // Bound: small systems by the chain of columns (under 1 us each: search, post,
 // barrier, fold, update), large ones by the passes over A22, n / 64 of them, and over
 // L21, once a strip, since the systems in flight (512 of n = 512 are 1 GB) do not
-// stay in cache.  512 threads and at most 128 registers, none of them in scratch,
-// keep 16 waves on a CU with two workgroups, where 256 threads with 196 registers
-// kept eight.  Before, A22 was passed over n / W times, the interchanges of a column
+// stay in cache.  512 threads and at most 128 registers keep 16 waves on a CU with
+// two workgroups, where 256 threads with 196 registers kept eight.  (In scratch are 16
+// bytes a lane with FP64 panels of 32 columns, read back once a block, and 28 of the
+// FP64 solve, six values a block of 64 rows; none within a panel, strip or triangle.)  Before, A22 was passed over n / W times, the interchanges of a column
 // were one after another in memory, U12 and A22 went through LDS with a barrier
 // around every 64 x 64 tile, and the search took eighteen lane exchanges.
 // Factorization and solve of 512 systems with interchanges, us, that -> strips behind
@@ -83,50 +84,6 @@ using Global = __attribute__((address_space(1))) T;
 
 typedef double bd4_t __attribute__((ext_vector_type(4)));
 typedef float bf4_t __attribute__((ext_vector_type(4)));
-
-// A barrier that waits for the workgroup's LDS traffic only: panel_regs stores to
-// global memory between barriers and nobody reads that before the panel's end.
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-template <int CTRL, int ROWS>
-__device__ __forceinline__ uint32_t dpp_max(uint32_t x)
-{
-    // lanes the move does not reach combine with 0
-    const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
-    return x > y ? x : y;
-}
-
-// Wave-wide maximum, uniform.
-__device__ __forceinline__ uint32_t wave_max(uint32_t x)
-{
-    x = dpp_max<0x121, 0xf>(x);
-    x = dpp_max<0x122, 0xf>(x);
-    x = dpp_max<0x124, 0xf>(x);
-    x = dpp_max<0x128, 0xf>(x);
-    x = dpp_max<0x142, 0xa>(x);
-    x = dpp_max<0x143, 0xc>(x);
-    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
-}
-
-// The value of lane S of the quad, in all four lanes.
-template <int S, typename T>
-__device__ __forceinline__ T quad_lane(T v)
-{
-    if constexpr (sizeof(T) == 8) {
-        const uint64_t u = __builtin_bit_cast(uint64_t, v);
-        const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, S * 0x55, 0xf, 0xf, false);
-        const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), S * 0x55, 0xf, 0xf, false);
-        return __builtin_bit_cast(T, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-    } else {
-        return __builtin_bit_cast(
-            T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), S * 0x55, 0xf, 0xf, false));
-    }
-}
 
 // A pivot candidate's rank, (hi, lo) compared as one number: 0 for no candidate,
 // then a NaN in row j (kept only if nothing is comparable), then |v|.
@@ -521,21 +478,6 @@ struct SolveLds {
     alignas(16) int piv[BATCHED_NMAX];
     int moved;
 };
-
-// The value of lane K of every row of 16 lanes, in all of them.
-template <int K, typename T>
-__device__ __forceinline__ T row_lane(T v)
-{
-    if constexpr (sizeof(T) == 8) {
-        const uint64_t u = __builtin_bit_cast(uint64_t, v);
-        const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, 0x150 + K, 0xf, 0xf, false);
-        const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), 0x150 + K, 0xf, 0xf, false);
-        return __builtin_bit_cast(T, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-    } else {
-        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
-                                                                 0x150 + K, 0xf, 0xf, false));
-    }
-}
 
 // Steps of a 16 x 16 triangle, top down (L, unit) or bottom up (U): lane l of a row
 // of 16 lanes holds row l of b[0], and in b[1] .. b[3] what the solved values take

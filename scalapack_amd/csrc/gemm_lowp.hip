@@ -165,24 +165,18 @@ __global__ __launch_bounds__(256, 2) void sgemm_nn_sub_direct_kernel(
     launch_stamp_end(stamp);
 }
 
-// Ragged edges (and small shapes) of either precision: one thread per element
-// of C, operands read through a converter.  Only a thin border ever lands here.
-template <typename TA>
-__device__ __forceinline__ float to_f(TA v) { return (float)v; }
-
-template <typename TA, bool AROW>
-__global__ __launch_bounds__(256) void gemm_lp_edge_kernel(int m, int n, int k, const TA *A,
-                                                           int lda, const TA *B, int ldb,
-                                                           float *C, int ldc)
+// BF16's ragged edges (and small shapes): one thread per element of C, A by rows.
+// Only a thin border ever lands here.
+__global__ __launch_bounds__(256) void gemm_bf16_edge_kernel(int m, int n, int k, const __bf16 *A,
+                                                             int lda, const __bf16 *B, int ldb,
+                                                             float *C, int ldc)
 {
     const int i = blockIdx.x * 16 + (threadIdx.x & 15);
     const int j = blockIdx.y * 16 + (threadIdx.x >> 4);
     if (i >= m || j >= n) return;
     float acc = 0.f;
-    for (int kk = 0; kk < k; kk++) {
-        const float av = AROW ? to_f(A[(size_t)i * lda + kk]) : to_f(A[i + (size_t)kk * lda]);
-        acc = fmaf(av, to_f(B[kk + (size_t)j * ldb]), acc);
-    }
+    for (int kk = 0; kk < k; kk++)
+        acc = fmaf((float)A[(size_t)i * lda + kk], (float)B[kk + (size_t)j * ldb], acc);
     C[i + (size_t)j * ldc] -= acc;
 }
 
@@ -807,8 +801,7 @@ void gemm_bf16_nn_sub(int m, int n, int k, const __bf16 *Ap, int ldak, const __b
                              C + (size_t)nf * ldc, ldc, s);
         return;
     }
-    hipLaunchKernelGGL((gemm_lp_edge_kernel<__bf16, true>), dim3(ceil_div(m, 16), ceil_div(n, 16)),
-                       dim3(256), 0, s, m, n, k, Ap, ldak, Bp, ldbk, C, ldc);
+    hipLaunchKernelGGL(gemm_bf16_edge_kernel, dim3(ceil_div(m, 16), ceil_div(n, 16)), dim3(256), 0, s, m, n, k, Ap, ldak, Bp, ldbk, C, ldc);
     SLA_LAUNCH_CHECK();
 }
 

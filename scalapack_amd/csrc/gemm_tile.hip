@@ -24,13 +24,12 @@
 // for LDS, global loads, the barrier and the tile's first and last accesses are
 // another's MFMAs -- so the tile is small enough for four workgroups a CU (at
 // most 128 registers, 33 KB of LDS), which also spreads small products over the
-// chip.  Two larger tiles measured slower: 128 x 256 in 512 threads, one
-// workgroup a CU, staged the same way (the kernel of the trailing update
-// before this one), and 128 x 64 in 256 threads (39 TF/s where this one has
-// 57).  C is loaded at the start, not at the end (54 against 58 TF/s).
-// Measured, before (that kernel, 128 x 128 ones for what it left, thin ones for
-// n, k <= 64) and now, us: m = n = 16128, k = 512: 4715, 4605 (57.8 TF/s); k =
-// 256: 2710, 2487; 8192, k = 512: 1210, 1211; 4096, k = 512: 292, 303; 3072,
+// chip and leaves room for a panel.  Larger tiles pay where many of them run for
+// long (gemm_wide.hip).  128 x 64 in 256 threads was slower (39 TF/s where this one
+// has 57), and so was loading C at the end, not at the start (54 against 58 TF/s).
+// Measured, with the kernels of 128 x 256 and 128 x 128 tiles, and thin ones for n, k
+// <= 64, that it replaced, and now, us: m = n = 16128, k = 512: 4715, 4605 (57.8
+// TF/s); k = 256: 2710, 2487; 8192, k = 512: 1210, 1211; 4096, k = 512: 292, 303; 3072,
 // k = 512: 290, 181; 2900, k = 128: 141, 59; 2900, k = 128, odd leading
 // dimension: 107, 59; 960, k = 64: 99, 8; m x 32 x 32, m = 16384: 8.2, 4.2.
 #include "sla_common.h"
@@ -240,7 +239,7 @@ void gemm_tile_sub(bool ta, int m, int n, int k, const T *A, int lda, const T *B
     // each) share a CU and a fourth does not fit.  37 KB of LDS and a quarter of
     // the registers stay free for the panel's kernels, which otherwise wait until
     // the update has no more workgroups to start: it has one ready whenever a slot
-    // is free.  The update alone gets 8 % slower (m = n = 16128, k = 512: 4574,
+    // is free.  The update alone gets 9 % slower (m = n = 16128, k = 512: 4574,
     // 4985 us); PDGETRF at N = 16384, NB = 256 takes 118 ms instead of 138.
     const unsigned lds = beside ? 8000 : 0;
     // offsets of 64 columns and a step in 32 bits, but for extreme leading dimensions

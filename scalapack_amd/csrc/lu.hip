@@ -671,7 +671,7 @@ void getrs_perm_device(Handle &h, bool trans, int n, int nrhs, const double *dA,
     if (n <= 0 || nrhs <= 0) return;
     // Up to 16 right-hand sides at a time in one launch per triangle; more in
     // blocked solves whose products run on the matrix cores (n = 5000, 400
-    // right-hand sides: 96 ms sixteen at a time, 2.9 ms blocked), in chunks that
+    // right-hand sides: 96 ms sixteen at a time, 3.4 ms blocked), in chunks that
     // bound the copy.
     int chunk = std::min(nrhs, nrhs > 16 ? 1024 : 16);
     // fewer columns at a time where the device has no memory for as many

@@ -110,27 +110,6 @@ __device__ __forceinline__ uint64_t mag_key(float v, bool valid, bool top)
     return mag_key((double)v, valid, top);
 }
 
-template <int CTRL, int ROWS>
-__device__ __forceinline__ uint32_t dpp_max(uint32_t x)
-{
-    // lanes the move does not reach combine with 0
-    const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
-    return x > y ? x : y;
-}
-
-// Wave-wide maximum, uniform: within rows of 16 lanes by rotation, then the
-// row maxima broadcast upwards (row_bcast:15 and :31), the result in lane 63.
-__device__ __forceinline__ uint32_t wave_max(uint32_t x)
-{
-    x = dpp_max<0x121, 0xf>(x);
-    x = dpp_max<0x122, 0xf>(x);
-    x = dpp_max<0x124, 0xf>(x);
-    x = dpp_max<0x128, 0xf>(x);
-    x = dpp_max<0x142, 0xa>(x);
-    x = dpp_max<0x143, 0xc>(x);
-    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
-}
-
 // The wave's first maximum by full keys: the lane holding the largest key and,
 // among equal keys, the lowest position; its key and position in every lane.
 __device__ __forceinline__ int wave_pick(uint64_t &key, int &pos)
@@ -216,7 +195,10 @@ struct LeafArgs {
 
 // A word for the other workgroups: through the L2 of the XCD (local: every
 // workgroup of the leaf runs on this one, and a load that bypasses the L1 finds
-// it there) or to where every XCD sees it.
+// it there) or to where every XCD sees it.  The local store has workgroup scope,
+// which promises other workgroups nothing in the language: that they see it rests on
+// the one L2 of an XCD, to which the L1 writes every store through.  A word that did
+// not arrive would end in the bounded wait's error, not in a wrong pivot.
 __device__ __forceinline__ void post_word(uint64_t *p, uint64_t v, bool local)
 {
     if (local) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -716,9 +698,9 @@ unsigned panel_leaf(T *A, int lda, int m, int wa, int lcols, int rcols, int row0
     return 0;  // the mailbox exchange adds no barrier arrivals
 }
 
-// The build compiles this file twice, SLA_PANEL_TYPE = 64 and 32, so that
-// the fully unrolled leaf instances of the two storage types build in
-// parallel; without the macro both are instantiated here.
+// The build compiles this file twice, SLA_PANEL_TYPE = 64 and 32, so that the
+// leaf instances of the two storage types build in parallel; without the macro
+// both are instantiated here.
 #if !defined(SLA_PANEL_TYPE) || SLA_PANEL_TYPE == 64
 template unsigned panel_leaf<double>(double *, int, int, int, int, int, int, int, int *,
                                      const PanelWork<double> &, hipStream_t);

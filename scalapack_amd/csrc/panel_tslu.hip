@@ -13,7 +13,7 @@
 // One launch of G <= 32 workgroups of 512 threads; the leaf's m rows are
 // spread as in panel.hip (row g*R + q*512 + tid, R = RPT*512).
 //   1. every workgroup runs partial-pivoting elimination on its own rows in
-//      registers (per column: wave argmax, two workgroup barriers, the pivot
+//      registers (per column: wave argmax, one workgroup barrier, the pivot
 //      row through LDS) and so chooses W candidate rows, published with their
 //      original values; workgroup 0 also publishes the leaf's top W rows;
 //   2. one device-wide barrier;
@@ -44,34 +44,6 @@ constexpr int TGMAX = TPT * TMR / TW;  // workgroups per launch at most (32)
 // candidate values are stored column by column (value c of candidate sid at
 // c * TCAND + sid), so the tournament's loads are contiguous across lanes
 constexpr int TCAND = TGMAX * TW;
-
-template <int CTRL, int ROWS>
-__device__ __forceinline__ uint32_t dpp_max(uint32_t x)
-{
-    // lanes the move does not reach combine with 0
-    const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
-    return x > y ? x : y;
-}
-
-// Wave-wide maximum, uniform.
-__device__ __forceinline__ uint32_t wave_max(uint32_t x)
-{
-    x = dpp_max<0x121, 0xf>(x);
-    x = dpp_max<0x122, 0xf>(x);
-    x = dpp_max<0x124, 0xf>(x);
-    x = dpp_max<0x128, 0xf>(x);
-    x = dpp_max<0x142, 0xa>(x);
-    x = dpp_max<0x143, 0xc>(x);
-    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
-}
-
-// A barrier that waits for the workgroup's LDS traffic only.
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 
 // Rank of a pivot candidate: 0 for no row, else 1 + |v|'s bits (monotone; a NaN
 // counts as zero).  Equal ranks are decided by the lower row.

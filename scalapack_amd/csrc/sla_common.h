@@ -147,9 +147,6 @@ __device__ __forceinline__ void launch_stamp_end(unsigned long long *stamp)
     }
 }
 
-// (|v|, row) ordering of the pivot search: larger magnitude wins, the lower
-// row wins a tie -- IDAMAX's "first index of the maximum" on the current row
-// order (PBLAS/SRC/pdamax_.c:421-425).
 // Value of v in lane `lane` (uniform index) of the wave.
 template <typename T>
 __device__ __forceinline__ T lane_read(T v, int lane)
@@ -164,9 +161,64 @@ __device__ __forceinline__ T lane_read(T v, int lane)
     }
 }
 
-__device__ __forceinline__ bool pivot_better(double v1, int r1, double v2, int r2)
+// The value of lane S of the quad, in all four lanes.
+template <int S, typename T>
+__device__ __forceinline__ T quad_lane(T v)
 {
-    return v1 > v2 || (v1 == v2 && r1 < r2);
+    if constexpr (sizeof(T) == 8) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, S * 0x55, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), S * 0x55, 0xf, 0xf, false);
+        return __builtin_bit_cast(T, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+    } else {
+        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                                                 S * 0x55, 0xf, 0xf, false));
+    }
+}
+
+// The value of lane K of every row of 16 lanes, in all of them.
+template <int K, typename T>
+__device__ __forceinline__ T row_lane(T v)
+{
+    if constexpr (sizeof(T) == 8) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, 0x150 + K, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), 0x150 + K, 0xf, 0xf, false);
+        return __builtin_bit_cast(T, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+    } else {
+        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                                                 0x150 + K, 0xf, 0xf, false));
+    }
+}
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_max(uint32_t x)
+{
+    // lanes the move does not reach combine with 0
+    const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
+    return x > y ? x : y;
+}
+
+// Wave-wide maximum, uniform: within rows of 16 lanes by rotation, then the
+// row maxima broadcast upwards (row_bcast:15 and :31), the result in lane 63.
+__device__ __forceinline__ uint32_t wave_max(uint32_t x)
+{
+    x = dpp_max<0x121, 0xf>(x);
+    x = dpp_max<0x122, 0xf>(x);
+    x = dpp_max<0x124, 0xf>(x);
+    x = dpp_max<0x128, 0xf>(x);
+    x = dpp_max<0x142, 0xa>(x);
+    x = dpp_max<0x143, 0xc>(x);
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+
+// A barrier that waits for the workgroup's LDS traffic only, for kernels whose global
+// stores between barriers nobody in the workgroup reads before a full one.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 }  // namespace sla

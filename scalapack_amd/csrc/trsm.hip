@@ -14,8 +14,8 @@
 //   (64 rows) is owned by the workgroup that takes ticket b; it accumulates
 //   -T[b, c] X[c] for every finished block c (X[c] read from a mailbox whose
 //   words carry the launch's epoch, bounded wait), then solves its 64 x 64
-//   diagonal block in registers of one wave (lane = row, values broadcast by
-//   lane reads) and publishes X[b].
+//   diagonal block as four 16 x 16 triangles, a right-hand side in each row of 16
+//   lanes, and publishes X[b].
 //   Tickets are taken in start order, so a workgroup only ever waits on
 //   workgroups that are already running.  The transposed solves read the
 //   off-diagonal block by columns (lane = column of the stored triangle,
@@ -95,20 +95,6 @@ __global__ __launch_bounds__(256) void trsm_llnu_strip_kernel(int m, int n, cons
 // with L's column from LDS.  The same products in the same order as above, in
 // 13 KB of LDS and one wave instead of 102 KB and four.
 constexpr int T32_NC = 16;
-
-template <int S, typename T>
-__device__ __forceinline__ T quad_lane(T v)
-{
-    if constexpr (sizeof(T) == 8) {
-        const uint64_t u = __builtin_bit_cast(uint64_t, v);
-        const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, S * 0x55, 0xf, 0xf, false);
-        const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), S * 0x55, 0xf, 0xf, false);
-        return __builtin_bit_cast(T, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-    } else {
-        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
-                                                                 S * 0x55, 0xf, 0xf, false));
-    }
-}
 
 template <int K, typename T>
 __device__ __forceinline__ void t32_steps(T (&b)[8], const T (*Ls)[33], int q)
@@ -210,21 +196,6 @@ __device__ __forceinline__ T tv_join(uint32_t lo, uint32_t hi)
     } else {
         (void)hi;
         return __builtin_bit_cast(T, lo);
-    }
-}
-
-// The value of lane K of every row of 16 lanes, in all of them.
-template <int K, typename T>
-__device__ __forceinline__ T row_lane(T v)
-{
-    if constexpr (sizeof(T) == 8) {
-        const uint64_t u = __builtin_bit_cast(uint64_t, v);
-        const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, 0x150 + K, 0xf, 0xf, false);
-        const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), 0x150 + K, 0xf, 0xf, false);
-        return __builtin_bit_cast(T, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-    } else {
-        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
-                                                                 0x150 + K, 0xf, 0xf, false));
     }
 }
 
@@ -840,7 +811,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void trsm_llnu_blocked_kernel(
 // reciprocals), then all waves subtract E_ik X_k from the rows below on MFMA, 16
 // rows a tile, the first tile's E loaded before the solve it waits for.  Bound
 // by that chain, about 3 us per 32 rows, and not by the work: with the GEMMs
-// n = 5000 and 400 right-hand sides take 2.9 ms where sixteen at a time through
+// n = 5000 and 400 right-hand sides take 3.4 ms where sixteen at a time through
 // trsv_persistent took 96 ms.
 constexpr int TT_M = 256, TT_T = 256;
 
@@ -889,7 +860,8 @@ __global__ __launch_bounds__(TT_T) void trsm_tri_kernel(int m, int n, const T *_
     };
     for (int k = 0; k < nblk; k++) {
         const int kr = 32 * k, ntile = (m32 - kr - 32) / 16;
-        // (the barrier at the end of the last block's update frees Es)
+        // (Es: wave 0, its only reader, was done with block k - 1's before the barrier
+        // that made X_{k-1} final)
         for (int idx = tid; idx < 1024; idx += TT_T) {
             const int r = idx & 31, c = idx >> 5;
             Es[c][r] = (c < r && kr + r < m) ? E[(kr + r) * rs + (kr + c) * cs] : T(0);
