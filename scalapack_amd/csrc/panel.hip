@@ -185,10 +185,10 @@ struct LeafArgs {
     uint64_t *box;  // this launch's mailbox region
     int *abort_flag;
     uint64_t spin_limit, t0;
-    unsigned *yield;    // where the leaf says that it gives way (null: it does not)
+    // of a leaf that may give way:
+    unsigned *yield;    // where it says so (null: it does not)
     unsigned yield_id;  // by this number
     uint64_t patience;  // ticks it waits in column 0 before it does
-    unsigned look;      // a wait looks at flags and clock when its count has none of these bits
     int G, g;       // workgroups of the leaf, this one
     uint32_t xcd;   // the die it runs on
 };
@@ -227,14 +227,16 @@ __device__ __forceinline__ void publish(const LeafArgs &ar, uint64_t *cb, bool l
 // that leaves there posts nothing more, so no other one gets past column 1, and
 // since nothing but the mailbox is written before the last column, all leave the
 // matrix as it was.  Once column 0 is through, every workgroup runs.
+template <bool YIELDS>
 __device__ __forceinline__ bool keep_waiting(const LeafArgs &ar, int j, unsigned &it, int *s_abort)
 {
-    if ((++it & ar.look) != 0) return true;
+    // without patience it looks at once
+    if ((++it & 15u) != 0 && !(YIELDS && ar.yield && ar.patience == 0)) return true;
     bool on = true;
     const uint64_t dt = wall_clock64() - ar.t0;
     if (coherent_load(ar.abort_flag)) on = false;
-    else if (ar.yield && coherent_load(ar.yield) == ar.yield_id) on = false;
-    else if (ar.yield && j == 0 && dt > ar.patience) {
+    else if (YIELDS && ar.yield && coherent_load(ar.yield) == ar.yield_id) on = false;
+    else if (YIELDS && ar.yield && j == 0 && dt > ar.patience) {
         coherent_store(ar.yield, ar.yield_id);
         on = false;
     } else if (dt > ar.spin_limit) {
@@ -276,7 +278,7 @@ __device__ __forceinline__ void update_rows(T (&x)[NQ][NC], const T (&l)[NQ], co
 // 1 .. live-1 hold the columns further right.  A row that is done (or beyond
 // the leaf) holds zeros there, so it neither wins a search nor is changed by an
 // update; its multipliers stay.
-template <typename T, int NC, int NQ, bool SOLO>
+template <typename T, int NC, int NQ, bool SOLO, bool YIELDS>
 __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][NC],
                                           int (&pos)[NQ], bool &local, bool &dead, LeafLds<T> &sl)
 {
@@ -343,12 +345,9 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
     }
     if (!found && lane == 0) sl.wpos[pb][wave] = INT_MAX;
     __syncthreads();
-    // a wait of the column before that gave up: all waves see it here, before the
-    // workgroup posts anything of this column
-    if constexpr (!SOLO) {
-        dead = sl.s_abort[pb ^ 1] != 0;
-        if (dead) return;
-    }
+    // a wait of the column before that gave up: all waves see it here, and the
+    // workgroup posts nothing of this column
+    if (!SOLO) dead = sl.s_abort[pb ^ 1] != 0;
     // the workgroup's: lane x looks at the candidate of wave x % 8
     int p, fw;
     bool nonzero = true;
@@ -380,7 +379,7 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
     // 2. the other workgroups
     if constexpr (!SOLO) {
         uint64_t *cb = ar.box + (size_t)j * PANEL_MAIL_COL;
-        if (wave == nw - 1) publish<T, NC>(ar, cb, local, prow, pv, p, lane);
+        if (wave == nw - 1 && !dead) publish<T, NC>(ar, cb, local, prow, pv, p, lane);
         const int G = ar.G;
         // values and positions of candidates lane and lane + 64
         uint64_t kv[2], kp[2];
@@ -397,7 +396,7 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
             }
         } while ((kv[0] == MAIL_EMPTY || kp[0] == MAIL_EMPTY || kv[1] == MAIL_EMPTY ||
                   kp[1] == MAIL_EMPTY) &&
-                 keep_waiting(ar, j, it, &sl.s_abort[pb]));
+                 keep_waiting<YIELDS>(ar, j, it, &sl.s_abort[pb]));
         int xp = lane < G ? (int)kp[0] : INT_MAX;
         T xv = mail_value<T>(kv[0]);
         const uint32_t h = xp != INT_MAX ? mag_hi(xv) : 0u;
@@ -437,7 +436,7 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
         // through the wave's own slot in LDS
         const uint64_t *rw = cb + (size_t)gw * PANEL_MAIL_CW + lane % (4 * NC);
         uint64_t w;
-        while ((w = coherent_load(rw)) == MAIL_EMPTY && keep_waiting(ar, j, it, &sl.s_abort[pb])) {
+        while ((w = coherent_load(rw)) == MAIL_EMPTY && keep_waiting<YIELDS>(ar, j, it, &sl.s_abort[pb])) {
         }
         if (lane < 4 * NC) sl.prow[wave][lane] = mail_value<T>(w);
         prow = sl.prow[wave];
@@ -494,6 +493,9 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     unsigned yield_id, unsigned after_id, uint64_t patience)
 {
     if (!SOLO && (int)blockIdx.x % stride != first) return;
+    // the kinds whose leaves take more than a quarter of an XCD; the others go without
+    // the code, which costs them registers and 1 us
+    constexpr bool YIELDS = !SOLO && NC == 8 && PT == 512;
     const int G = SOLO ? 1 : gridDim.x / stride, g = SOLO ? 0 : blockIdx.x / stride;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6, nw = (int)blockDim.x >> 6;
@@ -516,7 +518,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
                                        ? PANEL_MAIL_VAL + e - prev_g * PANEL_MAIL_CW
                                        : PANEL_MAIL_POS + e - prev_g * (PANEL_MAIL_CW + 1))],
                                MAIL_EMPTY);
-        if (after_id != 0 && coherent_load(yield) != after_id) return;
+        if (YIELDS && after_id != 0 && coherent_load(yield) != after_id) return;
     }
 
     // column 4 i + cg of the leaf in register i; columns right of a narrow
@@ -534,8 +536,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         }
     }
     const LeafArgs ar{mail + (size_t)region * PANEL_MAIL_REGION, abort_flag, spin_limit, (uint64_t)wall_clock64(),
-                      yield_id != 0 ? yield : nullptr, yield_id, patience,
-                      yield_id != 0 && patience == 0 ? 0u : 15u, G, g,
+                      YIELDS && yield_id != 0 ? yield : nullptr, yield_id, patience, G, g,
                       SOLO ? 0u : (uint32_t)__builtin_amdgcn_s_getreg(63508) & 0xffffu};  // XCC_ID
     bool local = false;
     __syncthreads();
@@ -547,7 +548,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     for (int t = 0; t < NC && !dead; t++) {
 #pragma unroll 1
         for (int j = 4 * t; j < min(4 * t + 4, wa) && !dead; j++)
-            leaf_step<T, NC, NQ, SOLO>(ar, j, a, pos, local, dead, sl);
+            leaf_step<T, NC, NQ, SOLO, YIELDS>(ar, j, a, pos, local, dead, sl);
 #pragma unroll
         for (int q = 0; q < NQ; q++) rotate_row<NC>(a[q], a[q][0]);
     }
@@ -655,8 +656,8 @@ void launch_leaf(T *A, int lda, int m, int wa, int lcols, int rcols, int row0, i
             ms.prev_g = G;
         };
         const unsigned id = std::max(1u, ms.launches + 1);
-        if (place == LEAF_ONE_XCD_YIELDS && wa < 2)
-            throw std::logic_error("panel leaf: a leaf of one column cannot give way");
+        if (place == LEAF_ONE_XCD_YIELDS && (wa < 2 || NC != 8 || PT != 512))
+            throw std::logic_error("panel leaf: a leaf of this kind or of one column cannot give way");
         go(place == LEAF_SPREAD ? 1 : XCDS, place == LEAF_ONE_XCD_YIELDS ? id : 0u, 0u);
         if (place == LEAF_ONE_XCD_YIELDS) go(1, 0u, id);
     }
