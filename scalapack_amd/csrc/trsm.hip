@@ -378,20 +378,12 @@ __global__ __launch_bounds__(256) void trsv_persistent_kernel(
     const int j = 4 * wave + lk;
     if (4 * wave < nrhs) {
         const T *y = Ys[MF ? j : 0];
+        const uint64_t tag = (uint64_t)epoch << 32;
         T yy[4];  // the rows of the current triangle, then those after it
 #pragma unroll
         for (int i = 0; i < 4; i++) yy[i] = y[16 * (FORWARD ? i : 3 - i) + lr];
-        const uint64_t tag = (uint64_t)epoch << 32;
-#pragma unroll 1
-        for (int i = 0; i < 4; i++) {
+        auto triangle = [&](int i) {
             const int r0 = 16 * (FORWARD ? i : 3 - i);
-            // no rows here (a short last block; yy then holds zeros): n = 1, both
-            // triangles of one right-hand side took 9.8 us with all four, now 7.0; n =
-            // 20 11.1, 9.1
-            if (r0 >= rows) {
-                yy[0] = yy[1], yy[1] = yy[2], yy[2] = yy[3];
-                continue;
-            }
             const T *e[4];  // rows r0, and those of yy[1] .. yy[3] (a row of the block if none)
 #pragma unroll
             for (int q = 0; q < 4; q++)
@@ -406,6 +398,26 @@ __global__ __launch_bounds__(256) void trsv_persistent_kernel(
                 X[(size_t)(rb + r0 + lr) + (size_t)j * ldx] = x;
             }
             yy[0] = yy[1] + bb[1], yy[1] = yy[2] + bb[2], yy[2] = yy[3] + bb[3];
+        };
+        // A short last block has fewer triangles with rows: n = 1, both solves with one
+        // right-hand side took 9.8 us with all four, now 6.9; n = 20 11.1, 9.0.
+        int first = 0, last = 4;
+        if (rows <= TV_BS - 16) {
+            const int none = 4 - (rows + 15) / 16;
+            if (FORWARD) last -= none;
+            else first = none;
+            if (!FORWARD)
+                for (int i = 0; i < none; i++) yy[0] = yy[1], yy[1] = yy[2], yy[2] = yy[3];
+        }
+        // A loop of its own for whole blocks: the plain solves are 2 % slower without
+        // it, the transposed ones with it (n = 8192, two right-hand sides: 1112 and 1130
+        // us, 1122 and 1078), by how the compiler schedules the steps.
+        if (!TRANS && rows > TV_BS - 16) {
+#pragma unroll 1
+            for (int i = 0; i < 4; i++) triangle(i);
+        } else {
+#pragma unroll 1
+            for (int i = first; i < last; i++) triangle(i);
         }
     }
 }
