@@ -68,6 +68,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 namespace sla {
 
@@ -485,7 +486,9 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
 // are dealt, they share one XCD and its L2 (checked in column 0).
 // yield_id: number by which the leaf gives way in *yield (0: it does not);
 // after_id: the leaf runs only if the launch of that number did (0: always).
-template <typename T, int NC, int NQ, bool SOLO, int PT, int WPE>
+// YIELDS: the leaf may give way, or runs after one that may have; the others go
+// without that code, which costs them scalar registers and 1 to 3 us.
+template <typename T, int NC, int NQ, bool SOLO, int PT, int WPE, bool YIELDS>
 __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(WPE))) void panel_leaf_kernel(
     T *__restrict__ A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0,
     int *__restrict__ ipiv, uint64_t *__restrict__ mail, int region, int prev_wa, int prev_g,
@@ -493,9 +496,6 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     unsigned yield_id, unsigned after_id, uint64_t patience)
 {
     if (!SOLO && (int)blockIdx.x % stride != first) return;
-    // the kinds whose leaves take more than a quarter of an XCD; the others go without
-    // the code, which costs them registers and 1 us
-    constexpr bool YIELDS = !SOLO && NC == 8 && PT == 512;
     const int G = SOLO ? 1 : gridDim.x / stride, g = SOLO ? 0 : blockIdx.x / stride;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6, nw = (int)blockDim.x >> 6;
@@ -637,16 +637,17 @@ void launch_leaf(T *A, int lda, int m, int wa, int lcols, int rcols, int row0, i
     if (threads > PT) throw std::logic_error("panel leaf: workgroup larger than its kernel's");
     if constexpr (SOLO) {
         // the mailbox and its record stay as the last exchanging launch left them
-        hipLaunchKernelGGL((panel_leaf_kernel<T, NC, NQ, true, PT, WPE>), dim3(1), dim3(threads), 0,
+        hipLaunchKernelGGL((panel_leaf_kernel<T, NC, NQ, true, PT, WPE, false>), dim3(1), dim3(threads), 0,
                            s, A, lda, m, wa, lcols, rcols, row0, col0, ipiv, pw.mail, 0, 0, 0,
                            pw.abort_flag, pw.zero_col, pw.spin_limit, 1, 0, pw.yield, 0u, 0u,
                            (uint64_t)0);
         SLA_LAUNCH_CHECK();
     } else {
-        auto go = [&](int stride, unsigned yield_id, unsigned after_id) {
+        auto go = [&](auto yields, int stride, unsigned yield_id, unsigned after_id) {
             const int first = stride == 1 ? 0 : (int)(ms.launches % XCDS);
-            hipLaunchKernelGGL((panel_leaf_kernel<T, NC, NQ, false, PT, WPE>), dim3(G * stride),
-                               dim3(threads), 0, s, A, lda, m, wa, lcols, rcols, row0, col0, ipiv,
+            hipLaunchKernelGGL((panel_leaf_kernel<T, NC, NQ, false, PT, WPE, decltype(yields)::value>),
+                               dim3(G * stride), dim3(threads), 0, s, A, lda, m, wa, lcols, rcols, row0,
+                               col0, ipiv,
                                pw.mail, (int)(ms.launches & 1u), ms.prev_wa, ms.prev_g,
                                pw.abort_flag, pw.zero_col, pw.spin_limit, stride, first, pw.yield,
                                yield_id, after_id, pw.patience);
@@ -655,11 +656,15 @@ void launch_leaf(T *A, int lda, int m, int wa, int lcols, int rcols, int row0, i
             ms.prev_wa = wa;
             ms.prev_g = G;
         };
-        const unsigned id = std::max(1u, ms.launches + 1);
-        if (place == LEAF_ONE_XCD_YIELDS && (wa < 2 || NC != 8 || PT != 512))
-            throw std::logic_error("panel leaf: a leaf of this kind or of one column cannot give way");
-        go(place == LEAF_SPREAD ? 1 : XCDS, place == LEAF_ONE_XCD_YIELDS ? id : 0u, 0u);
-        if (place == LEAF_ONE_XCD_YIELDS) go(1, 0u, id);
+        if (place != LEAF_ONE_XCD_YIELDS) return go(std::false_type(), place == LEAF_SPREAD ? 1 : XCDS, 0u, 0u);
+        if constexpr (leaf_may_yield(NC, PT)) {
+            if (wa < 2) throw std::logic_error("panel leaf: a leaf of one column cannot give way");
+            const unsigned id = std::max(1u, ms.launches + 1);
+            go(std::true_type(), XCDS, id, 0u);
+            go(std::true_type(), 1, 0u, id);
+        } else {
+            throw std::logic_error("panel leaf: a leaf of this kind does not give way");
+        }
     }
 }
 

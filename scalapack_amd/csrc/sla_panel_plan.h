@@ -24,6 +24,8 @@ struct LeafPlan {
 constexpr int leaf_nc(int wa) { return wa <= 8 ? 2 : wa <= 16 ? 4 : 8; }
 // Elements a thread holds in the smaller kinds.
 constexpr int leaf_values(int nc) { return nc == 2 ? 16 : 32; }
+// Kinds (by registers per row and lane, threads) that may be planned to give way.
+constexpr bool leaf_may_yield(int nc, int threads) { return nc == 8 && threads == 512; }
 // Quarters of a CU that a workgroup's registers take.
 constexpr int leaf_quarters(const LeafPlan &p) { return (p.values == 64 ? 2 : 1) * (p.waves > 4 ? 2 : 1); }
 
@@ -64,6 +66,8 @@ inline LeafPlan leaf_plan(int m, int wa, int panel_wgs, bool beside, bool xcds)
         return {v, 4, g1, xcds && g1 <= XCD_CUS ? LEAF_ONE_XCD : LEAF_SPREAD};
     if (nc == 8 && g2 <= panel_wgs) return {v, 8, g2, tall(g2)};
     if (nc == 8 && g3 <= panel_wgs) return {64, 8, g3, tall(g3)};
+    // with more than the caller prefers, the fewest, on one XCD
+    if (nc == 8 && g3 <= XCD_CUS) return {64, 8, g3, tall(g3)};
     // Over the XCDs the middle kind is the faster one (32 columns, m = 65536: 174 us
     // against 179 with half as many of the largest kind; 16 columns, 131072: 99, 115)
     if (g2 <= LEAF_GMAX) return {v, 8, g2, LEAF_SPREAD};

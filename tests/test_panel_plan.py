@@ -73,7 +73,7 @@ def test_waiting_workgroups_find_room(plans):
             assert p["xcds"] and 4 * p["wgs"] * p["quarters"] <= 4 * XCD_CUS, p
         elif p["place"] == ONE_XCD_YIELDS:
             # alone it fits; a leaf of one column ends before it could give way
-            assert p["xcds"] and p["wa"] > 1 and p["wgs"] * p["quarters"] <= 4 * XCD_CUS, p
+            assert p["xcds"] and p["wa"] > 1 and p["nc"] == 8 and p["waves"] == 8 and p["wgs"] * p["quarters"] <= 4 * XCD_CUS, p
         else:
             leaves = 8 if p["wgs"] <= 32 else 2
             per_xcd = -(-p["wgs"] // XCDS)
@@ -95,4 +95,4 @@ def test_preferred_workgroups(plans):
     for (m, wa, wgs), p in by.items():
         if p["nc"] == 8 and m <= wgs * 16 * 8 * 8:
             assert p["wgs"] <= wgs, p
-    assert [by[30011, 32, w]["wgs"] for w in (32, 64, 128)] == [30, 59, 118]
+    assert [by[30011, 32, w]["wgs"] for w in (8, 32, 64, 128)] == [30, 30, 59, 118]
