@@ -152,6 +152,7 @@ __device__ __forceinline__ void panel_regs(int n, int kb, int w, bool first, Glo
             v[q][c] = (r < n && c < w) ? (a + (size_t)(kb + c) * lda)[(unsigned)r] : T(0);
     }
     if (tid == 0) sl.pm.any = 0;
+    unsigned nopiv = 0;  // columns without a pivot
 #pragma unroll
     for (int jj = 0; jj < W; jj++) {
         if (jj < w) {  // uniform
@@ -210,9 +211,8 @@ __device__ __forceinline__ void panel_regs(int n, int kb, int w, bool first, Glo
             const T *prow = sl.rows[pb][fw];
             const T pv = prow[jj], rcp = sl.rcp[pb][fw];
             const bool nz = pv != T(0);
-            // no interchange without a pivot (p != j if row j holds a NaN and others zeros)
-            if (tid == 0) piv[j] = (nz ? p : j) + 1;
-            if (!nz && info == 0) info = j + 1;
+            if (tid == 0) piv[j] = p + 1;
+            if (!nz) nopiv |= 1u << jj;
 #pragma unroll
             for (int q = 0; q < RPT; q++) {
                 if (nz) pos[q] = pos[q] == p ? j : pos[q] == j ? p : pos[q];
@@ -224,6 +224,15 @@ __device__ __forceinline__ void panel_regs(int n, int kb, int w, bool first, Glo
                 }
             }
         }
+    }
+    if (nopiv) {
+        if (info == 0) info = kb + __builtin_ctz(nopiv) + 1;
+        // no rows were interchanged (p != j if row j holds a NaN and others zeros)
+        if (tid == 0)
+            for (unsigned m = nopiv; m; m &= m - 1) {
+                const int j = kb + __builtin_ctz(m);
+                piv[j] = j + 1;
+            }
     }
 #pragma unroll
     for (int q = 0; q < RPT; q++) {
