@@ -186,7 +186,7 @@ KERNEL_OF = {  # kernel symbol behind each timing class (for matching kernel tra
                         "tile borders by gemm_split_nn_sub_direct_kernel)",
     ("gemm", "fp16x3"): "gemm_split_lds_kernel<_Float16, 2> (trailing update, FP16x3; "
                         "tile borders by gemm_split_nn_sub_direct_kernel)",
-    ("panel", "fp64"): "panel_leaf_kernel<double, NC, NQ, SOLO, PT, WPE>",
+    ("panel", "fp64"): "panel_leaf_kernel<double, NC, NQ, SOLO, PT, WPE, YIELDS>",
 }
 
 

@@ -822,7 +822,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void trsm_llnu_blocked_kernel(
 // column, as trsm_llnu32_kernel; a non-unit diagonal as products with its
 // reciprocals), then all waves subtract E_ik X_k from the rows below on MFMA, 16
 // rows a tile, the first tile's E loaded before the solve it waits for.  Bound
-// by that chain, about 3 us per 32 rows, and not by the work: with the GEMMs
+// by that chain, about 6 us per 32 rows, and not by the work: with the GEMMs
 // n = 5000 and 400 right-hand sides take 3.4 ms where sixteen at a time through
 // trsv_persistent took 96 ms.
 constexpr int TT_M = 256, TT_T = 256;
