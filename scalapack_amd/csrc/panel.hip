@@ -488,6 +488,9 @@ __device__ __forceinline__ void leaf_step(const LeafArgs &ar, int j, T (&a)[NQ][
 // after_id: the leaf runs only if the launch of that number did (0: always).
 // YIELDS: the leaf may give way, or runs after one that may have; the others go
 // without that code, which costs them scalar registers and 1 to 3 us.
+// Scratch, FP64: five or six values a lane of the 32-column leaves at WPE = 4, stored
+// before the column loop and read after it; 68 and 92 bytes of the 8-column leaves with
+// 64 values a lane, within it.
 template <typename T, int NC, int NQ, bool SOLO, int PT, int WPE, bool YIELDS>
 __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(WPE))) void panel_leaf_kernel(
     T *__restrict__ A, int lda, int m, int wa, int lcols, int rcols, int row0, int col0,
